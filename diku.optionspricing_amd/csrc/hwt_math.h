@@ -27,7 +27,10 @@ struct OptConst {
     int32_t jmax, n, e, w; // half width, height, exercise step (-1: none), width
     int16_t type, unit;    // CALL 0 / PUT 1; 1 if the unit-diagonal stencil form is safe
     int32_t status;        // ST_*
-    int64_t work;          // stencil node updates this option needs
+    // how far from the path's mean, in standard deviations, the pricing
+    // windows follow it (window_sigmas); infinite: the whole light cone
+    float sigmas;
+    float pad;
 };
 static_assert(sizeof(OptConst) == 96, "OptConst layout");
 
@@ -212,7 +215,8 @@ HWT_HD int32_t option_constants(double strike, double T, double len, uint16_t te
     c.type = type;
     c.unit = 0;
     c.Pe = c.Pn = c.rho = c.rhop = 0.0;
-    c.work = 0;
+    c.sigmas = INFINITY;
+    c.pad = 0.0f;
     c.n = c.jmax = c.w = 0;
     c.e = -1;
     if ((type != 0 && type != 1) || termUnit == 0 || termSteps == 0 || !(a > 0.0) ||
@@ -251,7 +255,8 @@ HWT_HD int32_t constants_given(double t, double dt, double dr, double X, double 
     c.type = type;
     c.unit = 0;
     c.Pe = c.Pn = c.rho = c.rhop = 0.0;
-    c.work = 0;
+    c.sigmas = INFINITY;
+    c.pad = 0.0f;
     c.n = c.jmax = c.w = 0;
     c.e = -1;
     if ((type != 0 && type != 1) || termUnit == 0 || !(dt > 0.0) || !(dr >= 0.0) || !(M > -1.0 && M < 0.0) ||

@@ -52,7 +52,10 @@ constexpr int FLAT_HBUCKETS = 64;   // height buckets per flat part (one width e
 constexpr int MAX_PADS = 128;       // idle task slots padding row and flat parts, at most
 constexpr int KSMALL = 2;  // trees up to 64*KSMALL nodes wide go to the narrow-tree kernel
 #ifndef WIDE_WINDOW_STEP
-#define WIDE_WINDOW_STEP 4  // nodes per lane a wide tree's window grows or shrinks by
+#define WIDE_WINDOW_STEP 4  // nodes per lane a wide tree's light-cone window grows or shrinks by
+#endif
+#ifndef REACH_WINDOW_STEP
+#define REACH_WINDOW_STEP 1  // ... and its FP64 window along the reach
 #endif
 // k_setup's class switches
 constexpr int CLASS_ROWS = 1, CLASS_FLAT = 2;

@@ -37,11 +37,17 @@ __device__ __forceinline__ double price_option(const OptConst &cv, const double 
     // wide and narrow trees: 283 us with single steps, 252 us with 2, 243 us
     // with 4); the mid class (up to 128 nodes wide) keeps single steps
     constexpr int G = KMAX > KSMALL ? WIDE_WINDOW_STEP : 1;
-    forward_pass<T, KMAX, G>(t, e, lane, lds, etab, fscratch, flo, fhi, unit);
-    backward_pass<T, KMAX, G>(t, n, e, lane, lds, etab, blo, bhi, unit);
+    constexpr int RG = REACH_WINDOW_STEP;
+    const Reach reach = make_reach(cv.sigmas, t.M, t.dr, t.dt, n, t.jmax);
+    forward_pass<T, KMAX, G, RG>(t, reach, e, lane, lds, etab, fscratch, flo, fhi, unit);
+    backward_pass<T, KMAX, G, RG>(t, reach, n, e, lane, lds, etab, blo, bhi, unit);
 
     const int ep = min(e, t.jmax);
-    const int klo = t.jmax - ep, khi = t.jmax + ep;
+    int klo = t.jmax - ep, khi = t.jmax + ep;
+    if constexpr (sizeof(T) == sizeof(double)) {  // both windows hold the nodes kept at step e
+        klo = max(klo, max(flo, blo));
+        khi = min(khi, min(fhi, bhi) - 1);
+    }
     auto fy = [&](int k) { return (k >= flo && k < fhi) ? (double)fscratch[k] : 0.0; };
     auto fb = [&](int k) { return (k >= blo && k < bhi) ? (double)lds[k] : 0.0; };
     auto yk = [&](int k) {

@@ -281,7 +281,7 @@ __device__ __forceinline__ void copy_out(u32x4 *__restrict__ dst, const u32x4 *s
 }
 
 __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, int32_t sort, int32_t maxWidth,
-                                                       double unit_dmin, int32_t classes,
+                                                       double unit_dmin, int32_t classes, int32_t reach,
                                                        OptConst *__restrict__ cst, double *__restrict__ edge,
                                                        int2 *__restrict__ slot, int32_t *__restrict__ hist,
                                                        int32_t *__restrict__ tally, double *__restrict__ out)
@@ -389,17 +389,22 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, in
                 }
                 c.rho = t.rho;
                 c.rhop = t.rhop;
-                c.work = dual_node_updates(c.n, c.e, c.jmax);
-                work = (unsigned long long)c.work;
+                const bool wide = (c.w + WAVE - 1) / WAVE > KSMALL;
+                work = (unsigned long long)dual_node_updates(c.n, c.e, c.jmax);
                 seq_work = (unsigned long long)seq_node_updates(c.n, c.jmax);
+                // FP64 prices a wide tree over the nodes that carry weight
+                int64_t nodes = (int64_t)work;
+                if (wide && reach) {
+                    c.sigmas = window_sigmas(c);
+                    nodes = (int64_t)reach_updates(make_reach(c.sigmas, c.M, c.dr, c.dt, c.n, c.jmax), c.n, c.e);
+                }
                 int64_t key;
                 switch (sort) {
                 case 'W': case 'w': key = c.w; break;
                 case 'H': case 'h': key = c.n; break;
                 case '-': key = 0; break;
-                default: key = c.work; break;
+                default: key = nodes; break;
                 }
-                const bool wide = (c.w + WAVE - 1) / WAVE > KSMALL;
                 if (wide) b = B_WIDE + log_bucket(key, 8, NBUCKET - B_WIDE);
                 else if ((classes & CLASS_FLAT) && c.w <= FLAT_MAX_WIDTH) b = flat_bucket(c.w, c.n);
                 else if (c.w > ROW_MAX_WIDTH || !(classes & CLASS_ROWS)) b = B_MID + log_bucket(key, 4, B_WIDE - B_MID);
@@ -500,11 +505,11 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_order(int32_t n, const int32_t 
     if (s.x >= 0) order[soffs[s.x] + s.y] = i;
 }
 
-// What the wide-tree kernel's stencil steps executed in the last execution,
-// padding slots included, from the window schedule it walks
-// (forward_schedule / backward_schedule): operations (per lane and step 4K+1
-// in the unit-diagonal form, 5K in the plain one) and node slots (64 K per
-// step) per form.  One thread per wide task; run at sync time, never in the
+// The wide trees' stencil steps over their light-cone windows, padding slots
+// included (cone_forward / cone_backward; mixed mode executes these, the FP64
+// kernel about half of them, Reach): operations (per lane and step 4K+1 in
+// the unit-diagonal form, 5K in the plain one) and node slots (64 K per step)
+// per form.  One thread per wide task; run at sync time, never in the
 // timed pipeline.
 __global__ __launch_bounds__(256) void k_count_steps(const OptConst *__restrict__ cst,
                                                      const int32_t *__restrict__ order, int32_t *__restrict__ tally,
@@ -525,8 +530,8 @@ __global__ __launch_bounds__(256) void k_count_steps(const OptConst *__restrict_
             slots[u ? 0 : 1] += nn * win.K;
         };
         int lo, hi;
-        forward_schedule<WIDE_WINDOW_STEP>(t, c.e, lo, hi, count);
-        backward_schedule<WIDE_WINDOW_STEP>(t, c.n, c.e, lo, hi, count);
+        cone_forward<WIDE_WINDOW_STEP>(t, c.e, lo, hi, count);
+        cone_backward<WIDE_WINDOW_STEP>(t, c.n, c.e, lo, hi, count);
         atomicAdd(&part[0], ops);
         atomicAdd(&part[1], slots[0]);
         atomicAdd(&part[2], slots[1]);
@@ -714,10 +719,11 @@ static int launch_pipeline(hwt_plan *p, const DevOpts &o, const DevYield &y, dou
                                 ? 0
                                 : ((p->cfg.flags & HWT_FLAG_NO_ROWS) ? 0 : CLASS_ROWS) |
                                       ((p->cfg.flags & HWT_FLAG_NO_FLAT) ? 0 : CLASS_FLAT);
+        const int reach = p->cfg.form != HWT_FORM_LANE && p->cfg.precision == HWT_PREC_FP64 ? 1 : 0;
         // the lane form prices tasks one per lane: no row or flat groups, no pads
         // form 1 prices trees up to its column length; wider ones are unsupported
         const int max_width = p->cfg.form == HWT_FORM_LANE ? p->lane_width : WAVE_MAX_WIDTH;
-        k_setup<<<blocks, SETUP_BLOCK, 0, s>>>(o, y, sort, max_width, unit_dmin, classes, p->cst, p->edge,
+        k_setup<<<blocks, SETUP_BLOCK, 0, s>>>(o, y, sort, max_width, unit_dmin, classes, reach, p->cst, p->edge,
                                                p->slot, p->hist, p->tally, out);
         k_order<<<blocks, SETUP_BLOCK, 0, s>>>(n, o.count, p->slot, p->hist, p->order, p->tally, asc, classes);
         if (time_kernel) HWT_HIP(hipEventRecord(p->evk0, s));

@@ -135,8 +135,10 @@ typedef struct {
     double  wide_ms;          /* wide-tree pricing kernel alone (HWT_FLAG_NO_GRAPH), else 0 */
     double  narrow_ms;        /* narrow-tree pricing kernel alone (HWT_FLAG_NO_GRAPH), else 0 */
     int64_t device_memory;    /* bytes of device memory held by the plan */
-    int64_t node_updates;     /* stencil node updates performed (active tree region) */
-    int64_t wide_node_updates;/* ... of which by the wide-tree kernel */
+    int64_t node_updates;     /* tree nodes between the root and the exercise and bond dates that
+                                 the price depends on (light cones).  FP64 steps those of a
+                                 wide tree that carry weight, about half of them. */
+    int64_t wide_node_updates;/* ... of which in wide trees */
     int64_t seq_node_updates; /* node updates the reference's seq would perform (both passes) */
     int32_t tasks;            /* work items scheduled */
     int32_t wide_tasks;       /* ... of which wide trees */
@@ -144,14 +146,14 @@ typedef struct {
     int32_t fp64_repriced;    /* HWT_PREC_MIXED: options whose FP32 tree state left FP32's
                                  range (long, weakly mean-reverting bonds) and were priced
                                  again with FP64 states in the same execution */
-    int64_t wide_step_ops;    /* arithmetic operations the wide-tree kernel's stencil steps
-                                 executed, padding slots included: per lane and step 4K+1 in
-                                 the unit-diagonal form (K nodes per lane), 5K in the plain
-                                 form (FP64 FLOP in FP64 mode).  Counted by hwt_plan_sync
-                                 from the window schedule the kernel walks (a small kernel
+    int64_t wide_step_ops;    /* arithmetic operations of the wide trees' stencil steps over
+                                 their light-cone windows, padding slots included: per lane
+                                 and step 4K+1 in the unit-diagonal form (K nodes per lane),
+                                 5K in the plain form.  What mixed mode executes; FP64 steps
+                                 narrower windows.  Counted by hwt_plan_sync (a small kernel
                                  after the execution, run only when stats are asked for);
                                  0 for form 1 */
-    int64_t wide_unit_slots;  /* node slots it stepped in the unit-diagonal form (64 K per step) */
+    int64_t wide_unit_slots;  /* node slots of those in the unit-diagonal form (64 K per step) */
     int64_t wide_plain_slots; /* ... in the plain form */
 } hwt_stats;
 
