@@ -24,13 +24,28 @@ __device__ __forceinline__ double payoff(const OptConst &cv, double B)
 //   price = Pe / S1 * sum y payoff(scale b).
 // Sums are FP64 (compensated in mixed mode).
 
+__device__ __noinline__ static void make_edge_table(const TreeShape t, lds_f64 *etab)
+{
+    double tab[EDGE_TAB];
+    edge_table(t, tab);
+    for (int k = 0; k < EDGE_TAB; ++k) etab[k] = tab[k];
+}
+
 template <class T, int KMAX>
 __device__ __forceinline__ double price_option(const OptConst &cv, const double *edge, int lane,
                                                typename Lds<T>::type *lds, lds_f64 *etab, T *fscratch)
 {
     const TreeShape t = uni(TreeShape{cv.w, cv.jmax, cv.M, cv.dr, cv.dt, cv.rho, cv.rhop});
     const int n = uni(cv.n), e = uni(cv.e);
-    load_edge_table(edge, lane, etab);
+    bool made = false;
+    if constexpr (sizeof(T) == sizeof(double)) {
+        if (!edge) {  // FP64 plans keep no tables (hwt_tri.h); the few trees that come here make theirs
+            if (lane == 0) make_edge_table(t, etab);
+            __syncthreads();
+            made = true;
+        }
+    }
+    if (!made) load_edge_table(edge, lane, etab);
     int flo, fhi, blo, bhi;
     const bool unit = uni((int)cv.unit) != 0;
     // wide trees change window four nodes per lane at a time (a 60k batch of
@@ -173,7 +188,7 @@ __device__ __forceinline__ void price_tasks(const OptConst *__restrict__ cst, co
     while (t < last) {
         const int o = uni(order[t]);
         const OptConst c = cst[o];
-        const double *eo = edge + (size_t)o * EDGE_TAB;
+        const double *eo = edge ? edge + (size_t)o * EDGE_TAB : nullptr;
         double p;
         if (NARROW) {
             const int K = (uni(c.w) + WAVE - 1) / WAVE;
@@ -201,8 +216,10 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(2))) void 
     const OptConst *__restrict__ cst, const double *__restrict__ edge, const int32_t *__restrict__ order,
     int32_t *__restrict__ tally, double *__restrict__ out, double *__restrict__ scratch, int32_t *__restrict__ redo)
 {
-    clear_bucket_counts(tally);
-    const int nlarge = uni(tally[T_NLARGE]);
+    constexpr bool big = sizeof(T) == sizeof(double);  // FP64: the big class alone, usually empty
+    const int nlarge = uni(tally[big ? T_TBIG : T_NLARGE]);
+    if (big && nlarge == 0) return;
+    if (!big) clear_bucket_counts(tally);
     price_tasks<T, MAXK, false, true>(cst, edge, order, tally, T_QUEUE, 0, nlarge, out, scratch, redo);
     stamp_wave_end(tally);
 }

@@ -128,6 +128,7 @@ HWT_HD void edge_table_general(const TreeShape &t, double *tab)
 // interior discounts the same way, one multiplication per node).
 struct EdgeDiscounts {
     double E0, E1, E2, E3, Ea, Eb, Ec, Ed;
+    double q;  // e^{-h}
 };
 
 HWT_HD EdgeDiscounts edge_discounts(const TreeShape &t)
@@ -135,6 +136,7 @@ HWT_HD EdgeDiscounts edge_discounts(const TreeShape &t)
     const double h = t.dr * t.dt, X = t.jmax * h;
     const double q = exp(-h), qi = exp(h);
     EdgeDiscounts e;
+    e.q = q;
     e.E0 = exp(X);
     e.E1 = e.E0 * q;
     e.E2 = e.E1 * q;
@@ -743,13 +745,13 @@ __device__ __forceinline__ void cone_backward(const TreeShape &t, int n, int e, 
 // at most h (2 - 2 sqrt(w (2-w))) / (3 (1 - q^2) (1 - q)), w = q^n, over s
 // (at u = sqrt(w/(2-w))).  Discounting up to the exercise step only moves it
 // less.  Nodes below -(drift + c sd) or above c sd carry less than e^{-c^2/2}
-// of the sums: the windows leave them out, at c = sqrt(10^2 + z^2)
-// (window_sigmas), where e^{-50} = 2e-22 of the sums is five orders below
+// of the sums: the windows leave them out, at c = sqrt(9.5^2 + z^2)
+// (window_sigmas), where e^{-45} = 3e-20 of the sums is four orders below
 // the last bit of an FP64 sum; z is the strike's distance from the mean where
 // the option is out of the money, so that a price that is itself a tail keeps
-// its leading digits.  Prices come out the same to the last bit as from the whole
-// light cone (serial comparison over 1,600 random trees; differences begin at
-// c = 9).  On trees 270 to 1,330 nodes wide over 10 to 30 years this leaves 45%
+// its leading digits.  Prices come out as from the whole light cone, to 2e-16
+// (serial comparison over 1,600 random trees: bit for bit at 10, 2e-15 at 9,
+// 1e-11 at 8).  On trees 270 to 1,330 nodes wide over 10 to 30 years this leaves 45%
 // of the nodes: 60k skewed batch 275 -> 221 us (wide kernel 228 -> 166), 20k
 // 226 -> 171, 1M mix 12.0 -> 10.8 ms, widths up to 511 over up to 100 years
 // (69% of the nodes) 1.19 -> 1.12 ms.
@@ -757,7 +759,7 @@ __device__ __forceinline__ void cone_backward(const TreeShape &t, int n, int e, 
 // Evaluated in FP32 (two units of slack): only which nodes are kept depends on it.
 struct Reach {
     float c, k1, var, hd, dmax;  // sigmas, -log2 q, 1/(3(1-q^2)), h var/(1-q), the largest drift
-    int32_t n, jmax;
+    int32_t jmax;
     float wn;  // q^n
 };
 
@@ -773,7 +775,6 @@ __device__ __forceinline__ Reach make_reach(float sigmas, double M, double dr, d
     r.k1 = m < 0.0625f ? 1.44269504f * m * (1.0f + m * (0.5f + m * (0.33333333f + m * 0.25f))) : -log2_f(1.0f - m);
     r.var = 1.0f / (3.0f * m * (2.0f - m));
     r.hd = (float)(dr * dt) * r.var / m;
-    r.n = n;
     r.jmax = jmax;
     r.wn = exp2_f(-r.k1 * (float)n);
     const float eps = 1.0f - r.wn;
@@ -794,7 +795,7 @@ __device__ __forceinline__ void reach_at(const Reach &r, int s, int cone, int &l
 }
 
 // c for an option whose strike is z standard deviations out of the money.
-constexpr float WINDOW_SIGMAS = 10.0f;
+constexpr float WINDOW_SIGMAS = 9.5f;
 
 __device__ __forceinline__ float window_sigmas(const OptConst &c)
 {
@@ -848,12 +849,10 @@ __device__ __forceinline__ int ceil_window(int nodes, int G, int full)
     return min((K + G - 1) / G * G, full);
 }
 
-// FP64 schedules of the two passes, over the nodes kept.  The 64 lanes of the calling wave look 64 evenly spaced steps ahead for the
+// FP64 schedules of the two passes, over the nodes kept, one phase at a time.
+// The 64 lanes of the calling wave look 64 evenly spaced steps ahead for the
 // one where the window has to change (sizes are multiples of G nodes per
 // lane, at least MIN_WINDOW, up to the tree's own).
-// visit(win, nsteps, in_lo, in_hi, last): in_lo/in_hi bound the previous
-// window's tree nodes (empty for the first phase); last marks the forward
-// pass's final phase.
 constexpr int MIN_WINDOW = 2;
 
 // The lane'th of 64 evenly spaced counts in [1, steps], the last one steps.
@@ -862,68 +861,85 @@ __device__ __forceinline__ int look_ahead(int steps, int lane)
     return (int)(((int64_t)steps * (lane + 1) + WAVE - 1) / WAVE);
 }
 
-template <int G, class Visit>
-__device__ __forceinline__ void reach_forward(const TreeShape &t, const Reach &r, int e, int lane, int &lo, int &hi,
-                                                 Visit &&visit)
+struct ReachPhase {
+    Window win;
+    int end;  // the step the phase ends at
+};
+
+// The forward phase that starts at step i: the window that reaches the first
+// of the steps looked at, then as many of them as stay inside it.
+template <int G>
+__device__ __forceinline__ ReachPhase reach_ahead(const TreeShape &t, const Reach &r, int i, int e, int lane)
 {
     const int full = (t.w + WAVE - 1) / WAVE;
-    int in_lo = 0, in_hi = 0;  // empty: initial values
-    int i = 0;
-    for (;;) {
-        // the window that reaches the first of the steps looked at, then as
-        // many of them as stay inside it
-        const int s = i + look_ahead(e - i, lane);
-        int l, u;
-        reach_at(r, s, e, l, u);
-        const int K = max(ceil_window(uni(l + u + 1), G, full), min(MIN_WINDOW, full));
-        const unsigned long long out = K < full ? __ballot(l + u + 1 > WAVE * K) : 0ull;
-        const int at = out ? __builtin_ctzll(out) - 1 : WAVE - 1;  // the last step that fits
-        const int iend = __builtin_amdgcn_readlane(s, at);
-        const Window win = window_of(K, __builtin_amdgcn_readlane(l, at), __builtin_amdgcn_readlane(u, at), t);
-        const bool last = iend >= e;
-        visit(win, iend - i, in_lo, in_hi, last);
-        i = iend;
-        in_lo = win.base;
-        in_hi = min(win.base + WAVE * win.K, t.w);
-        if (last) break;
-    }
-    lo = in_lo;
-    hi = in_hi;
+    const int s = i + look_ahead(e - i, lane);
+    int l, u;
+    reach_at(r, s, e, l, u);
+    const int K = max(ceil_window(uni(l + u + 1), G, full), min(MIN_WINDOW, full));
+    const unsigned long long out = K < full ? __ballot(l + u + 1 > WAVE * K) : 0ull;
+    const int at = out ? __builtin_ctzll(out) - 1 : WAVE - 1;  // the last step that fits
+    return ReachPhase{window_of(K, __builtin_amdgcn_readlane(l, at), __builtin_amdgcn_readlane(u, at), t),
+                      __builtin_amdgcn_readlane(s, at)};
 }
 
-// The backward pass also keeps only the nodes that can still reach the
-// exercise nodes |j| <= min(e, jmax).
-template <int G, class Visit>
-__device__ __forceinline__ void reach_backward(const TreeShape &t, const Reach &r, int n, int e, int lane, int &lo,
-                                                  int &hi, Visit &&visit)
+// The backward phase that starts at step s with reach l0, u0 (replaced by the
+// reach at its end): down to the first step looked at that fits the next
+// window down.  The backward pass also keeps only the nodes that can still
+// reach the exercise nodes |j| <= min(e, jmax).
+template <int G>
+__device__ __forceinline__ ReachPhase reach_back(const TreeShape &t, const Reach &r, int s, int e, int lane, int &l0,
+                                                 int &u0)
 {
     const int full = (t.w + WAVE - 1) / WAVE;
-    const int ep = min(e, t.jmax);
+    const int K = max(ceil_window(l0 + u0 + 1, G, full), min(MIN_WINDOW, full));
+    const Window win = window_of(K, l0, u0, t);
+    const int below = (K - 1) / G * G;
+    const int sl = s - look_ahead(s - e, lane);
+    int l, u;
+    reach_at(r, sl, min(e, t.jmax) + (sl - e), l, u);
+    const unsigned long long fits = below >= MIN_WINDOW ? __ballot(l + u + 1 <= WAVE * below) : 0ull;
+    const int at = fits ? __builtin_ctzll(fits) : WAVE - 1;
+    l0 = __builtin_amdgcn_readlane(l, at);
+    u0 = __builtin_amdgcn_readlane(u, at);
+    return ReachPhase{win, __builtin_amdgcn_readlane(sl, at)};
+}
+
+// The passes' phases in order: visit(win, nsteps, in_lo, in_hi, last), where
+// in_lo/in_hi bound the previous window's tree nodes (empty for the first
+// phase) and last marks the forward pass's final phase.
+template <int G, class Visit>
+__device__ __forceinline__ void reach_forward(const TreeShape &t, const Reach &r, int e, int lane, int &lo, int &hi,
+                                              Visit &&visit)
+{
+    int i = 0;
+    lo = hi = 0;
+    bool last;
+    do {
+        const ReachPhase p = reach_ahead<G>(t, r, i, e, lane);
+        last = p.end >= e;
+        visit(p.win, p.end - i, lo, hi, last);
+        i = p.end;
+        lo = p.win.base;
+        hi = min(p.win.base + WAVE * p.win.K, t.w);
+    } while (!last);
+}
+
+template <int G, class Visit>
+__device__ __forceinline__ void reach_backward(const TreeShape &t, const Reach &r, int n, int e, int lane, int &lo,
+                                               int &hi, Visit &&visit)
+{
     int s = n, l0, u0;
-    reach_at(r, n, ep + (n - e), l0, u0);
+    reach_at(r, n, min(e, t.jmax) + (n - e), l0, u0);
     l0 = uni(l0);
     u0 = uni(u0);
-    int in_lo = 0, in_hi = 0;
+    lo = hi = 0;
     while (s > e) {
-        const int K = max(ceil_window(l0 + u0 + 1, G, full), min(MIN_WINDOW, full));
-        const Window win = window_of(K, l0, u0, t);
-        // down to the first step looked at that fits the next window down
-        const int below = (K - 1) / G * G;
-        const int sl = s - look_ahead(s - e, lane);
-        int l, u;
-        reach_at(r, sl, ep + (sl - e), l, u);
-        const unsigned long long fits = below >= MIN_WINDOW ? __ballot(l + u + 1 <= WAVE * below) : 0ull;
-        const int at = fits ? __builtin_ctzll(fits) : WAVE - 1;
-        const int send = __builtin_amdgcn_readlane(sl, at);
-        visit(win, s - send, in_lo, in_hi, false);
-        s = send;
-        l0 = __builtin_amdgcn_readlane(l, at);
-        u0 = __builtin_amdgcn_readlane(u, at);
-        in_lo = win.base;
-        in_hi = min(win.base + WAVE * win.K, t.w);
+        const ReachPhase p = reach_back<G>(t, r, s, e, lane, l0, u0);
+        visit(p.win, s - p.end, lo, hi, false);
+        s = p.end;
+        lo = p.win.base;
+        hi = min(p.win.base + WAVE * p.win.K, t.w);
     }
-    lo = in_lo;
-    hi = in_hi;
 }
 
 // Whether a phase of window size K runs the unit-diagonal form.

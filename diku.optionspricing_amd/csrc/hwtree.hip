@@ -29,6 +29,7 @@
 // per-step reductions, against 2n steps plus n reductions in seq/Seq.hpp.
 #include "hwt_lane.h"
 #include "hwt_pipeline.h"
+#include "hwt_tri.h"
 #include "../../include/hwtree.h"
 #include "hwt_internal.h"
 
@@ -77,6 +78,14 @@ __device__ __forceinline__ int flat_bucket(int w, int n)
     return flat_part(w) * FLAT_HBUCKETS + h;
 }
 
+// FP64 part class: 72 height buckets per part, exact heights below 24, then 8
+// buckets per octave.
+__device__ __forceinline__ int tri_bucket(int part, int n)
+{
+    const int h = n < 24 ? n : min(TRI_HBUCKETS - 1, 24 + (int)(8.0f * log2_f((float)n * (1.0f / 24.0f))));
+    return part * TRI_HBUCKETS + h;
+}
+
 // The part of the row or flat class bucket b belongs to: 0..ROW_MAXK-1 the
 // row parts (nodes per lane), then the flat parts (one per width); and the
 // number of tasks a wave takes from that part at once.
@@ -86,6 +95,26 @@ __device__ __forceinline__ int part_group(int part)
     return part < ROW_MAXK ? ROWS : flat_per_wave(flat_width(part - ROW_MAXK));
 }
 constexpr int NPARTS = ROW_MAXK + FLAT_PARTS;
+
+// The two task-list layouts: mixed mode's and form 1's (the classes of
+// hwt_pipeline.h), and FP64's (TRI).
+template <bool TRI>
+struct Layout {
+    static constexpr int NB = TRI ? NBUCKET_TRI : NBUCKET;
+    static constexpr int PARTS = TRI ? TRI_PARTS : NPARTS;
+    static constexpr int TOP = TRI ? B_TRI_BIG : B_WIDE;    // first bucket of the class that comes first
+    static constexpr int SECOND = TRI ? B_TRI_WIN : B_MID;  // ... of the class after it; parts below
+    static constexpr int PER = NB / 256;                    // scan positions per thread
+    static_assert(NB % 256 == 0, "scan positions per thread");
+    static __device__ __forceinline__ int part(int b) { return TRI ? b / TRI_HBUCKETS : part_of(b); }
+    static __device__ __forceinline__ int group(int p) { return TRI ? WAVE / tri_lanes(p) : part_group(p); }
+    // a part's lowest bucket: it comes last in the scan and takes the pad
+    static __device__ __forceinline__ bool lowest(int b)
+    {
+        if (TRI) return b % TRI_HBUCKETS == 0;
+        return b >= B_ROW ? (b - B_ROW) % ROW_HBUCKETS == 0 : b % FLAT_HBUCKETS == 0;
+    }
+};
 
 // Every counter and tally to zero: the empty batch's whole pipeline.
 __global__ void k_reset(int32_t *tally)
@@ -99,8 +128,7 @@ __global__ void k_reset(int32_t *tally)
 // counters hit by every option serialise in L2).
 constexpr int SETUP_BLOCK = 256;
 constexpr int SETUP_YMAX = 2048;  // knots staged in LDS by k_setup (24 KB)
-constexpr int SCAN_PER = NBUCKET / SETUP_BLOCK;
-static_assert(NBUCKET % SETUP_BLOCK == 0, "scan positions per thread");
+static_assert(SETUP_BLOCK == 256, "Layout::PER");
 static_assert(T_FLAT_START + FLAT_PARTS + 1 <= T_T0 && T_T0 + 2 <= T_FLAT_GROUP &&
                   T_FLAT_GROUP + FLAT_PARTS + 1 <= T_XFLOP && T_XPLAIN + 2 <= T_END && N_END <= SETUP_BLOCK,
               "tally layout");
@@ -108,12 +136,15 @@ static_assert(T_FLAT_START + FLAT_PARTS + 1 <= T_T0 && T_T0 + 2 <= T_FLAT_GROUP 
 // Bucket at scan position p: the wide class, then the mid class, each largest
 // key first unless an ascending order was asked for, then the row class by
 // decreasing (K, height), then the flat class by decreasing (width, height).
+// (FP64: big, window, then the parts by decreasing (part, height).)
+template <bool TRI>
 __device__ __forceinline__ int scan_bucket(int p, int asc)
 {
-    constexpr int NW = NBUCKET - B_WIDE, NM = B_WIDE - B_MID;
-    if (p < NW) return asc ? B_WIDE + p : NBUCKET - 1 - p;
-    if (p < NW + NM) return asc ? B_MID + (p - NW) : B_WIDE - 1 - (p - NW);
-    return NBUCKET - 1 - p;
+    using Y = Layout<TRI>;
+    constexpr int NW = Y::NB - Y::TOP, NM = Y::TOP - Y::SECOND;
+    if (p < NW) return asc ? Y::TOP + p : Y::NB - 1 - p;
+    if (p < NW + NM) return asc ? Y::SECOND + (p - NW) : Y::TOP - 1 - (p - NW);
+    return Y::NB - 1 - p;
 }
 
 // Run by every block of k_order (SETUP_BLOCK threads), after k_setup: the
@@ -127,31 +158,33 @@ __device__ __forceinline__ int scan_bucket(int p, int asc)
 // -1), so every group a wave takes shares one K or one width and an option's
 // arithmetic never depends on which options share its wave.  The flat parts'
 // first tasks and first group numbers go to the tally for the flat kernel.
+template <bool TRI>
 __device__ __forceinline__ void scan_offsets(const int32_t *__restrict__ hist, int32_t *soffs,
                                              int32_t *__restrict__ order, int32_t *__restrict__ tally, int32_t asc,
                                              int32_t classes, bool writer)
 {
     const int tid = threadIdx.x;
-    constexpr int NW = NBUCKET - B_WIDE, NM = B_WIDE - B_MID, NR = B_MID - B_ROW;
-    __shared__ int32_t ptot[NPARTS];  // options per part
-    __shared__ int32_t ppad[NPARTS];  // idle slots that round each part up to whole groups
+    using Y = Layout<TRI>;
+    constexpr int NW = Y::NB - Y::TOP, NM = Y::TOP - Y::SECOND, NR = B_MID - B_ROW, SCAN_PER = Y::PER;
+    __shared__ int32_t ptot[Y::PARTS];  // options per part
+    __shared__ int32_t ppad[Y::PARTS];  // idle slots that round each part up to whole groups
     __shared__ int32_t wtot[SETUP_BLOCK / WAVE];
     __shared__ int32_t nrow_end;
     int idx[SCAN_PER], cnt[SCAN_PER];
 #pragma unroll
     for (int q = 0; q < SCAN_PER; ++q) {
-        idx[q] = scan_bucket(tid * SCAN_PER + q, asc);
+        idx[q] = scan_bucket<TRI>(tid * SCAN_PER + q, asc);
         cnt[q] = hist[idx[q]];
     }
-    if (tid < NPARTS) ptot[tid] = 0;
+    if (tid < Y::PARTS) ptot[tid] = 0;
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < SCAN_PER; ++q)
-        if (idx[q] < B_MID && cnt[q]) atomicAdd(&ptot[part_of(idx[q])], cnt[q]);
+        if (idx[q] < Y::SECOND && cnt[q]) atomicAdd(&ptot[Y::part(idx[q])], cnt[q]);
     __syncthreads();
     // one thread per part works out its pad (a division by the part's group)
-    if (tid < NPARTS) {
-        const int g = part_group(tid);
+    if (tid < Y::PARTS) {
+        const int g = Y::group(tid);
         ppad[tid] = classes ? (g - ptot[tid] % g) % g : 0;
     }
     __syncthreads();
@@ -160,8 +193,7 @@ __device__ __forceinline__ void scan_offsets(const int32_t *__restrict__ hist, i
 #pragma unroll
     for (int q = 0; q < SCAN_PER; ++q) {
         const int b = idx[q];
-        const bool lowest = b < B_MID && (b >= B_ROW ? (b - B_ROW) % ROW_HBUCKETS == 0 : b % FLAT_HBUCKETS == 0);
-        pad[q] = lowest ? ppad[part_of(b)] : 0;
+        pad[q] = b < Y::SECOND && Y::lowest(b) ? ppad[Y::part(b)] : 0;
         v[q] = cnt[q] + pad[q];
         sum += v[q];
     }
@@ -185,18 +217,53 @@ __device__ __forceinline__ void scan_offsets(const int32_t *__restrict__ hist, i
         run += v[q];
         if (writer) {
             for (int j = 0; j < pad[q]; ++j) order[run - pad[q] + j] = -1;
-            if (p == NW - 1) tally[T_NLARGE] = run;
-            if (p == NW + NM - 1) tally[T_NMID] = run;
-            if (p == NW + NM + NR - 1) {
-                tally[T_NROW] = run;
-                nrow_end = run;
+            if (TRI) {
+                if (p == NW - 1) tally[T_TBIG] = run;
+                if (p == NW + NM - 1) {
+                    tally[T_TWIN] = run;
+                    nrow_end = run;
+                }
+            } else {
+                if (p == NW - 1) tally[T_NLARGE] = run;
+                if (p == NW + NM - 1) tally[T_NMID] = run;
+                if (p == NW + NM + NR - 1) {
+                    tally[T_NROW] = run;
+                    nrow_end = run;
+                }
             }
-            if (p == NBUCKET - 1) tally[T_NTASK] = run;
+            if (p == Y::NB - 1) tally[T_NTASK] = run;
         }
     }
     __syncthreads();  // orders nrow_end above before thread 0 reads it
     if (writer && tid < N_END) reinterpret_cast<unsigned long long *>(tally + T_END)[tid] = 0;
-    if (writer && tid == 0) {
+    if (TRI && writer && tid < 2 * TRI_QUEUES) tally[T_TQWIN + 32 * tid] = 0;
+    if (TRI && writer && tid < WAVE) {
+        // parts in task order, highest first: first task and first group, by
+        // a scan over the lanes
+        const int p = Y::PARTS - 1 - lane;
+        const int size = p >= 0 ? ptot[p] + ppad[p] : 0, groups = p >= 0 ? size / Y::group(p) : 0;
+        int start = size, group = groups, npad = p >= 0 ? ppad[p] : 0;
+#pragma unroll
+        for (int off = 1; off < WAVE; off <<= 1) {
+            const int t = __shfl_up(start, off, WAVE), g = __shfl_up(group, off, WAVE), d = __shfl_up(npad, off, WAVE);
+            if (lane >= off) {
+                start += t;
+                group += g;
+                npad += d;
+            }
+        }
+        if (p >= 0) {
+            tally[T_TSTART + lane] = nrow_end + start - size;
+            tally[T_TGROUP + lane] = group - groups;
+        }
+        if (lane == WAVE - 1) {
+            tally[T_TNGROUP] = group;
+            tally[T_NPAD] = npad;
+            tally[T_NLARGE] = tally[A_NWIDE];
+            tally[A_NWIDE] = 0;
+        }
+    }
+    if (!TRI && writer && tid == 0) {
         // flat parts in task order, widest first: first task and first group
         int start = nrow_end, group = 0, npad = 0;
 #pragma unroll
@@ -214,6 +281,8 @@ __device__ __forceinline__ void scan_offsets(const int32_t *__restrict__ hist, i
         tally[T_FLAT_GROUP + FLAT_PARTS] = group;
         tally[T_NFLATG] = group;
         tally[T_NPAD] = npad;
+    }
+    if (writer && tid == 0) {
         tally[T_QUEUE] = 0;
         tally[T_QUEUE_S] = 0;
         tally[T_QUEUE_R] = 0;
@@ -240,11 +309,18 @@ __device__ __forceinline__ void scan_offsets(const int32_t *__restrict__ hist, i
 // records out as contiguous 1 KB rows instead of one 16-byte piece per lane
 // and store (25.7 -> 22.7 us on the 60k skewed batch).  The kernel is bound
 // by writing its 24.6 MB, not by its arithmetic.
-constexpr int REC_TAB = EDGE_TAB / 2;                 // 16-byte units per edge table
-constexpr int REC_CST = (int)(sizeof(OptConst) / 16); // ... per constants record
-constexpr int STAGE_LANES = WAVE / 2;                 // tables staged per round
-constexpr int STAGE_UNITS = STAGE_LANES * REC_TAB;    // per wave: 9 KB
-static_assert(sizeof(OptConst) % 16 == 0 && WAVE * REC_CST <= STAGE_UNITS, "constants fit one round");
+// FP64 plans write the ten-entry edge record instead of the table, 176 bytes
+// per option in place of 384.
+template <bool TRI>
+struct Record {
+    static constexpr int TAB_DOUBLES = TRI ? TRI_EDGE : EDGE_TAB;
+    static constexpr int TAB = TAB_DOUBLES / 2;                // 16-byte units per edge table or record
+    static constexpr int CST = (int)(sizeof(OptConst) / 16);   // ... per constants record
+    static constexpr int ROUNDS = TRI ? 1 : 2;                 // tables staged in this many rounds
+    static constexpr int LANES = WAVE / ROUNDS;
+    static constexpr int UNITS = LANES * TAB > WAVE * CST ? LANES * TAB : WAVE * CST;  // per wave: 9 KB, TRI 6 KB
+};
+static_assert(sizeof(OptConst) % 16 == 0, "whole units");
 
 // Orders this wave's LDS accesses on either side (the staging slice is the
 // wave's own, so no other wave takes part).
@@ -280,18 +356,22 @@ __device__ __forceinline__ void copy_out(u32x4 *__restrict__ dst, const u32x4 *s
         if (lane + r * WAVE < units) dst[lane + r * WAVE] = v[r];
 }
 
+template <bool TRI>
 __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, int32_t sort, int32_t maxWidth,
-                                                       double unit_dmin, int32_t classes, int32_t reach,
+                                                       double unit_dmin, int32_t classes, int32_t spread,
+                                                       int32_t reprice,
                                                        OptConst *__restrict__ cst, double *__restrict__ edge,
                                                        int2 *__restrict__ slot, int32_t *__restrict__ hist,
                                                        int32_t *__restrict__ tally, double *__restrict__ out)
 {
-    __shared__ int32_t lh[NBUCKET];  // the block's histogram, then its first rank in each bucket
+    using Y = Layout<TRI>;
+    using R = Record<TRI>;
+    __shared__ int32_t lh[Y::NB];  // the block's histogram, then its first rank in each bucket
     __shared__ unsigned long long lsum[3];  // work, seq work, wide work
-    __shared__ int32_t lbad[2];             // invalid, unsupported
+    __shared__ int32_t lbad[3];             // invalid, unsupported, wide
     __shared__ double yr[SETUP_YMAX];       // the yield curve, staged once per block
     __shared__ int32_t yd[SETUP_YMAX];
-    __shared__ u32x4 stage[SETUP_BLOCK / WAVE][STAGE_UNITS];
+    __shared__ u32x4 stage[SETUP_BLOCK / WAVE][R::UNITS];
     const int tid = threadIdx.x;
     const int lane = tid % WAVE;
     const int i = tid + blockIdx.x * SETUP_BLOCK;
@@ -314,9 +394,9 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, in
         sigma = o.sigma[i];
         type = o.type[i];
     }
-    for (int k = tid; k < NBUCKET; k += SETUP_BLOCK) lh[k] = 0;
+    for (int k = tid; k < Y::NB; k += SETUP_BLOCK) lh[k] = 0;
     if (tid < 3) lsum[tid] = 0ull;
-    if (tid < 2) lbad[tid] = 0;
+    if (tid < 3) lbad[tid] = 0;
     // Curves that fit are read from LDS, by binary search when their days
     // never decrease (every real curve); anything else keeps the reference's
     // linear scan over global memory.  Both give the same value.
@@ -337,11 +417,11 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, in
         return sorted ? yield_at_sorted(t, tu, yr, yd, y.n) : yield_at(t, tu, y.rate, y.day, y.n);
     };
     OptConst c{};
-    double tab[EDGE_TAB];  // the edge table; zeros for options that have none
+    double tab[R::TAB_DOUBLES];  // the edge table (TRI: record); zeros for options that have none
 #pragma unroll
-    for (int k = 0; k < EDGE_TAB; ++k) tab[k] = 0.0;
+    for (int k = 0; k < R::TAB_DOUBLES; ++k) tab[k] = 0.0;
     unsigned long long work = 0, seq_work = 0, wide_work = 0;
-    bool invalid = false, unsupported = false;
+    bool invalid = false, unsupported = false, is_wide = false;
     int b = -1, r = 0;  // bucket, rank among the block's options in it
     if (mine) {
         int32_t st;
@@ -371,10 +451,16 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, in
                 const double te = c.e * c.dt;
                 c.Pe = exp(-yield(te, tu) * te);
                 TreeShape t{c.w, c.jmax, c.M, c.dr, c.dt, 0.0, 0.0};
-                // trees of 7 or more nodes (all but the tiniest) take their
-                // edge discounts from four exponentials and the table from
-                // its closed form
-                if (t.w >= 7) {
+                TriEdge edges{};
+                if constexpr (TRI) {
+                    const EdgeDiscounts ed = edge_discounts(t);
+                    edge_factors(t, ed);
+                    edges = tri_edge(t, ed);
+                    __builtin_memcpy(tab, &edges, sizeof(edges));
+                } else if (t.w >= 7) {
+                    // trees of 7 or more nodes (all but the tiniest) take their
+                    // edge discounts from four exponentials and the table from
+                    // its closed form
                     const EdgeDiscounts ed = edge_discounts(t);
                     edge_factors(t, ed);
                     edge_table_closed(t, ed, tab);
@@ -389,23 +475,44 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, in
                 }
                 c.rho = t.rho;
                 c.rhop = t.rhop;
-                const bool wide = (c.w + WAVE - 1) / WAVE > KSMALL;
                 work = (unsigned long long)dual_node_updates(c.n, c.e, c.jmax);
                 seq_work = (unsigned long long)seq_node_updates(c.n, c.jmax);
-                // FP64 prices a wide tree over the nodes that carry weight
-                int64_t nodes = (int64_t)work;
-                if (wide && reach) {
-                    c.sigmas = window_sigmas(c);
-                    nodes = (int64_t)reach_updates(make_reach(c.sigmas, c.M, c.dr, c.dt, c.n, c.jmax), c.n, c.e);
+                const bool wide = (c.w + WAVE - 1) / WAVE > KSMALL;
+                is_wide = wide;
+                if (!TRI && wide && reprice) c.sigmas = window_sigmas(c);  // should FP64 price it again
+                int64_t key = (int64_t)work;
+                bool grouped = false, held = false;  // TRI: a part's tree; the tridiagonal form holds it
+                if constexpr (TRI) {
+                    grouped = c.w <= (spread ? TRI_SPREAD_WIDTH : TRI_GROUP_WIDTH);
+                    int lo = c.jmax, up = c.jmax;
+                    if (!grouped) {
+                        // priced over the nodes that carry weight, most at step n
+                        c.sigmas = window_sigmas(c);
+                        const Reach reach = make_reach(c.sigmas, c.M, c.dr, c.dt, c.n, c.jmax);
+                        key = (int64_t)reach_updates(reach, c.n, c.e);
+                        reach_at(reach, c.n, min(c.e, c.jmax) + (c.n - c.e), lo, up);
+                    }
+                    held = tri_ok(t, edges, c.n, max(lo, up), grouped ? 100.0f : 200.0f) &&
+                           (grouped || lo + up + 17 <= TRI_MAX_NODES);
+                    if (!held) {
+                        // the general kernel's scales (unit_form_ok)
+                        double etab[EDGE_TAB];
+                        edge_table(t, etab);
+                        c.unit = unit_form_ok(t, etab, unit_dmin) ? 1 : 0;
+                        c.sigmas = window_sigmas(c);
+                    }
                 }
-                int64_t key;
                 switch (sort) {
                 case 'W': case 'w': key = c.w; break;
                 case 'H': case 'h': key = c.n; break;
                 case '-': key = 0; break;
-                default: key = nodes; break;
+                default: break;
                 }
-                if (wide) b = B_WIDE + log_bucket(key, 8, NBUCKET - B_WIDE);
+                if (TRI) {
+                    if (!held) b = B_TRI_BIG + log_bucket(key, 2, NBUCKET_TRI - B_TRI_BIG);
+                    else if (!grouped) b = B_TRI_WIN + log_bucket(key, 8, B_TRI_BIG - B_TRI_WIN);
+                    else b = tri_bucket(tri_part(c.w, spread != 0), c.n);
+                } else if (wide) b = B_WIDE + log_bucket(key, 8, NBUCKET - B_WIDE);
                 else if ((classes & CLASS_FLAT) && c.w <= FLAT_MAX_WIDTH) b = flat_bucket(c.w, c.n);
                 else if (c.w > ROW_MAX_WIDTH || !(classes & CLASS_ROWS)) b = B_MID + log_bucket(key, 4, B_WIDE - B_MID);
                 else b = row_bucket(c.w, c.n);
@@ -421,26 +528,29 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, in
     wide_work = wave_total_count(wide_work);
     const int n_invalid = __popcll(__ballot(invalid));
     const int n_unsup = __popcll(__ballot(unsupported));
+    const int n_wide = __popcll(__ballot(is_wide));
     if (lane == 0) {
         if (work) atomicAdd(&lsum[0], work);
         if (seq_work) atomicAdd(&lsum[1], seq_work);
         if (wide_work) atomicAdd(&lsum[2], wide_work);
         if (n_invalid) atomicAdd(&lbad[0], n_invalid);
         if (n_unsup) atomicAdd(&lbad[1], n_unsup);
+        if (TRI && n_wide) atomicAdd(&lbad[2], n_wide);
     }
     // The block's slots in each bucket: the global histogram's old value is
     // the block's first rank there.  Requested after the first round of the
     // copy-out below and read after the last, so the atomics' round trip
     // overlaps the rest of it; requested before the first round, they held
     // its stores back (k_setup 26.5 -> 24.8 us on the 60k skewed batch).
+    constexpr int SCAN_PER = Y::PER;
     int first_rank[SCAN_PER];
     // the wave's records out through its LDS slice: edge tables in two rounds
     // of 32 lanes, then the constants
     const int first = i - lane;  // the wave's first option
     const int count = max(0, min(WAVE, nopt - first));
     u32x4 *slice = stage[tid / WAVE];
-    for (int half = 0; half < 2; ++half) {
-        if (half == 1) {
+    for (int half = 0; half < R::ROUNDS; ++half) {
+        if (half == R::ROUNDS - 1) {
             __syncthreads();  // every lane's LDS histogram count is in
 #pragma unroll
             for (int q = 0; q < SCAN_PER; ++q) {
@@ -448,27 +558,27 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, in
                 first_rank[q] = lh[k] ? atomicAdd(&hist[k], lh[k]) : 0;
             }
         }
-        if (lane / STAGE_LANES == half) {
-            u32x4 u[REC_TAB];
+        if (lane / R::LANES == half) {
+            u32x4 u[R::TAB];
             __builtin_memcpy(u, tab, sizeof(u));
-            u32x4 *r = slice + (lane % STAGE_LANES) * REC_TAB;
+            u32x4 *r = slice + (lane % R::LANES) * R::TAB;
 #pragma unroll
-            for (int k = 0; k < REC_TAB; ++k) r[k] = u[k];
+            for (int k = 0; k < R::TAB; ++k) r[k] = u[k];
         }
         wave_lds_order();
-        const int recs = max(0, min(STAGE_LANES, count - half * STAGE_LANES));
-        copy_out<STAGE_UNITS>(reinterpret_cast<u32x4 *>(edge) + (size_t)(first + half * STAGE_LANES) * REC_TAB,
-                              slice, recs * REC_TAB, lane);
+        const int recs = max(0, min(R::LANES, count - half * R::LANES));
+        copy_out<R::LANES * R::TAB>(reinterpret_cast<u32x4 *>(edge) + (size_t)(first + half * R::LANES) * R::TAB,
+                                    slice, recs * R::TAB, lane);
         wave_lds_order();
     }
     {
-        u32x4 u[REC_CST];
+        u32x4 u[R::CST];
         __builtin_memcpy(u, &c, sizeof(u));
-        u32x4 *r = slice + lane * REC_CST;
+        u32x4 *r = slice + lane * R::CST;
 #pragma unroll
-        for (int k = 0; k < REC_CST; ++k) r[k] = u[k];
+        for (int k = 0; k < R::CST; ++k) r[k] = u[k];
         wave_lds_order();
-        copy_out<WAVE * REC_CST>(reinterpret_cast<u32x4 *>(cst) + (size_t)first * REC_CST, slice, count * REC_CST,
+        copy_out<WAVE * R::CST>(reinterpret_cast<u32x4 *>(cst) + (size_t)first * R::CST, slice, count * R::CST,
                                  lane);
     }
 #pragma unroll
@@ -481,6 +591,7 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, in
         if (lsum[2]) atomicAdd((unsigned long long *)&tally[A_WORKW], lsum[2]);
         if (lbad[0]) atomicAdd(&tally[A_INVALID], lbad[0]);
         if (lbad[1]) atomicAdd(&tally[A_UNSUP], lbad[1]);
+        if (lbad[2]) atomicAdd(&tally[A_NWIDE], lbad[2]);
     }
 }
 
@@ -491,17 +602,18 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, in
 // k_setup's blocks reached the histogram (options are independent).  One
 // kernel instead of a scan kernel and a scatter kernel saves a kernel
 // boundary per execution.
+template <bool TRI>
 __global__ __launch_bounds__(SETUP_BLOCK) void k_order(int32_t n, const int32_t *__restrict__ count,
                                                        const int2 *__restrict__ slot,
                                                        const int32_t *__restrict__ hist, int32_t *__restrict__ order,
                                                        int32_t *__restrict__ tally, int32_t asc, int32_t classes)
 {
-    __shared__ int32_t soffs[NBUCKET];
+    __shared__ int32_t soffs[Layout<TRI>::NB];
     const int tid = threadIdx.x;
     const int i = tid + blockIdx.x * SETUP_BLOCK;
     if (count) n = min(*count, n);
     const int2 s = (i < n) ? slot[i] : make_int2(-1, 0);  // requested first, so it arrives during the scan
-    scan_offsets(hist, soffs, order, tally, asc, classes, blockIdx.x == 0);
+    scan_offsets<TRI>(hist, soffs, order, tally, asc, classes, blockIdx.x == 0);
     if (s.x >= 0) order[soffs[s.x] + s.y] = i;
 }
 
@@ -509,19 +621,25 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_order(int32_t n, const int32_t 
 // included (cone_forward / cone_backward; mixed mode executes these, the FP64
 // kernel about half of them, Reach): operations (per lane and step 4K+1 in
 // the unit-diagonal form, 5K in the plain one) and node slots (64 K per step)
-// per form.  One thread per wide task; run at sync time, never in the
-// timed pipeline.
+// per form.  One thread per option; run at sync time, never in the timed
+// pipeline.
 __global__ __launch_bounds__(256) void k_count_steps(const OptConst *__restrict__ cst,
-                                                     const int32_t *__restrict__ order, int32_t *__restrict__ tally,
-                                                     int32_t mixed)
+                                                     int32_t n, int32_t *__restrict__ tally, int32_t mixed,
+                                                     double unit_dmin)
 {
     __shared__ unsigned long long part[3];
     if (threadIdx.x < 3) part[threadIdx.x] = 0;
     __syncthreads();
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < tally[T_NLARGE]) {
-        const OptConst c = cst[order[i]];
+    if (i < n && cst[i].status == ST_OK && cst[i].n > 0 && cst[i].e >= 0 && (cst[i].w + WAVE - 1) / WAVE > KSMALL) {
+        OptConst c = cst[i];
         const TreeShape t{c.w, c.jmax, c.M, c.dr, c.dt, c.rho, c.rhop};
+        if (!mixed) {  // FP64 plans keep no tables and check the unit form's scales only where they use it
+            const EdgeDiscounts ed = edge_discounts(t);
+            double tab[EDGE_TAB];
+            edge_table_closed(t, ed, tab);
+            c.unit = unit_form_ok(t, tab, unit_dmin, ed.E0, ed.Ea) ? 1 : 0;
+        }
         unsigned long long ops = 0, slots[2] = {0, 0};
         auto count = [&](const Window &win, int nsteps, int, int, bool) {
             const bool u = mixed ? unit_phase<float>(win.K, c.unit != 0) : unit_phase<double>(win.K, c.unit != 0);
@@ -662,7 +780,7 @@ struct hwt_plan {
     hipStream_t stream = nullptr;
     int32_t capacity = 0, ycap = 0;
     hwt_config cfg{};
-    int grid_wide = 0, grid_narrow = 0, grid_fused = 0;
+    int grid_wide = 0, grid_narrow = 0, grid_fused = 0, grid_tri = 0;
     hipStream_t side = nullptr;       // narrow-tree kernel runs here, concurrently
     hipEvent_t fork = nullptr, join = nullptr;
     double *scratch_wide = nullptr;
@@ -699,6 +817,18 @@ struct hwt_plan {
 
 static std::atomic<uint64_t> g_plan_serial{0};
 
+// Whether a plan of these settings prices through the tridiagonal form.
+static bool plan_tri(const hwt_config &c) { return c.form != HWT_FORM_LANE && c.precision == HWT_PREC_FP64; }
+
+// Resident waves per CU of a persistent pricing kernel (one wave per workgroup).
+template <class Kernel>
+static int waves_per_cu(Kernel *k, int fallback)
+{
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void *)k, WAVE, 0) != hipSuccess || n < 1) n = fallback;
+    return n;
+}
+
 static int launch_pipeline(hwt_plan *p, const DevOpts &o, const DevYield &y, double *out, hipStream_t s, bool time_kernel)
 {
     const int n = o.n;
@@ -719,13 +849,39 @@ static int launch_pipeline(hwt_plan *p, const DevOpts &o, const DevYield &y, dou
                                 ? 0
                                 : ((p->cfg.flags & HWT_FLAG_NO_ROWS) ? 0 : CLASS_ROWS) |
                                       ((p->cfg.flags & HWT_FLAG_NO_FLAT) ? 0 : CLASS_FLAT);
-        const int reach = p->cfg.form != HWT_FORM_LANE && p->cfg.precision == HWT_PREC_FP64 ? 1 : 0;
         // the lane form prices tasks one per lane: no row or flat groups, no pads
         // form 1 prices trees up to its column length; wider ones are unsupported
         const int max_width = p->cfg.form == HWT_FORM_LANE ? p->lane_width : WAVE_MAX_WIDTH;
-        k_setup<<<blocks, SETUP_BLOCK, 0, s>>>(o, y, sort, max_width, unit_dmin, classes, reach, p->cst, p->edge,
-                                               p->slot, p->hist, p->tally, out);
-        k_order<<<blocks, SETUP_BLOCK, 0, s>>>(n, o.count, p->slot, p->hist, p->order, p->tally, asc, classes);
+        const bool tri = plan_tri(p->cfg);
+        if (tri) {
+            k_setup<true><<<blocks, SETUP_BLOCK, 0, s>>>(o, y, sort, max_width, unit_dmin, CLASS_ROWS,
+                                                         n <= TRI_SPREAD ? 1 : 0, 0, p->cst, p->edge, p->slot, p->hist,
+                                                         p->tally, out);
+            k_order<true><<<blocks, SETUP_BLOCK, 0, s>>>(n, o.count, p->slot, p->hist, p->order, p->tally, asc,
+                                                         CLASS_ROWS);
+            if (time_kernel) {
+                HWT_HIP(hipEventRecord(p->evk0, s));
+                HWT_HIP(hipEventRecord(p->evw0, s));
+            }
+            k_price_wide<double><<<std::min(p->grid_wide, n), WAVE, 0, s>>>(p->cst, nullptr, p->order, p->tally, out,
+                                                                            p->scratch_wide, nullptr);
+            // no more waves than options: a small batch's launch would mostly
+            // start waves that find nothing (1,000 options: 41 -> 22 us)
+            k_price_tri<<<std::min(p->grid_tri, n), WAVE, 0, s>>>(p->cst, p->edge, p->order, p->tally, out,
+                                                                  p->scratch_wide);
+            if (time_kernel) {
+                HWT_HIP(hipEventRecord(p->evw1, s));
+                HWT_HIP(hipEventRecord(p->evn0, s));  // no separate narrow kernel: narrow_ms ~ 0
+                HWT_HIP(hipEventRecord(p->evn1, s));
+                HWT_HIP(hipEventRecord(p->evk1, s));
+            }
+            HWT_HIP(hipGetLastError());
+            return HWT_OK;
+        }
+        k_setup<false><<<blocks, SETUP_BLOCK, 0, s>>>(o, y, sort, max_width, unit_dmin, classes, 0,
+                                                      p->cfg.precision == HWT_PREC_MIXED ? 1 : 0, p->cst, p->edge,
+                                                      p->slot, p->hist, p->tally, out);
+        k_order<false><<<blocks, SETUP_BLOCK, 0, s>>>(n, o.count, p->slot, p->hist, p->order, p->tally, asc, classes);
         if (time_kernel) HWT_HIP(hipEventRecord(p->evk0, s));
         if (p->cfg.form == HWT_FORM_LANE) {
             const int lb = p->lane_block;
@@ -735,15 +891,11 @@ static int launch_pipeline(hwt_plan *p, const DevOpts &o, const DevYield &y, dou
             HWT_HIP(hipGetLastError());
             return HWT_OK;
         }
-        const bool mixed = p->cfg.precision == HWT_PREC_MIXED;
+        // mixed mode
         if (p->cfg.flags & HWT_FLAG_FUSED) {
             if (time_kernel) HWT_HIP(hipEventRecord(p->evw0, s));
-            if (mixed)
-                k_price_fused<float><<<p->grid_fused, WAVE, 0, s>>>(p->cst, p->edge, p->order, p->tally, out,
-                                                                    p->scratch_wide, p->redo);
-            else
-                k_price_fused<double><<<p->grid_fused, WAVE, 0, s>>>(p->cst, p->edge, p->order, p->tally, out,
-                                                                     p->scratch_wide, p->redo);
+            k_price_fused<float><<<p->grid_fused, WAVE, 0, s>>>(p->cst, p->edge, p->order, p->tally, out,
+                                                                p->scratch_wide, p->redo);
             if (time_kernel) {
                 HWT_HIP(hipEventRecord(p->evw1, s));
                 HWT_HIP(hipEventRecord(p->evn0, s));  // no separate narrow kernel: narrow_ms ~ 0
@@ -759,30 +911,20 @@ static int launch_pipeline(hwt_plan *p, const DevOpts &o, const DevYield &y, dou
                 HWT_HIP(hipStreamWaitEvent(p->side, p->fork, 0));
             }
             if (time_kernel) HWT_HIP(hipEventRecord(p->evw0, s));
-            if (mixed)
-                k_price_wide<float><<<p->grid_wide, WAVE, 0, s>>>(p->cst, p->edge, p->order, p->tally, out,
-                                                                  p->scratch_wide, p->redo);
-            else
-                k_price_wide<double><<<p->grid_wide, WAVE, 0, s>>>(p->cst, p->edge, p->order, p->tally, out,
-                                                                   p->scratch_wide, p->redo);
+            k_price_wide<float><<<p->grid_wide, WAVE, 0, s>>>(p->cst, p->edge, p->order, p->tally, out,
+                                                              p->scratch_wide, p->redo);
             if (time_kernel) HWT_HIP(hipEventRecord(p->evw1, s));
             if (time_kernel) HWT_HIP(hipEventRecord(p->evn0, ns));
-            if (mixed)
-                k_price_narrow<float><<<p->grid_narrow, WAVE, 0, ns>>>(p->cst, p->edge, p->order, p->tally, out,
-                                                                       p->redo);
-            else
-                k_price_narrow<double><<<p->grid_narrow, WAVE, 0, ns>>>(p->cst, p->edge, p->order, p->tally, out,
-                                                                        p->redo);
+            k_price_narrow<float><<<p->grid_narrow, WAVE, 0, ns>>>(p->cst, p->edge, p->order, p->tally, out, p->redo);
             if (time_kernel) HWT_HIP(hipEventRecord(p->evn1, ns));
             if (!serial) {
                 HWT_HIP(hipEventRecord(p->join, p->side));
                 HWT_HIP(hipStreamWaitEvent(s, p->join, 0));
             }
         }
-        // mixed mode: FP64 re-pricing of the options whose FP32 state left its
-        // range, after every FP32 kernel has handed its options over
-        if (mixed)
-            k_price_redo<<<p->grid_redo, WAVE, 0, s>>>(p->cst, p->edge, p->redo, p->tally, out, p->scratch_wide);
+        // FP64 re-pricing of the options whose FP32 state left its range, after
+        // every FP32 kernel has handed its options over
+        k_price_redo<<<p->grid_redo, WAVE, 0, s>>>(p->cst, p->edge, p->redo, p->tally, out, p->scratch_wide);
         if (time_kernel) HWT_HIP(hipEventRecord(p->evk1, s));
     }
     HWT_HIP(hipGetLastError());
@@ -858,40 +1000,22 @@ int hwt_plan_create(hwt_plan **out, int32_t capacity, int32_t yield_capacity, co
         hipEventCreateWithFlags(&p->join, hipEventDisableTiming) != hipSuccess)
         return bail(HWT_EHIP, "hipEventCreate failed");
     // Persistent grids: as many single-wave workgroups as can be resident.
-    int cus = 0, per_cu_w = 0, per_cu_n = 0;
+    int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) != hipSuccess || cus < 1)
         cus = 256;
-    const bool mixed = p->cfg.precision == HWT_PREC_MIXED;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu_w, mixed ? (const void *)k_price_wide<float> : (const void *)k_price_wide<double>, WAVE, 0) !=
-            hipSuccess ||
-        per_cu_w < 1)
-        per_cu_w = 8;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu_n, mixed ? (const void *)k_price_narrow<float> : (const void *)k_price_narrow<double>, WAVE, 0) !=
-            hipSuccess ||
-        per_cu_n < 1)
-        per_cu_n = 8;
+    const bool mixed = p->cfg.precision == HWT_PREC_MIXED, tri = plan_tri(p->cfg);
+    int per_cu_w = mixed ? waves_per_cu(k_price_wide<float>, 8) : waves_per_cu(k_price_wide<double>, 8);
+    int per_cu_n = mixed ? waves_per_cu(k_price_narrow<float>, 8) : waves_per_cu(k_price_tri, 8);
     if (p->cfg.wide_per_cu > 0) per_cu_w = std::min(per_cu_w, p->cfg.wide_per_cu);
     if (p->cfg.narrow_per_cu > 0) per_cu_n = std::min(per_cu_n, p->cfg.narrow_per_cu);
     p->grid_wide = per_cu_w * cus;
-    p->grid_narrow = per_cu_n * cus;
-    // the fused kernel shares the wide kernel's scratch slots, so its grid
-    // never exceeds the wide kernel's
-    int per_cu_f = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu_f, mixed ? (const void *)k_price_fused<float> : (const void *)k_price_fused<double>, WAVE, 0) !=
-            hipSuccess ||
-        per_cu_f < 1)
-        per_cu_f = per_cu_w;
-    p->grid_fused = std::min(per_cu_f, per_cu_w) * cus;
-    // mixed mode's FP64 re-pricing kernel shares the wide kernel's scratch
-    // slots as well
-    int per_cu_x = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_x, (const void *)k_price_redo, WAVE, 0) != hipSuccess ||
-        per_cu_x < 1)
-        per_cu_x = 1;
-    p->grid_redo = std::min(per_cu_x, per_cu_w) * cus;
+    p->grid_narrow = p->grid_tri = per_cu_n * cus;
+    // mixed mode's fused and FP64 re-pricing kernels share the wide kernel's
+    // scratch slots, so their grids never exceed the wide kernel's
+    if (mixed) {
+        p->grid_fused = std::min(waves_per_cu(k_price_fused<float>, per_cu_w), per_cu_w) * cus;
+        p->grid_redo = std::min(waves_per_cu(k_price_redo, 1), per_cu_w) * cus;
+    }
     if (const char *v = getenv("HWT_VERBOSE"); v && *v && *v != '0')
         fprintf(stderr, "hwtree plan: device %d, %d CUs, wide kernel %d blocks (%d/CU), narrow kernel %d blocks (%d/CU)\n",
                 p->device, cus, p->grid_wide, per_cu_w, p->grid_narrow, per_cu_n);
@@ -903,13 +1027,15 @@ int hwt_plan_create(hwt_plan **out, int32_t capacity, int32_t yield_capacity, co
         return at;
     };
     const size_t o_cst = carve(cap * sizeof(OptConst));
-    const size_t o_edge = carve(cap * EDGE_TAB * sizeof(double));
+    const size_t o_edge = carve(cap * (tri ? TRI_EDGE : EDGE_TAB) * sizeof(double));
     const size_t o_slot = carve(cap * sizeof(int2));
     const size_t o_order = carve((cap + MAX_PADS) * sizeof(int32_t));  // + row and flat pads
     const size_t o_tally = carve(T_ALLOC * sizeof(int32_t));  // with the histogram
     const bool lane = p->cfg.form == HWT_FORM_LANE;
-    // the wide-tree kernels' parked forward states (form 2 only)
-    const size_t o_scw = carve(lane ? 0 : (size_t)p->grid_wide * WAVE * MAXK * sizeof(double));
+    // the parked forward states of the wide trees' waves (form 2 only); the
+    // kernels that park run one after the other and share it
+    const size_t wide_nodes = (size_t)p->grid_wide * WAVE * MAXK, tri_nodes = tri ? (size_t)p->grid_tri * TRI_MAX_NODES : 0;
+    const size_t o_scw = carve(lane ? 0 : std::max(wide_nodes, tri_nodes) * sizeof(double));
     const size_t o_redo = carve(p->cfg.precision == HWT_PREC_MIXED ? cap * sizeof(int32_t) : 0);
     if (lane) {
         const int bs = p->cfg.block_size;
@@ -1067,8 +1193,9 @@ int hwt_plan_sync(hwt_plan *p, hwt_stats *stats)
     // execution, counted once from its schedule (form 2 only)
     if (stats && !p->steps_counted && p->last_n > 0 && p->cfg.form != HWT_FORM_LANE) {
         (void)hipGetLastError();
-        k_count_steps<<<(p->last_n + 255) / 256, 256, 0, s>>>(p->cst, p->order, p->tally,
-                                                             p->cfg.precision == HWT_PREC_MIXED ? 1 : 0);
+        k_count_steps<<<(p->last_n + 255) / 256, 256, 0, s>>>(p->cst, p->last_n, p->tally,
+                                                             p->cfg.precision == HWT_PREC_MIXED ? 1 : 0,
+                                                             UnitRange<double>::dmin);
         HWT_HIP(hipGetLastError());
         p->steps_counted = true;
     }
@@ -1536,11 +1663,12 @@ int hwt_price_constants_f32(const hwt_option_constants_f32 *consts, int32_t n, c
 // order[N + row pads], counters with the histogram, and the wide-tree kernel's parked forward states (one
 // 64 x MAXK double slot per resident wave, at most NOALLOC_WIDE_SLOTS).
 constexpr int NOALLOC_MAX_OPTIONS = HWT_NOALLOC_MAX_OPTIONS;
-constexpr int NOALLOC_WIDE_SLOTS = 1024;
+constexpr int NOALLOC_WIDE_SLOTS = 2048;
+constexpr int NOALLOC_TRI_SLOTS = NOALLOC_WIDE_SLOTS * (WAVE * MAXK) / TRI_MAX_NODES;
 constexpr size_t noalloc_part(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 constexpr size_t NOALLOC_O_CST = 0;
 constexpr size_t NOALLOC_O_EDGE = NOALLOC_O_CST + noalloc_part((size_t)NOALLOC_MAX_OPTIONS * sizeof(OptConst));
-constexpr size_t NOALLOC_O_SLOT = NOALLOC_O_EDGE + noalloc_part((size_t)NOALLOC_MAX_OPTIONS * EDGE_TAB * 8);
+constexpr size_t NOALLOC_O_SLOT = NOALLOC_O_EDGE + noalloc_part((size_t)NOALLOC_MAX_OPTIONS * TRI_EDGE * 8);
 constexpr size_t NOALLOC_O_ORDER = NOALLOC_O_SLOT + noalloc_part((size_t)NOALLOC_MAX_OPTIONS * sizeof(int2));
 constexpr size_t NOALLOC_O_TALLY = NOALLOC_O_ORDER + noalloc_part(((size_t)NOALLOC_MAX_OPTIONS + MAX_PADS) * 4);
 constexpr size_t NOALLOC_O_WIDE = NOALLOC_O_TALLY + noalloc_part(T_ALLOC * 4);
@@ -1555,7 +1683,7 @@ namespace {
 // memory), and the persistent grids, which need occupancy queries.
 struct NoallocDevice {
     unsigned char *ptr = nullptr;
-    int grid_wide = 0, grid_narrow = 0;
+    int grid_wide = 0, grid_tri = 0;
 };
 constexpr int NOALLOC_MAX_DEVICES = 64;
 std::mutex g_noalloc_mu;
@@ -1571,19 +1699,11 @@ int noalloc_device(int dev, NoallocDevice &out)
         const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
         if (e != hipSuccess || !ptr)
             return fail(HWT_EHIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
-        int cus = 0, per_w = 0, per_n = 0;
+        int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
             cus = 256;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_w, (const void *)k_price_wide<double>, WAVE, 0) !=
-                hipSuccess ||
-            per_w < 1)
-            per_w = 2;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_n, (const void *)k_price_narrow<double>, WAVE, 0) !=
-                hipSuccess ||
-            per_n < 1)
-            per_n = 4;
-        d.grid_wide = std::min(per_w * cus, NOALLOC_WIDE_SLOTS);
-        d.grid_narrow = per_n * cus;
+        d.grid_wide = std::min(waves_per_cu(k_price_wide<double>, 2) * cus, NOALLOC_WIDE_SLOTS);
+        d.grid_tri = std::min(waves_per_cu(k_price_tri, 4) * cus, NOALLOC_TRI_SLOTS);
         d.ptr = (unsigned char *)ptr;
     }
     out = d;
@@ -1614,7 +1734,7 @@ int hwt_price_device_noalloc(const hwt_options_f64 *dopts, const hwt_yield_f64 *
     hwt_config_init(&v.cfg);
     v.device = dev;
     v.grid_wide = d.grid_wide;
-    v.grid_narrow = d.grid_narrow;
+    v.grid_tri = d.grid_tri;
     v.cst = (OptConst *)(d.ptr + NOALLOC_O_CST);
     v.edge = (double *)(d.ptr + NOALLOC_O_EDGE);
     v.slot = (int2 *)(d.ptr + NOALLOC_O_SLOT);
@@ -1917,3 +2037,8 @@ static_assert(ROW_MAXK * (ROWS - 1) + [] {
     for (int p = 0; p < FLAT_PARTS; ++p) pads += flat_per_wave(flat_width(p)) - 1;
     return pads;
 }() <= MAX_PADS, "task-list room for the row and flat padding");
+static_assert([] {
+    int pads = 0;
+    for (int p = 0; p < TRI_PARTS; ++p) pads += WAVE / tri_lanes(p) - 1;
+    return pads;
+}() <= MAX_PADS, "task-list room for the FP64 parts' padding");

@@ -101,6 +101,8 @@ typedef struct {
 /* Launch the plan's kernels one by one instead of replaying its HIP graph;
  * hwt_stats.kernel_ms then times the pricing kernel alone. */
 #define HWT_FLAG_NO_GRAPH 1
+/* The next four choose between arrangements of mixed mode's pricing kernels;
+ * FP64 prices every tree in one persistent kernel and takes them as given. */
 /* Form 2: price trees up to 64 nodes wide one per wavefront instead of four
  * per wavefront (16-lane rows). */
 #define HWT_FLAG_NO_ROWS  2
@@ -132,7 +134,8 @@ typedef struct {
                                  its start to the last pricing wavefront's end (the
                                  first kernel's launch is not included); 0 for an
                                  empty batch. */
-    double  wide_ms;          /* wide-tree pricing kernel alone (HWT_FLAG_NO_GRAPH), else 0 */
+    double  wide_ms;          /* wide-tree pricing kernel alone (HWT_FLAG_NO_GRAPH), else 0;
+                                 FP64: the kernels that price every tree */
     double  narrow_ms;        /* narrow-tree pricing kernel alone (HWT_FLAG_NO_GRAPH), else 0 */
     int64_t device_memory;    /* bytes of device memory held by the plan */
     int64_t node_updates;     /* tree nodes between the root and the exercise and bond dates that

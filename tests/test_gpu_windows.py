@@ -50,3 +50,29 @@ def test_windows_price_the_whole_tree(pkg, oracle, kind):
     print(f"\n{kind}: {tail.sum()} prices from {ref[tail].min():.1e}, max relative error {rel.max():.2e}")
     assert rel.max() <= 1e-10, np.nonzero(rel > 1e-10)[0][:5]
     assert np.all(np.abs(got[fin] - ref[fin]) <= parity_tol(ref[fin]))
+
+
+@pytest.mark.parametrize("n", [400, 17000], ids=["spread", "packed"])
+def test_groups_price_every_width(pkg, oracle, n):
+    """Every odd width from 3 to 181 (the lane groups of L = 1 to 16, their
+    K = 2 to 11, the first windows beyond), heights from one step to 300 in one
+    batch, exercise from step 0 to the last: against the oracle as above.  n
+    decides how many lanes a tree gets (TRI_SPREAD)."""
+    r = np.random.default_rng(23)
+    width = np.resize(np.arange(3, 182, 2), n)
+    a = np.where(width == 3, 3.0, -np.log1p(-0.184 / (width // 2 - 0.5)) * 12)
+    h = r.integers(1, 301, n)
+    h[: width.size // 4] = r.integers(1, 6, width.size // 4)
+    e = np.where(r.uniform(size=n) < 0.1, 0, (r.uniform(size=n) * h).astype(int))
+    opts = pkg.Options(strike=r.uniform(60, 100, n), maturity=(h + 0.5) / 12, length=(e + 0.5) / 12,
+                       term_unit=np.full(n, 365, np.uint16), term_steps=np.full(n, 12, np.uint16), a=a,
+                       sigma=r.uniform(0.001, 0.05, n), type=r.integers(0, 2, n).astype(np.int8))
+    y = pkg.datasets.synthetic_yield()
+    got = pkg.capi.price(opts, y)
+    sub = np.arange(0, n, max(1, n // 1500))
+    assert {oracle.constants(opts, int(i)).width for i in np.arange(min(n, 90))} == set(range(3, 182, 2))
+    ref = oracle.price(opts.take(sub), y)
+    tail = ref > 1e-250
+    rel = np.abs(got[sub][tail] - ref[tail]) / ref[tail]
+    assert rel.max() <= 1e-10, (width[sub][tail][rel.argmax()], rel.max())
+    assert np.all(np.abs(got[sub] - ref) <= parity_tol(ref))
