@@ -62,17 +62,18 @@ __device__ __forceinline__ TriEdge tri_edge(const TreeShape &t, const EdgeDiscou
 }
 
 // Whether a tree stepped over `half` nodes either side of the root stays in
-// range: ln d1 and ln d2 change by at most ln of the least 6 p (at x = half M)
-// and by the discounts' exponent per node, the state by 6 e^{h half} per step,
-// rescaled every 64 steps; and the scales exist (nonzero entries) where the
-// edges are inside.  `lim` bounds |ln d|: 200 for windows (normalised at the root),
-// 100 for groups (normalised at node 0), so that products of two scales and a
-// state stay below e^700.
+// range.  Going out, ln d1 and ln d2 change per node by at most -ln(1 - 3x + 3x^2)
+// at x = j |M|, which is convex up to x = 1/4 (so at most half of its last value on
+// average), and by the discount's j h; the state by 6 e^{h half} per step, scaled back
+// as it goes.  The scales have to exist (entries away from zero) where the edges
+// are inside.  `lim` bounds |ln d|: 200 where the scales are normalised at the root,
+// 100 for groups, which normalise at node 0, so that products of two scales and
+// a state stay below e^700.
 __device__ __forceinline__ bool tri_ok(const TreeShape &t, const TriEdge &e, int n, int half, float lim)
 {
-    const float x = (float)half * (float)-t.M, h = (float)(t.dr * t.dt);
+    const float x = (float)half * (float)-t.M, h = (float)(t.dr * t.dt), mean = x <= 0.25f ? 0.5f : 1.0f;
     const float per = -0.69314718f * log2_f(fminf(1.0f, 1.0f - 3.0f * x + 3.0f * x * x));
-    bool ok = (float)half * (per + h * (float)half) <= lim && h * (float)half <= 0.5f &&
+    bool ok = (float)half * (mean * per + 0.5f * h * (float)(half + 1)) <= lim && h * (float)half <= 0.5f &&
               (float)n * h * (float)half <= 300.0f && x < 0.75f;
     if (half >= t.jmax)
         ok = ok && fabs(e.d1_0) > 1e-6 && fabs(e.d1_0) < 1e6 && fabs(e.d2_t) > 1e-6 && fabs(e.d2_t) < 1e6 &&

@@ -660,8 +660,10 @@ __global__ __launch_bounds__(256) void k_count_steps(const OptConst *__restrict_
 }
 
 // Form 1: one lane per option over every scheduled task (tasks ordered by
-// decreasing work, so the lanes of a wave carry similar trees).
-__global__ void k_price_lane(const OptConst *__restrict__ cst, const double *__restrict__ edge,
+// decreasing work, so the lanes of a wave carry similar trees).  BLOCK: the most
+// lanes per workgroup (1,024 leaves 128 VGPRs, too few for eight steps a sweep).
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_price_lane(const OptConst *__restrict__ cst, const double *__restrict__ edge,
                              const int32_t *__restrict__ order, int32_t *__restrict__ tally,
                              double *__restrict__ out, double *__restrict__ cols, int32_t colw)
 {
@@ -671,8 +673,11 @@ __global__ void k_price_lane(const OptConst *__restrict__ cst, const double *__r
     if (o >= 0) {
         const OptConst c = cst[o];
         double *base = cols + (size_t)(gid / WAVE) * (2 * (size_t)colw * WAVE) + (gid % WAVE);
-        out[o] = lane_price(c, edge + (size_t)o * EDGE_TAB, LaneColumn{base},
-                            LaneColumn{base + (size_t)colw * WAVE});
+        const LaneColumn Y{base}, B{base + (size_t)colw * WAVE};
+        const TreeShape t{c.w, c.jmax, c.M, c.dr, c.dt, c.rho, c.rhop};
+        const TriEdge ed = tri_edge(t, edge_discounts(t));
+        out[o] = tri_ok(t, ed, c.n, c.jmax, 200.0f) ? lane_price_tri<BLOCK <= 256 ? 8 : 4>(c, t, ed, Y, B)
+                                                    : lane_price(c, edge + (size_t)o * EDGE_TAB, Y, B);
     }
     stamp_wave_end(tally);
 }
@@ -787,7 +792,7 @@ struct hwt_plan {
     int32_t *redo = nullptr;  // mixed mode: options re-priced in FP64
     int grid_redo = 0;
     double *cols = nullptr;  // form 1 tree columns
-    int lane_block = 256;
+    int lane_block = LANE_BLOCK;
     int lane_width = LANE_MAX_WIDTH;  // form 1: column length, the widest tree priced
     // device workspace, one allocation
     void *ws = nullptr;
@@ -885,8 +890,12 @@ static int launch_pipeline(hwt_plan *p, const DevOpts &o, const DevYield &y, dou
         if (time_kernel) HWT_HIP(hipEventRecord(p->evk0, s));
         if (p->cfg.form == HWT_FORM_LANE) {
             const int lb = p->lane_block;
-            k_price_lane<<<(n + lb - 1) / lb, lb, 0, s>>>(p->cst, p->edge, p->order, p->tally, out, p->cols,
-                                                          p->lane_width);
+            if (lb <= 256)
+                k_price_lane<256><<<(n + lb - 1) / lb, lb, 0, s>>>(p->cst, p->edge, p->order, p->tally, out, p->cols,
+                                                                   p->lane_width);
+            else
+                k_price_lane<1024><<<(n + lb - 1) / lb, lb, 0, s>>>(p->cst, p->edge, p->order, p->tally, out, p->cols,
+                                                                    p->lane_width);
             if (time_kernel) HWT_HIP(hipEventRecord(p->evk1, s));
             HWT_HIP(hipGetLastError());
             return HWT_OK;
@@ -1039,7 +1048,7 @@ int hwt_plan_create(hwt_plan **out, int32_t capacity, int32_t yield_capacity, co
     const size_t o_redo = carve(p->cfg.precision == HWT_PREC_MIXED ? cap * sizeof(int32_t) : 0);
     if (lane) {
         const int bs = p->cfg.block_size;
-        p->lane_block = (bs >= WAVE && bs <= 1024 && bs % WAVE == 0) ? bs : 256;
+        p->lane_block = (bs >= WAVE && bs <= 1024 && bs % WAVE == 0) ? bs : LANE_BLOCK;
         const int lw = p->cfg.lane_max_width;
         p->lane_width = (lw > 0 && lw < LANE_MAX_WIDTH) ? lw : LANE_MAX_WIDTH;
     }

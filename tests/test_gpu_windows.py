@@ -76,3 +76,24 @@ def test_groups_price_every_width(pkg, oracle, n):
     rel = np.abs(got[sub][tail] - ref[tail]) / ref[tail]
     assert rel.max() <= 1e-10, (width[sub][tail][rel.argmax()], rel.max())
     assert np.all(np.abs(got[sub] - ref) <= parity_tol(ref))
+
+
+@pytest.mark.parametrize("block", [0, 512])
+def test_lane_form_sweeps(pkg, oracle, block):
+    """Form 1 steps its columns several steps to a sweep: every count of steps
+    from 0 to 40 in both passes, columns narrower and wider than a chunk, both
+    workgroup sizes' kernels, and trees that leave the tridiagonal form."""
+    h, e = np.meshgrid(np.arange(1, 42), np.arange(0, 41))
+    h, e = h[e < h], e[e < h]
+    n = h.size
+    r = np.random.default_rng(29)
+    width = np.resize([3, 5, 7, 9, 15, 17, 19, 25, 47, 61, 127], n)
+    a = np.where(width == 3, 3.0, -np.log1p(-0.184 / (width // 2 - 0.5)) * 12)
+    sigma = np.where(np.arange(n) % 9 == 0, 4.0, r.uniform(0.001, 0.05, n))
+    opts = pkg.Options(strike=r.uniform(60, 100, n), maturity=(h + 0.5) / 12, length=(e + 0.5) / 12,
+                       term_unit=np.full(n, 365, np.uint16), term_steps=np.full(n, 12, np.uint16), a=a, sigma=sigma,
+                       type=r.integers(0, 2, n).astype(np.int8))
+    y = pkg.datasets.synthetic_yield()
+    got = pkg.capi.price(opts, y, pkg.capi.config(form=pkg.capi.FORM_LANE, block_size=block))
+    ref = oracle.price(opts, y)
+    assert np.all(np.abs(got - ref) <= parity_tol(ref)), np.nonzero(~(np.abs(got - ref) <= parity_tol(ref)))[0][:5]
