@@ -23,7 +23,7 @@ FLAG_NO_GRAPH, FLAG_NO_ROWS, FLAG_CONCURRENT, FLAG_FUSED, FLAG_NO_FLAT, FLAG_DIR
 
 # The exported C symbols, in include/hwtree.h order.
 EXPORTS = (
-    "hwt_config_init", "hwt_price_f64", "hwt_plan_create", "hwt_plan_execute",
+    "hwt_config_init", "hwt_price_f64", "hwt_trim", "hwt_plan_create", "hwt_plan_execute",
     "hwt_plan_sync", "hwt_plan_destroy", "hwt_price_f32", "hwt_price_constants_f64", "hwt_price_constants_f32",
     "hwt_batch_create", "hwt_batch_create_f32", "hwt_batch_price", "hwt_batch_device_memory", "hwt_batch_destroy",
     "hwt_price_device_noalloc", "hwt_alphas_f64", "hwt_autotune", "hwt_max_width", "hwt_strerror",
@@ -109,6 +109,8 @@ def lib():
         L.hwt_config_init.argtypes = [C.POINTER(ConfigC)]
         L.hwt_config_init.restype = None
         L.hwt_price_f64.argtypes = [C.POINTER(OptionsC), C.POINTER(YieldC), P, C.POINTER(ConfigC), C.POINTER(StatsC)]
+        L.hwt_trim.argtypes = []
+        L.hwt_trim.restype = None
         L.hwt_plan_create.argtypes = [C.POINTER(P), C.c_int32, C.c_int32, C.POINTER(ConfigC)]
         L.hwt_plan_execute.argtypes = [P, C.POINTER(OptionsC), C.POINTER(YieldC), P, P]
         L.hwt_plan_sync.argtypes = [P, C.POINTER(StatsC)]
@@ -169,9 +171,14 @@ def price(opts: Options, y: Yield, cfg: ConfigC | None = None, stats: bool = Fal
     out = np.empty(opts.N, dtype=np.float64)
     st = StatsC()
     rc = lib().hwt_price_f64(C.byref(_host_opts(opts)), C.byref(_host_yield(y)), out.ctypes.data,
-                             C.byref(cfg) if cfg is not None else None, C.byref(st))
+                             C.byref(cfg) if cfg is not None else None, C.byref(st) if stats else None)
     _check(rc)
     return (out, st.as_dict()) if stats else out
+
+
+def trim() -> None:
+    """hwt_trim: gives back the idle workspaces that one-shot calls keep."""
+    lib().hwt_trim()
 
 
 def price_status(opts: Options, y: Yield, cfg: ConfigC | None = None):
@@ -195,7 +202,7 @@ def price_f32(opts: Options, y: Yield, cfg: ConfigC | None = None, stats: bool =
     out = np.empty(opts.N, dtype=np.float32)
     st = StatsC()
     _check(lib().hwt_price_f32(C.byref(o), C.byref(yc), out.ctypes.data, C.byref(cfg) if cfg is not None else None,
-                               C.byref(st)))
+                               C.byref(st) if stats else None))
     return (out, st.as_dict()) if stats else out
 
 
@@ -251,7 +258,7 @@ class Batch:
         out = np.empty(self.N, dtype=np.float64)
         st = StatsC()
         _check(lib().hwt_batch_price(self._b, out.ctypes.data, C.byref(cfg) if cfg is not None else None,
-                                     C.byref(st)))
+                                     C.byref(st) if stats else None))
         return (out, st.as_dict()) if stats else out
 
     @property

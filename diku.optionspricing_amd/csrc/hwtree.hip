@@ -49,6 +49,7 @@
 #include <mutex>
 #include <sstream>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 using namespace hwt;
@@ -940,6 +941,19 @@ static int launch_pipeline(hwt_plan *p, const DevOpts &o, const DevYield &y, dou
     return HWT_OK;
 }
 
+// hipMalloc; when memory is short, again after the idle one-shot workspaces have
+// been given back.
+static hipError_t dev_malloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        hwt_trim();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
 extern "C" {
 
 void hwt_config_init(hwt_config *cfg)
@@ -1055,7 +1069,7 @@ int hwt_plan_create(hwt_plan **out, int32_t capacity, int32_t yield_capacity, co
     const size_t lane_waves = lane ? (cap + WAVE - 1) / WAVE : 0;
     const size_t o_cols = carve(lane_waves * 2 * (size_t)p->lane_width * WAVE * sizeof(double));
     p->ws_bytes = off;
-    if (hipMalloc(&p->ws, p->ws_bytes) != hipSuccess) return bail(HWT_ENOMEM, "hipMalloc workspace failed");
+    if (dev_malloc(&p->ws, p->ws_bytes) != hipSuccess) return bail(HWT_ENOMEM, "hipMalloc workspace failed");
     char *base = (char *)p->ws;
     p->cst = (OptConst *)(base + o_cst);
     p->edge = (double *)(base + o_edge);
@@ -1208,7 +1222,6 @@ int hwt_plan_sync(hwt_plan *p, hwt_stats *stats)
         HWT_HIP(hipGetLastError());
         p->steps_counted = true;
     }
-    HWT_HIP(hipStreamSynchronize(s));
     // the tallies are fetched here, once, rather than by a copy queued behind
     // every execution: back-to-back executions then run without a transfer
     // between them
@@ -1280,7 +1293,7 @@ static int upload(const hwt_options_f64 *h, const hwt_yield_f64 *hy, DeviceBatch
     const size_t o_strike = carve(n * 8), o_mat = carve(n * 8), o_len = carve(n * 8), o_tu = carve(n * 2),
                  o_ts = carve(n * 2), o_a = carve(n * 8), o_sig = carve(n * 8), o_type = carve(n),
                  o_rate = carve(ny * 8), o_day = carve(ny * 4), o_out = carve(need_out ? n * 8 : 0);
-    if (hipMalloc(&d.mem, std::max<size_t>(off, 256)) != hipSuccess) return fail(HWT_ENOMEM, "hipMalloc batch failed");
+    if (dev_malloc(&d.mem, std::max<size_t>(off, 256)) != hipSuccess) return fail(HWT_ENOMEM, "hipMalloc batch failed");
     d.bytes = std::max<size_t>(off, 256);
     char *b = (char *)d.mem;
     auto put = [&](size_t at, const void *src, size_t bytes) {
@@ -1382,7 +1395,7 @@ static int batch_of_constants(hwt_batch *b, const hwt_option_constants_f64 *k, i
     auto part = [](size_t bytes) { return (bytes + 255) & ~(size_t)255; };
     const size_t cb = part((size_t)n * sizeof(*k)), rb = part(ny * 8), db = part(ny * 4);
     const size_t bytes = cb + rb + db + part((size_t)n * 8);
-    if (hipMalloc(&b->cmem, bytes) != hipSuccess) return fail(HWT_ENOMEM, "hipMalloc constants batch failed");
+    if (dev_malloc(&b->cmem, bytes) != hipSuccess) return fail(HWT_ENOMEM, "hipMalloc constants batch failed");
     b->bytes = bytes;
     char *base = (char *)b->cmem;
     auto *dc = (hwt_option_constants_f64 *)base;
@@ -1478,7 +1491,233 @@ static int widen_f32(const hwt_options_f32 *opts, const hwt_yield_f32 *yield, st
     return HWT_OK;
 }
 
+// ------------------------------------------------------- one-shot workspaces
+// What a one-shot call on host arrays needs beside its arguments: a plan, device
+// memory for its inputs and prices, and pinned host memory to send and fetch them
+// as one copy each.  Making these, and ten pageable copies, took 440 of the 490 us
+// of a five-option call (51 us from an idle workspace), so a call leaves its
+// workspace behind for the next one on the same device and settings: at most IDLE and
+// IDLE_BYTES in all, the least recently used given back first, all of them by
+// hwt_trim or when a device allocation of this library fails.  A workspace belongs
+// to one call at a time, which waits for its stream before it lets go.  Calls above
+// MAX_OPTIONS, whose pinned copies would be large, and form 1, whose columns fit one
+// batch, allocate for themselves.
+namespace {
+
+struct OneShot {
+    static constexpr int MAX_OPTIONS = 1 << 17;
+    static constexpr size_t IDLE = 4, IDLE_BYTES = (size_t)512 << 20;
+    int device = 0, cap = 0, ycap = 0;
+    hwt_config cfg{};
+    hwt_plan *plan = nullptr;
+    char *dmem = nullptr, *hmem = nullptr;
+    size_t bytes = 0;
+    ~OneShot()
+    {
+        if (plan) hwt_plan_destroy(plan);
+        if (dmem) (void)hipFree(dmem);
+        if (hmem) (void)hipHostFree(hmem);
+    }
+    size_t held() const { return bytes + plan->ws_bytes; }
+};
+
+std::mutex g_idle_mu;
+// most recently used last; never destroyed, since the HIP runtime may be gone first
+std::vector<OneShot *> &idle_workspaces()
+{
+    static auto *v = new std::vector<OneShot *>();
+    return *v;
+}
+
+int32_t round_up_pow2(int32_t v, int32_t least)
+{
+    int32_t r = least;
+    while (r < v) r *= 2;
+    return r;
+}
+
+constexpr size_t part256(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+
+int one_shot_acquire(const hwt_config &c, int32_t n, int32_t ny, OneShot *&out)
+{
+    out = nullptr;
+    int dev = 0;
+    HWT_HIP(hipGetDevice(&dev));
+    {
+        std::lock_guard<std::mutex> lk(g_idle_mu);
+        auto &v = idle_workspaces();
+        size_t best = v.size();
+        for (size_t i = 0; i < v.size(); ++i)
+            if (v[i]->device == dev && v[i]->cap >= n && v[i]->ycap >= ny && std::memcmp(&v[i]->cfg, &c, sizeof(c)) == 0 &&
+                (best == v.size() || v[i]->cap < v[best]->cap))
+                best = i;
+        if (best < v.size()) {
+            out = v[best];
+            v.erase(v.begin() + (std::ptrdiff_t)best);
+        }
+    }
+    // a device reset since the last call has taken the workspace with it
+    if (out && hipStreamQuery(out->plan->stream) != hipSuccess) {
+        (void)hipGetLastError();
+        out = nullptr;
+    }
+    if (out) return HWT_OK;
+    OneShot *s = new (std::nothrow) OneShot();
+    if (!s) return fail(HWT_ENOMEM, "one-shot workspace: host allocation");
+    s->device = dev;
+    s->cfg = c;
+    s->cap = round_up_pow2(n, 1024);
+    s->ycap = round_up_pow2(std::min(ny, 1 << 30), 256);
+    int rc = hwt_plan_create(&s->plan, s->cap, s->ycap, &c);
+    if (rc == HWT_OK) {
+        // raw options (45 bytes) or constants (56), curve, prices, each part on a
+        // 256-byte line
+        static_assert(sizeof(hwt_option_constants_f64) <= 64, "input bytes per option");
+        s->bytes = part256((size_t)s->cap * 64 + (size_t)s->ycap * 12 + (size_t)s->cap * 8 + 16 * 256);
+        if (dev_malloc((void **)&s->dmem, s->bytes) != hipSuccess)
+            rc = fail(HWT_ENOMEM, "one-shot workspace: hipMalloc failed");
+        else if (hipHostMalloc((void **)&s->hmem, s->bytes, hipHostMallocDefault) != hipSuccess)
+            rc = fail(HWT_ENOMEM, "one-shot workspace: hipHostMalloc failed");
+    }
+    if (rc) {
+        delete s;
+        return rc;
+    }
+    out = s;
+    return HWT_OK;
+}
+
+void one_shot_release(OneShot *s)
+{
+    std::vector<OneShot *> out;
+    try {
+        std::lock_guard<std::mutex> lk(g_idle_mu);
+        auto &v = idle_workspaces();
+        v.reserve(OneShot::IDLE + 1);
+        out.reserve(v.size() + 1);
+        size_t held = s->held();
+        for (OneShot *w : v) held += w->held();
+        while (!v.empty() && (v.size() >= OneShot::IDLE || held > OneShot::IDLE_BYTES)) {
+            out.push_back(v.front());
+            held -= v.front()->held();
+            v.erase(v.begin());
+        }
+        if (held > OneShot::IDLE_BYTES) out.push_back(s);
+        else v.push_back(s);
+    } catch (const std::bad_alloc &) {
+        out.clear();
+        delete s;
+        return;
+    }
+    for (OneShot *w : out) delete w;
+}
+
+bool one_shot_fits(const hwt_config &c, int32_t n, int32_t ny)
+{
+    return c.form != HWT_FORM_LANE && n <= OneShot::MAX_OPTIONS && ny <= OneShot::MAX_OPTIONS;
+}
+
+// One call: fill(h, d, o, y) lays the inputs out in the pinned memory at h, points
+// o and y at their places from d on in device memory and returns their bytes
+// (whole 256s); take(prices) reads the result.
+template <class Fill, class Take>
+int one_shot(hwt_config c, int32_t n, int32_t ny, hwt_stats *stats, Fill &&fill, Take &&take)
+{
+    c.flags |= HWT_FLAG_NO_GRAPH;  // one execution: a graph would not be replayed
+    c.device = -1;
+    OneShot *s = nullptr;
+    int rc = one_shot_acquire(c, n, ny, s);
+    if (rc) return rc;
+    DevOpts o{};
+    DevYield y{};
+    const size_t in = fill(s->hmem, s->dmem, o, y);
+    double *dout = (double *)(s->dmem + in), *hout = (double *)(s->hmem + in);
+    hipStream_t st = s->plan->stream;
+    hipError_t e = hipMemcpyAsync(s->dmem, s->hmem, in, hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) {
+        // the event records that time the kernels only for a caller who asks
+        s->plan->last_stream = st;
+        s->plan->last_n = n;
+        s->plan->steps_counted = false;
+        rc = launch_pipeline(s->plan, o, y, dout, st, stats != nullptr);
+        if (rc == HWT_OK) e = hipMemcpyAsync(hout, dout, (size_t)n * 8, hipMemcpyDeviceToHost, st);
+    }
+    if (rc || e != hipSuccess) {
+        (void)hipStreamSynchronize(st);
+        delete s;
+        return rc ? rc : fail(HWT_EHIP, std::string("one-shot copy: ") + hipGetErrorString(e));
+    }
+    rc = hwt_plan_sync(s->plan, stats);
+    if (rc == HWT_EHIP) {
+        delete s;
+        return rc;
+    }
+    take((const double *)hout);
+    one_shot_release(s);
+    return rc;
+}
+
+// Host SoA options and curve into a workspace.
+size_t place_options(const hwt_options_f64 &h, const hwt_yield_f64 &hy, char *hm, char *dm, DevOpts &o, DevYield &y)
+{
+    const size_t n = (size_t)h.n, ny = (size_t)hy.n;
+    size_t off = 0;
+    auto put = [&](const auto *src, size_t count) {
+        using T = std::remove_cv_t<std::remove_reference_t<decltype(*src)>>;
+        if (count) std::memcpy(hm + off, src, count * sizeof(T));
+        const T *at = (const T *)(dm + off);
+        off += part256(count * sizeof(T));
+        return at;
+    };
+    o.n = h.n;
+    o.strike = put(h.strike, n);
+    o.maturity = put(h.maturity, n);
+    o.length = put(h.length, n);
+    o.term_unit = put(h.term_unit, n);
+    o.term_steps = put(h.term_steps, n);
+    o.a = put(h.a, n);
+    o.sigma = put(h.sigma, n);
+    o.type = put(h.type, n);
+    y.n = hy.n;
+    y.rate = put(hy.rate, ny);
+    y.day = put(hy.day, ny);
+    return off;
+}
+
+// n constants, each from constant(i), and the curve (rate(i) widened) likewise.
+template <class Constant, class Rate>
+size_t place_constants(int32_t n, Constant &&constant, int32_t ny, Rate &&rate, const int32_t *day, bool f32, char *hm,
+                       char *dm, DevOpts &o, DevYield &y)
+{
+    auto *k = (hwt_option_constants_f64 *)hm;
+    for (int32_t i = 0; i < n; ++i) k[i] = constant(i);
+    o.n = n;
+    o.consts = (const hwt_option_constants_f64 *)dm;
+    o.consts_f32 = f32 ? 1 : 0;
+    size_t off = part256((size_t)n * sizeof(*k));
+    auto *r = (double *)(hm + off);
+    for (int32_t i = 0; i < ny; ++i) r[i] = rate(i);
+    y.n = ny;
+    y.rate = (const double *)(dm + off);
+    off += part256((size_t)ny * 8);
+    if (ny) std::memcpy(hm + off, day, (size_t)ny * 4);
+    y.day = (const int32_t *)(dm + off);
+    return off + part256((size_t)ny * 4);
+}
+
+} // namespace
+
 extern "C" {
+
+void hwt_trim(void)
+{
+    std::vector<OneShot *> out;
+    {
+        std::lock_guard<std::mutex> lk(g_idle_mu);
+        out.swap(idle_workspaces());
+    }
+    for (OneShot *w : out) delete w;
+}
 
 int hwt_batch_create(hwt_batch **out, const hwt_options_f64 *opts, const hwt_yield_f64 *yield)
 {
@@ -1576,6 +1815,11 @@ int hwt_price_f64(const hwt_options_f64 *opts, const hwt_yield_f64 *yield, doubl
     if (rc) return rc;
     if (stats) std::memset(stats, 0, sizeof(*stats));
     if (opts->n == 0) return HWT_OK;
+    if (one_shot_fits(c, opts->n, yield->n))
+        return one_shot(
+            c, opts->n, yield->n, stats,
+            [&](char *h, char *d, DevOpts &o, DevYield &y) { return place_options(*opts, *yield, h, d, o, y); },
+            [&](const double *p) { std::memcpy(out_prices, p, (size_t)opts->n * 8); });
     hwt_batch *b = nullptr;
     rc = hwt_batch_create(&b, opts, yield);
     if (rc) return rc;
@@ -1599,6 +1843,14 @@ static int price_constants(const hwt_option_constants_f64 *consts, int32_t n, co
     if (rc) return rc;
     if (stats) std::memset(stats, 0, sizeof(*stats));
     if (n == 0) return HWT_OK;
+    if (one_shot_fits(c, n, yield->n))
+        return one_shot(
+            c, n, yield->n, stats,
+            [&](char *h, char *d, DevOpts &o, DevYield &y) {
+                return place_constants(n, [&](int32_t i) { return consts[i]; }, yield->n,
+                                       [&](int32_t i) { return yield->rate[i]; }, yield->day, f32, h, d, o, y);
+            },
+            [&](const double *p) { std::memcpy(host_out, p, (size_t)n * 8); });
     hwt_batch *b = nullptr;
     rc = new_batch(&b, b);
     if (rc) return rc;
@@ -1617,6 +1869,29 @@ int hwt_price_f32(const hwt_options_f32 *opts, const hwt_yield_f32 *yield, float
     g_last_error.clear();
     if (!valid_opts_f32(opts) || !valid_yield_f32(yield) || (opts->n > 0 && !out_prices))
         return fail(HWT_EINVAL, "hwt_price_f32: null or negative-size argument");
+    hwt_config c;
+    if (cfg) c = *cfg;
+    else hwt_config_init(&c);
+    if (opts->n > 0 && one_shot_fits(c, opts->n, yield->n)) {
+        DeviceGuard g;
+        const int rg = g.enter(c.device);
+        if (rg) return rg;
+        if (stats) std::memset(stats, 0, sizeof(*stats));
+        return one_shot(
+            c, opts->n, yield->n, stats,
+            [&](char *h, char *d, DevOpts &o, DevYield &y) {
+                return place_constants(
+                    opts->n,
+                    [&](int32_t i) {
+                        return constants_f32(opts->strike[i], opts->maturity[i], opts->length[i], opts->term_unit[i],
+                                             opts->term_steps[i], opts->a[i], opts->sigma[i], opts->type[i]);
+                    },
+                    yield->n, [&](int32_t i) { return (double)yield->rate[i]; }, yield->day, true, h, d, o, y);
+            },
+            [&](const double *p) {
+                for (int32_t i = 0; i < opts->n; ++i) out_prices[i] = (float)p[i];
+            });
+    }
     std::vector<hwt_option_constants_f64> k;
     std::vector<double> rates, prices;
     int rc = widen_f32(opts, yield, k, rates);
@@ -1784,7 +2059,7 @@ int hwt_alphas_f64(const hwt_options_f64 *opts, const hwt_yield_f64 *yield, int6
     void *mem = nullptr;
     const size_t total = (size_t)offsets[opts->n];
     const size_t bytes = total * 8 + (size_t)(opts->n + 1) * 8 + T_NCOUNT * 4;
-    if (hipMalloc(&mem, bytes) != hipSuccess) return fail(HWT_ENOMEM, "hipMalloc alphas failed");
+    if (dev_malloc(&mem, bytes) != hipSuccess) return fail(HWT_ENOMEM, "hipMalloc alphas failed");
     double *dal = (double *)mem;
     int64_t *doff = (int64_t *)(dal + total);
     int32_t *tally = (int32_t *)(doff + opts->n + 1);

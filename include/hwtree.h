@@ -169,6 +169,13 @@ void hwt_config_init(hwt_config *cfg);
 int hwt_price_f64(const hwt_options_f64 *opts, const hwt_yield_f64 *yield,
                   double *out_prices, const hwt_config *cfg, hwt_stats *stats);
 
+/* One-shot calls (hwt_price_*) on up to 131,072 options leave their plan and
+ * buffers behind for the next call on the same device with the same settings: at
+ * most four such workspaces and 512 MB in all, the least recently used given back
+ * first, and all idle ones when a device allocation of this library fails.
+ * hwt_trim gives them back at once. */
+void hwt_trim(void);
+
 /* Reusable plan over device-resident inputs (no allocation per execution;
  * the pipeline is captured into a HIP graph).  capacity = max options per
  * execution, yield_capacity = max yield knots. */
