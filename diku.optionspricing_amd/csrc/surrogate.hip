@@ -45,9 +45,9 @@ constexpr int HID = HWT_SURR_HIDDEN;
 constexpr int NPAR = HWT_SURR_NPARAMS;
 constexpr int PSTRIDE = 200192;          // per-member stride of parameter-shaped vectors
 constexpr int LAYER_W = HID * HID;        // elements of one 256x256 weight matrix
-constexpr int GEMM_ROWS = 128;            // rows per GEMM workgroup (4 waves x 32)
+constexpr int BATCH_STEP = 128;           // the batch is a multiple (DW_SPLIT parts of whole 16-row blocks)
 constexpr int DW_SPLIT = 8;               // split of the batch in the weight-gradient GEMMs
-constexpr int HEAD_ROWS = 32;             // rows per head / input-layer workgroup
+constexpr int HEAD_ROWS = 32;             // rows per partial sum of the output layer's gradients
 constexpr int INF_ROWS = 128;             // options per inference workgroup
 constexpr int ACT_LD = HID + 8;           // LDS row pitch (bf16) of the inference activations
 constexpr double RES = HWT_SURR_RESIDUAL_SCALE;
@@ -216,19 +216,15 @@ __global__ void k_gather(const float *__restrict__ X, const float *__restrict__ 
 struct Net {
     // per member, strides in elements
     float *P;          // FP32 masters [member][PSTRIDE]
-    uint16_t *Wb;      // BF16 [member][3][256*256] (layers 2..4), row-major [n][k]
-    uint16_t *WbT;     // BF16 transposes [member][3][256*256], [k][n]
+    uint16_t *Wb;      // BF16 [member][3][256*256] (layers 2..4), [n][k] in fragment order (weight_at)
+    uint16_t *WbT;     // BF16 transposes [member][3][256*256], [k][n], likewise
 };
 
 struct Acts {
     int B;                 // rows per member
     float *xb, *tb;        // [m][B][8], [m][B]
-    float *z;              // [m][4][B][256]  z1..z4
-    uint16_t *a;           // [m][3][B][256]  a1..a3 (bf16)
-    uint16_t *aT;          // [m][3][256][B]
-    float *a4;             // [m][B][256]     FP32 last hidden activation
-    uint16_t *dz;          // [m][3][B][256]  dz2..dz4 (bf16)
-    uint16_t *dzT;         // [m][3][256][B]
+    uint16_t *aT;          // [m][3][256][B]  a1..a3 (bf16), in fragment order (frag_unit)
+    uint16_t *dzT;         // [m][3][256][B]  dz2..dz4 (bf16), likewise
     float *dz1T;           // [m][256][B]
     float *y;              // [m][B] network outputs
     float *gw;             // [m][3][DW_SPLIT][256*256] weight-gradient partials (layers 2..4)
@@ -238,268 +234,403 @@ struct Acts {
     float *g;              // [m][PSTRIDE] dense gradient
 };
 
-__host__ __device__ inline size_t zoff(const Acts &s, int m, int l) { return (((size_t)m * 4 + (l - 1)) * s.B) * HID; }
 __host__ __device__ inline size_t aoff(const Acts &s, int m, int l) { return (((size_t)m * 3 + (l - 1)) * s.B) * HID; }
 __host__ __device__ inline size_t dzoff(const Acts &s, int m, int l) { return (((size_t)m * 3 + (l - 2)) * s.B) * HID; }
 
-// Input layer (FP32): z1 = W1 x + b1, a1 = silu(z1).  Block = 256 neurons x
-// HEAD_ROWS rows.
-__global__ __launch_bounds__(HID) void k_layer1(Net net, Acts s, int m0)
+// Both transposed batch arrays are kept in the order in which the weight-gradient
+// GEMM's matrix fragments read them: 16-byte units of eight batch rows of one
+// neuron, the 32 neurons of a block side by side, then the other eight rows of a
+// block of 16, then the blocks of neurons.  A fragment load is one contiguous
+// kilobyte, and so is what a wave stores.
+__host__ __device__ inline size_t frag_unit(int n, int r8)  // neuron, batch row / 8
 {
-    const int m = m0 + blockIdx.y;
-    const int n = threadIdx.x;
-    const int r0 = blockIdx.x * HEAD_ROWS;
-    __shared__ float xs[HEAD_ROWS * NIN];
-    if (n < HEAD_ROWS * NIN) xs[n] = s.xb[((size_t)m * s.B + r0) * NIN + n];
-    __syncthreads();
-    const float *P = net.P + (size_t)m * PSTRIDE;
-    float w[NIN];
-#pragma unroll
-    for (int k = 0; k < NIN; ++k) w[k] = P[HWT_SURR_W1 + n * NIN + k];
-    const float b = P[HWT_SURR_B1 + n];
-    float *z = s.z + zoff(s, m, 1);
-    uint16_t *a = s.a + aoff(s, m, 1);
-    uint16_t *aT = s.aT + aoff(s, m, 1);
-    uint32_t packed[HEAD_ROWS / 2];
-#pragma unroll
-    for (int r = 0; r < HEAD_ROWS; ++r) {
-        float acc = b;
-#pragma unroll
-        for (int k = 0; k < NIN; ++k) acc = fmaf(w[k], xs[r * NIN + k], acc);
-        const size_t row = (size_t)(r0 + r);
-        z[row * HID + n] = acc;
-        const uint16_t h = to_bf16(silu(acc));
-        a[row * HID + n] = h;
-        if (r & 1) packed[r / 2] |= (uint32_t)h << 16;
-        else packed[r / 2] = h;
-    }
-    uint4 *dst = reinterpret_cast<uint4 *>(aT + (size_t)n * s.B + r0);
-#pragma unroll
-    for (int q = 0; q < HEAD_ROWS / 8; ++q)
-        dst[q] = make_uint4(packed[4 * q], packed[4 * q + 1], packed[4 * q + 2], packed[4 * q + 3]);
+    return ((size_t)(r8 >> 1) * (HID / 32) + (n >> 5)) * 64 + (r8 & 1) * 32 + (n & 31);
+}
+// The weights likewise: element (row, k) of a 256 x 256 operand A[row][k].  (As rows
+// a fragment load was 32 pieces: inference of 475,000 rows 1196 us, now 1085.)
+__host__ __device__ inline int weight_at(int row, int k)
+{
+    return (((row >> 5) * (HID / 16) + (k >> 4)) * 64 + ((k >> 3) & 1) * 32 + (row & 31)) * 8 + (k & 7);
 }
 
-enum GemmMode { G_FWD = 0, G_FWD_LAST = 1, G_DX = 2, G_DX_FIRST = 3, G_DW = 4 };
+// Two floats to a packed BF16 pair (a in the low half), round to nearest
+// even, as one v_cvt_pk_bf16_f32 (the value-by-value form costs a convert,
+// a shift and an or per pair).
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ inline uint32_t pack_bf16x2(float a, float b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
+}
 
-struct GemmArgs {
-    const uint16_t *A;   // [M][K] (member stride sA)
-    const uint16_t *Bm;  // [N][K] (member stride sB)
-    size_t sA, sB;
-    int lda, ldb, K;     // K: reduction length handled by one workgroup
-    int kz;              // split index stride: workgroup z = member * nsplit + split
-    int nsplit;
-    int m0;              // first member
-    Net net;
-    Acts s;
-    int layer;           // forward: output layer l; DX: layer whose input gradient is formed; DW: layer
+// --- forward and backward of one tile of the batch
+// A workgroup (8 waves) takes TILE_ROWS rows of one member through the whole
+// network and back: wave w holds neurons [32w, 32w + 32) of every layer for all 64
+// rows, D[neuron][row] = W A^T on the matrix cores (A operand: weights from L2 in
+// fragment order; B operand: the layer's BF16 tile in LDS).  The FP32
+// pre-activations z1..z3 stay in the accumulator layout in registers until the
+// backward pass multiplies by their slopes, so of the 800 MB that a layer at a time
+// moves per step of 4 x 8192 rows (z, a, dz and a4 out and back, two layouts) only
+// what the weight gradients need leaves the chip: a1..a3 and dz2..dz4 (BF16) and dz1,
+// 134 MB.  Registers allow one workgroup per CU; a layer's first weights are
+// requested before the barrier that its input waits for.  4 x 8192 rows: 115 us,
+// where eight kernels took 344.
+constexpr int TILE_ROWS = 64;
+constexpr int TILE_LD = HID + 8;   // LDS row pitch (bf16): rows start 16 bytes on in the banks
+constexpr int TILE_LDF = HID + 4;  // ... of the FP32 tile
+
+typedef f32x16 Tile[2];  // value v of block rb: neuron n0 + 8 (v/4) + 4 (lane/32) + v%4, row 32 rb + lane%32
+
+// A wave's weights of one layer, TILE_AHEAD of the 16 fragments in flight.
+constexpr int TILE_AHEAD = 8;
+struct TileWeights {
+    bf16x8 w[TILE_AHEAD];
+    const uint16_t *p;
+    __device__ void start(const uint16_t *W, int n0, int lane)
+    {
+        p = W + ((size_t)(n0 >> 5) * (HID / 16) * 64 + lane) * 8;
+#pragma unroll
+        for (int k = 0; k < TILE_AHEAD; ++k) w[k] = load_frag(p + k * 64 * 8);
+    }
 };
 
-// C = A B^T on BF16 MFMA, FP32 accumulation.  Workgroup: 4 waves, 128 x 64
-// outputs (each wave 32 rows x two 32-column blocks).  The epilogue depends
-// on the mode (see the per-mode comments below).
-template <int MODE>
-__global__ __launch_bounds__(256) void k_gemm(GemmArgs g)
+__device__ inline void tile_gemm(TileWeights &w, const uint16_t *in, int lane, Tile &acc)
+{
+    const uint16_t *b = in + (lane & 31) * TILE_LD + 8 * (lane >> 5);
+    acc[0] = acc[1] = f32x16{};
+#pragma unroll
+    for (int k = 0; k < HID / 16; ++k) {
+        const bf16x8 a = w.w[k % TILE_AHEAD];
+        if (k + TILE_AHEAD < HID / 16) w.w[k % TILE_AHEAD] = load_frag(w.p + (k + TILE_AHEAD) * 64 * 8);
+        const bf16x8 b0 = load_frag(b + 16 * k), b1 = load_frag(b + 32 * TILE_LD + 16 * k);
+        acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b0, acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b1, acc[1], 0, 0, 0);
+    }
+}
+
+// The tile's values, rounded to BF16, into LDS: four neurons of a row at a time.
+template <class F>
+__device__ inline void tile_store(uint16_t *out, int n0, int lane, F &&value)
+{
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint2 pk = make_uint2(pack_bf16x2(value(rb, 4 * q), value(rb, 4 * q + 1)),
+                                        pack_bf16x2(value(rb, 4 * q + 2), value(rb, 4 * q + 3)));
+            *reinterpret_cast<uint2 *>(out + (32 * rb + (lane & 31)) * TILE_LD + n0 + 8 * q + 4 * (lane >> 5)) = pk;
+        }
+}
+
+// A BF16 tile from LDS to its place in a transposed batch array.
+__device__ inline void tile_transposed(const uint16_t *in, uint16_t *T, int r0)
+{
+    const int n = threadIdx.x & (HID - 1);
+#pragma unroll
+    for (int i = 0; i < TILE_ROWS / 16; ++i) {
+        const int j = (threadIdx.x >> 8) + 2 * i;
+        uint32_t v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            v[e] = (uint32_t)in[(8 * j + 2 * e) * TILE_LD + n] | ((uint32_t)in[(8 * j + 2 * e + 1) * TILE_LD + n] << 16);
+        reinterpret_cast<uint4 *>(T)[frag_unit(n, r0 / 8 + j)] = make_uint4(v[0], v[1], v[2], v[3]);
+    }
+}
+
+__device__ inline void tile_bias(Tile &z, const float *bias, int n0, int lane)
+{
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const float4 b = *reinterpret_cast<const float4 *>(bias + n0 + 8 * q + 4 * (lane >> 5));
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) {
+            z[rb][4 * q] += b.x;
+            z[rb][4 * q + 1] += b.y;
+            z[rb][4 * q + 2] += b.z;
+            z[rb][4 * q + 3] += b.w;
+        }
+    }
+}
+
+// Layers:  z1 = W1 x + b1 (FP32), z_l = a_{l-1} W_l^T + b_l, a_l = silu(z_l);
+//   head (FP32): y = w5 . a4 + b5, loss = mean (y - t)^2, dy = 2 (y - t) / B,
+//   dz4 = dy w5 * silu'(z4), and per 32 rows the partial sums of dw5 = sum dy a4 and
+//   db5 = sum dy;
+//   dz_{l-1} = (dz_l W_l) * silu'(z_{l-1}).
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_train_tile(Net net, Acts s, int m0,
+                                                                                             int Bn)
+{
+    __shared__ __attribute__((aligned(16))) uint16_t tile[2][TILE_ROWS * TILE_LD];
+    __shared__ __attribute__((aligned(16))) float a4[TILE_ROWS * TILE_LDF];
+    __shared__ float dys[TILE_ROWS], lossp[TILE_ROWS / HEAD_ROWS * 4];
+    const int m = m0 + blockIdx.y;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int r0 = blockIdx.x * TILE_ROWS, n0 = 32 * wave;
+    const float *P = net.P + (size_t)m * PSTRIDE;
+    const uint16_t *Wb = net.Wb + (size_t)m * 3 * LAYER_W, *WbT = net.WbT + (size_t)m * 3 * LAYER_W;
+    auto layer = [](const uint16_t *W, int l) { return W + (size_t)(l - 2) * LAYER_W; };
+    TileWeights w;
+    Tile z1, z2, z3, z;
+    w.start(layer(Wb, 2), n0, lane);
+    {
+        float x[2][NIN];
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) {
+            const float4 *xb =
+                reinterpret_cast<const float4 *>(s.xb + ((size_t)m * s.B + r0 + 32 * rb + (lane & 31)) * NIN);
+#pragma unroll
+            for (int k = 0; k < NIN / 4; ++k) {
+                const float4 v = xb[k];
+                x[rb][4 * k] = v.x;
+                x[rb][4 * k + 1] = v.y;
+                x[rb][4 * k + 2] = v.z;
+                x[rb][4 * k + 3] = v.w;
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int n = n0 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4;
+            const float *w1 = P + HWT_SURR_W1 + n * NIN;
+            const float b = P[HWT_SURR_B1 + n];
+            z1[0][v] = z1[1][v] = b;
+#pragma unroll
+            for (int k = 0; k < NIN; ++k) {
+                z1[0][v] = fmaf(w1[k], x[0][k], z1[0][v]);
+                z1[1][v] = fmaf(w1[k], x[1][k], z1[1][v]);
+            }
+            // no more than four neurons' weights at a time in registers
+            if (v % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    tile_store(tile[0], n0, lane, [&](int rb, int v) { return silu(z1[rb][v]); });
+    __syncthreads();
+    tile_gemm(w, tile[0], lane, z2);
+    w.start(layer(Wb, 3), n0, lane);
+    tile_transposed(tile[0], s.aT + aoff(s, m, 1), r0);
+    tile_bias(z2, P + boff(2), n0, lane);
+    tile_store(tile[1], n0, lane, [&](int rb, int v) { return silu(z2[rb][v]); });
+    __syncthreads();
+    tile_gemm(w, tile[1], lane, z3);
+    w.start(layer(Wb, 4), n0, lane);
+    tile_transposed(tile[1], s.aT + aoff(s, m, 2), r0);
+    tile_bias(z3, P + boff(3), n0, lane);
+    tile_store(tile[0], n0, lane, [&](int rb, int v) { return silu(z3[rb][v]); });
+    __syncthreads();
+    tile_gemm(w, tile[0], lane, z);
+    w.start(layer(WbT, 4), n0, lane);
+    tile_transposed(tile[0], s.aT + aoff(s, m, 3), r0);
+    tile_bias(z, P + boff(4), n0, lane);
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<float4 *>(a4 + (32 * rb + (lane & 31)) * TILE_LDF + n0 + 8 * q + 4 * (lane >> 5)) =
+                make_float4(silu(z[rb][4 * q]), silu(z[rb][4 * q + 1]), silu(z[rb][4 * q + 2]), silu(z[rb][4 * q + 3]));
+    __syncthreads();
+    {
+        // four waves per 32 rows
+        const int half = wave >> 2;
+        float w5[4], lsum = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w5[q] = P[HWT_SURR_W5 + lane + 64 * q];
+        for (int r = wave & 3; r < HEAD_ROWS; r += 4) {
+            const int row = HEAD_ROWS * half + r;
+            float p = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) p = fmaf(w5[q], a4[row * TILE_LDF + lane + 64 * q], p);
+            const float yv = wave_sum_f(p) + P[HWT_SURR_B5];
+            const float err = yv - s.tb[(size_t)m * s.B + r0 + row];
+            if (lane == 0) {
+                s.y[(size_t)m * s.B + r0 + row] = yv;
+                dys[row] = 2.0f * err / (float)Bn;
+            }
+            lsum += err * err;
+        }
+        if (lane == 0) lossp[wave] = lsum;
+    }
+    __syncthreads();
+    {
+        const int n = t & (HID - 1), half = t >> 8;
+        float dw = 0.0f, db = 0.0f;
+#pragma unroll 8
+        for (int r = 0; r < HEAD_ROWS; ++r) {
+            const float dy = dys[HEAD_ROWS * half + r];
+            dw = fmaf(dy, a4[(HEAD_ROWS * half + r) * TILE_LDF + n], dw);
+            db += dy;
+        }
+        float *hp = s.hp + ((size_t)m * (s.B / HEAD_ROWS) + 2 * blockIdx.x + half) * (HID + 1);
+        hp[n] = dw;
+        if (n == 0) {
+            const float *lp = lossp + 4 * half;
+            hp[HID] = db;
+            atomicAdd(&s.loss[m], (double)(lp[0] + lp[1] + lp[2] + lp[3]));
+        }
+    }
+    {
+        const float dy[2] = {dys[lane & 31], dys[32 + (lane & 31)]};
+        tile_store(tile[1], n0, lane, [&](int rb, int v) {
+            return dy[rb] * P[HWT_SURR_W5 + n0 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4] * dsilu(z[rb][v]);
+        });
+    }
+    __syncthreads();
+    tile_gemm(w, tile[1], lane, z);
+    w.start(layer(WbT, 3), n0, lane);
+    tile_transposed(tile[1], s.dzT + dzoff(s, m, 4), r0);
+    tile_store(tile[0], n0, lane, [&](int rb, int v) { return z[rb][v] * dsilu(z3[rb][v]); });
+    __syncthreads();
+    tile_gemm(w, tile[0], lane, z);
+    w.start(layer(WbT, 2), n0, lane);
+    tile_transposed(tile[0], s.dzT + dzoff(s, m, 3), r0);
+    tile_store(tile[1], n0, lane, [&](int rb, int v) { return z[rb][v] * dsilu(z2[rb][v]); });
+    __syncthreads();
+    tile_gemm(w, tile[1], lane, z);
+    tile_transposed(tile[1], s.dzT + dzoff(s, m, 2), r0);
+    float *dz1 = s.dz1T + (size_t)m * HID * s.B + r0 + (lane & 31);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        const size_t n = n0 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4;
+        dz1[n * s.B] = z[0][v] * dsilu(z1[0][v]);
+        dz1[n * s.B + 32] = z[1][v] * dsilu(z1[1][v]);
+    }
+}
+
+// --- weight gradients
+// dW_l[n][k] = sum_b dz_l[b][n] a_{l-1}[b][k], one of DW_SPLIT parts of the batch per
+// workgroup and 128 x 128 outputs: each wave 64 x 64, four fragments (a contiguous
+// kilobyte each) per four matrix instructions, all layers in one launch, with the
+// small gradients: 60 us for 4 x 8192 rows, where four launches took 127.
+constexpr int DW_TILE = 128;
+constexpr int DW_BLOCKS = 3 * (HID / DW_TILE) * (HID / DW_TILE) * DW_SPLIT;  // per member
+__device__ inline void weight_gradient(const Acts &s, int m, int block, int Bn)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int mz = blockIdx.z;
-    const int m = g.m0 + (MODE == G_DW ? mz / g.nsplit : mz);
-    const int split = MODE == G_DW ? mz % g.nsplit : 0;
-    const int row0 = blockIdx.x * GEMM_ROWS + wave * 32;
-    const int col0 = blockIdx.y * 64;
-    const int kbase = split * g.K;
-    const uint16_t *A = g.A + (size_t)m * g.sA + (size_t)(row0 + (lane & 31)) * g.lda + kbase + 8 * (lane >> 5);
-    const uint16_t *B0 = g.Bm + (size_t)m * g.sB + (size_t)(col0 + (lane & 31)) * g.ldb + kbase + 8 * (lane >> 5);
-    const uint16_t *B1 = B0 + (size_t)32 * g.ldb;
-    f32x16 acc0 = {}, acc1 = {};
-    for (int k = 0; k < g.K; k += 16) {
-        const bf16x8 a = load_frag(A + k);
-        const bf16x8 b0 = load_frag(B0 + k);
-        const bf16x8 b1 = load_frag(B1 + k);
-        acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b0, acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b1, acc1, 0, 0, 0);
+    const int split = block % DW_SPLIT, rest = block / DW_SPLIT;
+    const int l = 2 + rest / 4, row0 = (rest & 1) * DW_TILE + (wave & 1) * 64, col0 = (rest >> 1 & 1) * DW_TILE + (wave >> 1) * 64;
+    const int K = Bn / DW_SPLIT;  // a multiple of 16
+    const size_t k0 = (size_t)(split * K / 16) * (HID / 32) * 64 * 8;
+    const uint16_t *A = s.dzT + dzoff(s, m, l) + k0 + ((size_t)(row0 >> 5) * 64 + lane) * 8;
+    const uint16_t *B = s.aT + aoff(s, m, l - 1) + k0 + ((size_t)(col0 >> 5) * 64 + lane) * 8;
+    f32x16 acc[2][2] = {};
+#pragma unroll 4
+    for (int k = 0; k < K / 16; ++k) {
+        const size_t at = (size_t)k * (HID / 32) * 64 * 8;
+        const bf16x8 a0 = load_frag(A + at), a1 = load_frag(A + at + 64 * 8);
+        const bf16x8 b0 = load_frag(B + at), b1 = load_frag(B + at + 64 * 8);
+        acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b0, acc[0][0], 0, 0, 0);
+        acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b1, acc[0][1], 0, 0, 0);
+        acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b0, acc[1][0], 0, 0, 0);
+        acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, acc[1][1], 0, 0, 0);
     }
-    const Acts &s = g.s;
-    const int l = g.layer;
-    const float *P = g.net.P + (size_t)m * PSTRIDE;
+    float *gw = s.gw + (((size_t)m * 3 + (l - 2)) * DW_SPLIT + split) * LAYER_W;
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
-        const f32x16 &acc = cb ? acc1 : acc0;
-        const int col = col0 + cb * 32 + (lane & 31);
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int grp = 0; grp < 4; ++grp) {
-            // this lane's rows rbase .. rbase+3 of column col
-            const int rbase = row0 + 8 * grp + 4 * (lane >> 5);
-            float ov[4];
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int row = rbase + q;
-                const float v = acc[4 * grp + q];
-                if (MODE == G_FWD || MODE == G_FWD_LAST) {
-                    // z_l = a_{l-1} W_l^T + b_l; a_l = silu(z_l)
-                    const float zz = v + P[boff(l) + col];
-                    s.z[zoff(s, m, l) + (size_t)row * HID + col] = zz;
-                    ov[q] = silu(zz);
-                    if (MODE == G_FWD) s.a[aoff(s, m, l) + (size_t)row * HID + col] = to_bf16(ov[q]);
-                    else s.a4[(size_t)m * s.B * HID + (size_t)row * HID + col] = ov[q];
-                } else if (MODE == G_DX || MODE == G_DX_FIRST) {
-                    // d a_{l-1} = dz_l W_l; dz_{l-1} = d a_{l-1} * silu'(z_{l-1})
-                    ov[q] = v * dsilu(s.z[zoff(s, m, l - 1) + (size_t)row * HID + col]);
-                    if (MODE == G_DX) s.dz[dzoff(s, m, l - 1) + (size_t)row * HID + col] = to_bf16(ov[q]);
-                } else {
-                    // dW_l[n][k] partial over this split of the batch
-                    s.gw[(((size_t)m * 3 + (l - 2)) * DW_SPLIT + split) * LAYER_W + (size_t)row * HID + col] = v;
-                    ov[q] = 0.0f;
-                }
-            }
-            if (MODE == G_FWD || MODE == G_DX) {
-                uint16_t *T = (MODE == G_FWD) ? s.aT + aoff(s, m, l) : s.dzT + dzoff(s, m, l - 1);
-                const uint2 pk = make_uint2((uint32_t)to_bf16(ov[0]) | ((uint32_t)to_bf16(ov[1]) << 16),
-                                            (uint32_t)to_bf16(ov[2]) | ((uint32_t)to_bf16(ov[3]) << 16));
-                *reinterpret_cast<uint2 *>(T + (size_t)col * s.B + rbase) = pk;
-            } else if (MODE == G_DX_FIRST) {
-                *reinterpret_cast<float4 *>(s.dz1T + (size_t)m * HID * s.B + (size_t)col * s.B + rbase) =
-                    make_float4(ov[0], ov[1], ov[2], ov[3]);
-            }
-        }
-    }
+            for (int v = 0; v < 16; ++v)
+                gw[(size_t)(row0 + 32 * i + 8 * (v / 4) + 4 * (lane >> 5) + v % 4) * HID + col0 + 32 * j + (lane & 31)] =
+                    acc[i][j][v];
 }
 
-// Output layer (FP32), loss and the start of the backward pass:
-//   y = w5 . a4 + b5,  loss = mean (y - t)^2,  dy = 2 (y - t) / B,
-//   dz4 = dy w5 * silu'(z4) (BF16, both layouts),
-//   per-block partial sums of dw5 = sum dy a4 and db5 = sum dy.
-__global__ __launch_bounds__(HID) void k_head(Net net, Acts s, int m0, int Bn)
-{
-    const int m = m0 + blockIdx.y;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int r0 = blockIdx.x * HEAD_ROWS;
-    const float *P = net.P + (size_t)m * PSTRIDE;
-    __shared__ float dys[HEAD_ROWS];
-    __shared__ float lossp[4];
-    const float *a4 = s.a4 + (size_t)m * s.B * HID;
-    float lsum = 0.0f;
-    for (int r = wave; r < HEAD_ROWS; r += 4) {
-        const size_t row = r0 + r;
-        float p = 0.0f;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) p = fmaf(P[HWT_SURR_W5 + lane + 64 * q], a4[row * HID + lane + 64 * q], p);
-        const float yv = wave_sum_f(p) + P[HWT_SURR_B5];
-        const float err = yv - s.tb[(size_t)m * s.B + row];
-        if (lane == 0) {
-            s.y[(size_t)m * s.B + row] = yv;
-            dys[r] = 2.0f * err / (float)Bn;
-        }
-        lsum += err * err;
-    }
-    if (lane == 0) lossp[wave] = lsum;
-    __syncthreads();
-    const int n = t;
-    const float w5 = P[HWT_SURR_W5 + n];
-    const float *z4 = s.z + zoff(s, m, 4);
-    uint16_t *dz = s.dz + dzoff(s, m, 4);
-    float dw = 0.0f, db = 0.0f;
-    uint32_t packed[HEAD_ROWS / 2];
-#pragma unroll
-    for (int r = 0; r < HEAD_ROWS; ++r) {
-        const size_t row = r0 + r;
-        const float dy = dys[r];
-        dw = fmaf(dy, a4[row * HID + n], dw);
-        db += dy;
-        const uint16_t h = to_bf16(dy * w5 * dsilu(z4[row * HID + n]));
-        dz[row * HID + n] = h;
-        if (r & 1) packed[r / 2] |= (uint32_t)h << 16;
-        else packed[r / 2] = h;
-    }
-    uint4 *dst = reinterpret_cast<uint4 *>(s.dzT + dzoff(s, m, 4) + (size_t)n * s.B + r0);
-#pragma unroll
-    for (int q = 0; q < HEAD_ROWS / 8; ++q)
-        dst[q] = make_uint4(packed[4 * q], packed[4 * q + 1], packed[4 * q + 2], packed[4 * q + 3]);
-    float *hp = s.hp + ((size_t)m * (s.B / HEAD_ROWS) + blockIdx.x) * (HID + 1);
-    hp[n] = dw;
-    if (n == 0) {
-        hp[HID] = db;
-        atomicAdd(&s.loss[m], (double)(lossp[0] + lossp[1] + lossp[2] + lossp[3]));
-    }
-}
-
-// Gradients of the input layer and of the biases, one workgroup per neuron:
+// Gradients of the input layer and of the biases, SMALL_N neurons per workgroup:
 //   dW1[n][i] = sum_b dz1[b][n] x[b][i], db1[n] = sum_b dz1[b][n],
 //   db_l[n] = sum_b dz_l[b][n] (l = 2..4).
-__global__ __launch_bounds__(256) void k_small_grads(Acts s, int m0, int Bn)
+// A thread sums the rows of one residue of 256; the neurons share its x row and the
+// 128-byte lines in which the transposed arrays hold eight neurons' rows.
+constexpr int SMALL_N = 4, SMALL_BLOCKS = HID / SMALL_N;
+__device__ inline void small_gradients(const Acts &s, int m, int block, int Bn)
 {
-    const int m = m0 + blockIdx.y;
-    const int n = blockIdx.x;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    float acc[12];
-#pragma unroll
-    for (int k = 0; k < 12; ++k) acc[k] = 0.0f;
-    const float *dz1 = s.dz1T + (size_t)m * HID * s.B + (size_t)n * s.B;
-    const float *xb = s.xb + (size_t)m * s.B * NIN;
+    const int n0 = block * SMALL_N;
+    float acc[SMALL_N][12] = {};
+    const float *dz1 = s.dz1T + (size_t)m * HID * s.B + (size_t)n0 * s.B;
+    const float4 *xb = reinterpret_cast<const float4 *>(s.xb + (size_t)m * s.B * NIN);
+#pragma unroll 2
     for (int r = t; r < Bn; r += 256) {
-        const float d = dz1[r];
+        const float4 x0 = xb[2 * (size_t)r], x1 = xb[2 * (size_t)r + 1];
+        const float x[NIN] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
 #pragma unroll
-        for (int k = 0; k < NIN; ++k) acc[k] = fmaf(d, xb[(size_t)r * NIN + k], acc[k]);
-        acc[8] += d;
+        for (int j = 0; j < SMALL_N; ++j) {
+            const float d = dz1[(size_t)j * s.B + r];
 #pragma unroll
-        for (int l = 2; l <= 4; ++l) acc[7 + l] += from_bf16(s.dzT[dzoff(s, m, l) + (size_t)n * s.B + r]);
+            for (int k = 0; k < NIN; ++k) acc[j][k] = fmaf(d, x[k], acc[j][k]);
+            acc[j][8] += d;
+#pragma unroll
+            for (int l = 2; l <= 4; ++l)
+                acc[j][7 + l] += from_bf16(s.dzT[dzoff(s, m, l) + frag_unit(n0 + j, r >> 3) * 8 + (r & 7)]);
+        }
     }
-    __shared__ float red[4][12];
+    __shared__ float red[4][SMALL_N * 12];
 #pragma unroll
-    for (int k = 0; k < 12; ++k) {
-        const float v = wave_sum_f(acc[k]);
-        if (lane == 0) red[wave][k] = v;
-    }
+    for (int j = 0; j < SMALL_N; ++j)
+#pragma unroll
+        for (int k = 0; k < 12; ++k) {
+            const float v = wave_sum_f(acc[j][k]);
+            if (lane == 0) red[wave][12 * j + k] = v;
+        }
     __syncthreads();
-    if (t < 12) {
+    if (t < SMALL_N * 12) {
         const float v = red[0][t] + red[1][t] + red[2][t] + red[3][t];
+        const int n = n0 + t / 12, k = t % 12;
         float *gs = s.gs + (size_t)m * PSTRIDE;
-        if (t < NIN) gs[HWT_SURR_W1 + n * NIN + t] = v;
-        else if (t == 8) gs[HWT_SURR_B1 + n] = v;
-        else gs[boff(t - 7) + n] = v;
+        if (k < NIN) gs[HWT_SURR_W1 + n * NIN + k] = v;
+        else if (k == 8) gs[HWT_SURR_B1 + n] = v;
+        else gs[boff(k - 7) + n] = v;
     }
 }
 
-// Dense gradient of every parameter from the partial sums.
-__global__ void k_grad_reduce(Acts s, int m0, int nhead)
+// Both in one launch: the small gradients' loads fill the time in which the matrix
+// instructions' blocks finish.
+__global__ __launch_bounds__(256) void k_gradients(Acts s, int m0, int Bn)
 {
     const int m = m0 + blockIdx.y;
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= NPAR) return;
-    float g;
+    if (blockIdx.x < SMALL_BLOCKS) small_gradients(s, m, blockIdx.x, Bn);
+    else weight_gradient(s, m, blockIdx.x - SMALL_BLOCKS, Bn);
+}
+
+// Dense gradient of parameter p from the partial sums, each in order.
+__device__ inline float gradient_of(const Acts &s, int m, int p, int nhead)
+{
+    float g = 0.0f;
     if (p >= HWT_SURR_W2 && p < HWT_SURR_B4 && !(p >= HWT_SURR_B2 && p < HWT_SURR_W3) &&
         !(p >= HWT_SURR_B3 && p < HWT_SURR_W4)) {
         const int l = p < HWT_SURR_B2 ? 2 : (p < HWT_SURR_B3 ? 3 : 4);
-        const int idx = p - woff(l);
-        const float *src = s.gw + ((size_t)m * 3 + (l - 2)) * DW_SPLIT * LAYER_W + idx;
-        g = 0.0f;
+        const float *src = s.gw + ((size_t)m * 3 + (l - 2)) * DW_SPLIT * LAYER_W + (p - woff(l));
 #pragma unroll
         for (int q = 0; q < DW_SPLIT; ++q) g += src[(size_t)q * LAYER_W];
-    } else if (p >= HWT_SURR_W5) {
-        const int idx = p - HWT_SURR_W5;  // 0..255 = w5, 256 = b5
-        const float *src = s.hp + (size_t)m * (s.B / HEAD_ROWS) * (HID + 1) + idx;
-        g = 0.0f;
-        for (int q = 0; q < nhead; ++q) g += src[(size_t)q * (HID + 1)];
-    } else {
-        g = s.gs[(size_t)m * PSTRIDE + p];
+        return g;
     }
-    s.g[(size_t)m * PSTRIDE + p] = g;
+    if (p < HWT_SURR_W5) return s.gs[(size_t)m * PSTRIDE + p];
+    // w5 and b5: a chain of adds over the tiles, its loads 32 at a time (one at a time
+    // they were 100 us of a step)
+    const float *src = s.hp + (size_t)m * (s.B / HEAD_ROWS) * (HID + 1) + (p - HWT_SURR_W5);
+    constexpr int AHEAD = 32;
+    for (int q = 0; q < nhead; q += AHEAD) {
+        float v[AHEAD];
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k) v[k] = src[(size_t)min(q + k, nhead - 1) * (HID + 1)];
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k)
+            if (q + k < nhead) g += v[k];
+    }
+    return g;
 }
 
-// Adam on the FP32 masters; refreshes the BF16 copies (and transposes) of
-// the 256x256 layers.  c1 = 1/(1-beta1^t), c2 = 1/(1-beta2^t).
-__global__ void k_adam(Net net, const float *__restrict__ grad, float *__restrict__ m1, float *__restrict__ m2,
-                       float lr, float beta1, float beta2, float eps, float c1, float c2)
+// Adam on parameter p of the FP32 masters; refreshes the BF16 copies (and
+// transposes) of the 256x256 layers.
+struct AdamArgs {
+    float *m1, *m2;
+    float lr, beta1, beta2, eps;
+    float c1, c2;  // 1/(1-beta1^t), 1/(1-beta2^t)
+};
+__device__ inline void adam_step(const Net &net, const AdamArgs &a, int m, int p, float g)
 {
-    const int m = blockIdx.y;
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= NPAR) return;
     const size_t i = (size_t)m * PSTRIDE + p;
-    const float g = grad[i];
-    const float mm = beta1 * m1[i] + (1.0f - beta1) * g;
-    const float vv = beta2 * m2[i] + (1.0f - beta2) * g * g;
-    m1[i] = mm;
-    m2[i] = vv;
-    const float w = net.P[i] - lr * (mm * c1) / (sqrtf(vv * c2) + eps);
+    const float mm = a.beta1 * a.m1[i] + (1.0f - a.beta1) * g;
+    const float vv = a.beta2 * a.m2[i] + (1.0f - a.beta2) * g * g;
+    a.m1[i] = mm;
+    a.m2[i] = vv;
+    const float w = net.P[i] - a.lr * (mm * a.c1) / (sqrtf(vv * a.c2) + a.eps);
     net.P[i] = w;
     int l = 0;
     if (p >= HWT_SURR_W2 && p < HWT_SURR_B2) l = 2;
@@ -509,9 +640,36 @@ __global__ void k_adam(Net net, const float *__restrict__ grad, float *__restric
         const int idx = p - woff(l), nn = idx / HID, kk = idx % HID;
         const size_t base = ((size_t)m * 3 + (l - 2)) * LAYER_W;
         const uint16_t h = to_bf16(w);
-        net.Wb[base + idx] = h;
-        net.WbT[base + (size_t)kk * HID + nn] = h;
+        net.Wb[base + weight_at(nn, kk)] = h;
+        net.WbT[base + weight_at(kk, nn)] = h;
     }
+}
+
+constexpr int PAR_BLOCKS = (NPAR + 255) / 256;
+// The gradient of one evaluation, for callers who ask for it.
+__global__ void k_grad_reduce(Acts s, int m0, int nhead)
+{
+    const int m = m0 + blockIdx.y;
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < NPAR) s.g[(size_t)m * PSTRIDE + p] = gradient_of(s, m, p, nhead);
+}
+
+// Adam on a given gradient.
+__global__ void k_adam(Net net, AdamArgs a, const float *__restrict__ grad)
+{
+    const int m = blockIdx.y;
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < NPAR) adam_step(net, a, m, p, grad[(size_t)m * PSTRIDE + p]);
+}
+
+// A training step's: the gradient goes from its partial sums straight into Adam (17 us
+// for four members; 116 us as two kernels, the head's chains one load at a time).  The
+// head's chains are the longest, so their blocks start first.
+__global__ __launch_bounds__(256) void k_update(Net net, AdamArgs a, Acts s, int nhead)
+{
+    const int m = blockIdx.y;
+    const int p = (PAR_BLOCKS - 1 - blockIdx.x) * 256 + threadIdx.x;
+    if (p < NPAR) adam_step(net, a, m, p, gradient_of(s, m, p, nhead));
 }
 
 // BF16 copies from the masters (after initialisation or a load).
@@ -523,8 +681,8 @@ __global__ void k_refresh_bf16(Net net, int members)
     const int l = 2 + idx / LAYER_W, e = idx % LAYER_W, nn = e / HID, kk = e % HID;
     const uint16_t h = to_bf16(net.P[(size_t)m * PSTRIDE + woff(l) + e]);
     const size_t base = ((size_t)m * 3 + (l - 2)) * LAYER_W;
-    net.Wb[base + e] = h;
-    net.WbT[base + (size_t)kk * HID + nn] = h;
+    net.Wb[base + weight_at(nn, kk)] = h;
+    net.WbT[base + weight_at(kk, nn)] = h;
 }
 
 // --------------------------------------------------------------- inference
@@ -558,16 +716,6 @@ struct InferArgs {
     const int32_t *rows;      // option of each row (null: row i is option i)
     const int32_t *row_count; // number of listed rows (with `rows`)
 };
-
-// Two floats to a packed BF16 pair (a in the low half), round to nearest
-// even, as one v_cvt_pk_bf16_f32 (the value-by-value form costs a convert,
-// a shift and an or per pair).
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-__device__ inline uint32_t pack_bf16x2(float a, float b)
-{
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
-}
 
 // Accumulators of a wave's 2 x 4 blocks D[neuron][row] seeded with the
 // layer's bias: lane l's value v belongs to neuron 32 mb + 8 (v/4) + 4 (l/32)
@@ -687,14 +835,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         __syncthreads();
         for (int l = 2; l <= 4; ++l) {
             const uint16_t *W = g.net.Wb + ((size_t)m * 3 + (l - 2)) * LAYER_W;
-            const uint16_t *wa0 = W + (size_t)(n0 + mrow) * HID + khalf;
-            const uint16_t *wa1 = wa0 + (size_t)32 * HID;
+            const uint16_t *wa0 = W + ((size_t)(n0 >> 5) * (HID / 16) * 64 + lane) * 8;
+            const uint16_t *wa1 = wa0 + (HID / 16) * 64 * 8;
             const uint16_t *ab = act + mrow * ACT_LD + khalf;
             f32x16 acc[2][4];
             bias_init(acc, P + boff(l), n0, lane);
 #pragma unroll 2
             for (int k = 0; k < HID; k += 16) {
-                const bf16x8 a0 = load_frag(wa0 + k), a1 = load_frag(wa1 + k);
+                const bf16x8 a0 = load_frag(wa0 + 32 * k), a1 = load_frag(wa1 + 32 * k);
 #pragma unroll
                 for (int nb = 0; nb < 4; ++nb) {
                     const bf16x8 b =
@@ -918,81 +1066,12 @@ struct hwt_surrogate {
 
 namespace {
 
-int gemm_launch(hwt_surrogate *s, int mode, int l, int m0, int mc, int Bn)
-{
-    GemmArgs g{};
-    g.net = s->net;
-    g.s = s->acts;
-    g.m0 = m0;
-    g.layer = l;
-    g.nsplit = 1;
-    const Acts &a = s->acts;
-    const size_t actm = (size_t)3 * a.B * HID;  // member stride of a/aT/dz/dzT
-    dim3 grid;
-    switch (mode) {
-    case G_FWD:
-    case G_FWD_LAST:
-        // A = a_{l-1} [B][256], B = W_l [256][256]
-        g.A = a.a + aoff(a, 0, l - 1);
-        g.sA = actm;
-        g.lda = HID;
-        g.Bm = s->net.Wb + (size_t)(l - 2) * LAYER_W;
-        g.sB = (size_t)3 * LAYER_W;
-        g.ldb = HID;
-        g.K = HID;
-        grid = dim3(Bn / GEMM_ROWS, HID / 64, mc);
-        break;
-    case G_DX:
-    case G_DX_FIRST:
-        // A = dz_l [B][256], B = W_l^T [256][256]
-        g.A = a.dz + dzoff(a, 0, l);
-        g.sA = actm;
-        g.lda = HID;
-        g.Bm = s->net.WbT + (size_t)(l - 2) * LAYER_W;
-        g.sB = (size_t)3 * LAYER_W;
-        g.ldb = HID;
-        g.K = HID;
-        grid = dim3(Bn / GEMM_ROWS, HID / 64, mc);
-        break;
-    default:
-        // A = dz_l^T [256][B], B = a_{l-1}^T [256][B], K = B split DW_SPLIT ways
-        g.A = a.dzT + dzoff(a, 0, l);
-        g.sA = actm;
-        g.lda = a.B;
-        g.Bm = a.aT + aoff(a, 0, l - 1);
-        g.sB = actm;
-        g.ldb = a.B;
-        g.K = Bn / DW_SPLIT;
-        g.nsplit = DW_SPLIT;
-        grid = dim3(HID / GEMM_ROWS, HID / 64, mc * DW_SPLIT);
-        break;
-    }
-    switch (mode) {
-    case G_FWD: k_gemm<G_FWD><<<grid, 256, 0, s->stream>>>(g); break;
-    case G_FWD_LAST: k_gemm<G_FWD_LAST><<<grid, 256, 0, s->stream>>>(g); break;
-    case G_DX: k_gemm<G_DX><<<grid, 256, 0, s->stream>>>(g); break;
-    case G_DX_FIRST: k_gemm<G_DX_FIRST><<<grid, 256, 0, s->stream>>>(g); break;
-    default: k_gemm<G_DW><<<grid, 256, 0, s->stream>>>(g); break;
-    }
-    return HWT_OK;
-}
-
 // Forward + backward of members [m0, m0+mc) on the gathered rows; leaves the
-// dense gradient in acts.g.
+// gradient's partial sums in acts.
 int forward_backward(hwt_surrogate *s, int m0, int mc, int Bn)
 {
-    hipStream_t st = s->stream;
-    k_layer1<<<dim3(Bn / HEAD_ROWS, mc), HID, 0, st>>>(s->net, s->acts, m0);
-    gemm_launch(s, G_FWD, 2, m0, mc, Bn);
-    gemm_launch(s, G_FWD, 3, m0, mc, Bn);
-    gemm_launch(s, G_FWD_LAST, 4, m0, mc, Bn);
-    k_head<<<dim3(Bn / HEAD_ROWS, mc), HID, 0, st>>>(s->net, s->acts, m0, Bn);
-    gemm_launch(s, G_DX, 4, m0, mc, Bn);
-    gemm_launch(s, G_DX, 3, m0, mc, Bn);
-    gemm_launch(s, G_DX_FIRST, 2, m0, mc, Bn);
-    for (int l = 2; l <= 4; ++l) gemm_launch(s, G_DW, l, m0, mc, Bn);
-    k_small_grads<<<dim3(HID, mc), 256, 0, st>>>(s->acts, m0, Bn);
-    k_grad_reduce<<<dim3((NPAR + 255) / 256, mc), 256, 0, st>>>(s->acts, m0, Bn / HEAD_ROWS);
+    k_train_tile<<<dim3(Bn / TILE_ROWS, mc), 512, 0, s->stream>>>(s->net, s->acts, m0, Bn);
+    k_gradients<<<dim3(SMALL_BLOCKS + DW_BLOCKS, mc), 256, 0, s->stream>>>(s->acts, m0, Bn);
     SURR_HIP(hipGetLastError());
     return HWT_OK;
 }
@@ -1006,14 +1085,18 @@ float lr_at(const hwt_surrogate *s, int64_t step, int64_t total)
     return (float)(c.lr_min + 0.5 * (c.lr_max - c.lr_min) * (1.0 + std::cos(M_PI * f)));
 }
 
-int adam_launch(hwt_surrogate *s, float lr)
+// Adam on the gradient in acts.g, or on the partial sums a step over nhead head
+// blocks has left in acts.
+int adam_launch(hwt_surrogate *s, float lr, int nhead)
 {
     const hwt_surr_config &c = s->cfg;
     const double t = (double)(s->step + 1);
-    const float c1 = (float)(1.0 / (1.0 - std::pow((double)c.beta1, t)));
-    const float c2 = (float)(1.0 / (1.0 - std::pow((double)c.beta2, t)));
-    k_adam<<<dim3((NPAR + 255) / 256, s->members), 256, 0, s->stream>>>(s->net, s->acts.g, s->m1, s->m2, lr, c.beta1,
-                                                                         c.beta2, c.eps, c1, c2);
+    const AdamArgs a{s->m1, s->m2, lr, c.beta1, c.beta2, c.eps,
+                     (float)(1.0 / (1.0 - std::pow((double)c.beta1, t))),
+                     (float)(1.0 / (1.0 - std::pow((double)c.beta2, t)))};
+    const dim3 grid(PAR_BLOCKS, s->members);
+    if (nhead) k_update<<<grid, 256, 0, s->stream>>>(s->net, a, s->acts, nhead);
+    else k_adam<<<grid, 256, 0, s->stream>>>(s->net, a, s->acts.g);
     SURR_HIP(hipGetLastError());
     ++s->step;
     return HWT_OK;
@@ -1099,7 +1182,7 @@ int hwt_surr_create(hwt_surrogate **out, int32_t train_capacity, int32_t infer_c
     if (cfg) s->cfg = *cfg;
     else hwt_surr_config_init(&s->cfg);
     const hwt_surr_config &c = s->cfg;
-    if (c.members < 1 || c.members > HWT_SURR_MAX_MEMBERS || c.batch < GEMM_ROWS || c.batch % GEMM_ROWS != 0 ||
+    if (c.members < 1 || c.members > HWT_SURR_MAX_MEMBERS || c.batch < BATCH_STEP || c.batch % BATCH_STEP != 0 ||
         c.batch > (1 << 20) || !(c.lr_max > 0.0f) || !(c.beta1 >= 0.0f && c.beta1 < 1.0f) ||
         !(c.beta2 >= 0.0f && c.beta2 < 1.0f) || !(c.eps > 0.0f) || !(c.spread_threshold >= 0.0f)) {
         delete s;
@@ -1135,9 +1218,8 @@ int hwt_surr_create(hwt_surrogate **out, int32_t train_capacity, int32_t infer_c
     };
     const size_t oP = carve(M * PSTRIDE * 4), oWb = carve(M * 3 * LAYER_W * 2), oWbT = carve(M * 3 * LAYER_W * 2);
     const size_t om1 = carve(M * PSTRIDE * 4), om2 = carve(M * PSTRIDE * 4);
-    const size_t oxb = carve(M * B * NIN * 4), otb = carve(M * B * 4), oz = carve(M * 4 * B * HID * 4);
-    const size_t oa = carve(M * 3 * B * HID * 2), oaT = carve(M * 3 * B * HID * 2), oa4 = carve(M * B * HID * 4);
-    const size_t odz = carve(M * 3 * B * HID * 2), odzT = carve(M * 3 * B * HID * 2), odz1 = carve(M * HID * B * 4);
+    const size_t oxb = carve(M * B * NIN * 4), otb = carve(M * B * 4);
+    const size_t oaT = carve(M * 3 * B * HID * 2), odzT = carve(M * 3 * B * HID * 2), odz1 = carve(M * HID * B * 4);
     const size_t oy = carve(M * B * 4), ogw = carve(M * 3 * DW_SPLIT * LAYER_W * 4), ogs = carve(M * PSTRIDE * 4);
     const size_t ohp = carve(M * (B / HEAD_ROWS) * (HID + 1) * 4), oloss = carve(M * 8), og = carve(M * PSTRIDE * 4);
     const size_t oX = carve(T * NIN * 4), otg = carve(T * 4), operm = carve(M * T * 4), orows = carve(B * 4);
@@ -1146,7 +1228,13 @@ int hwt_surr_create(hwt_surrogate **out, int32_t train_capacity, int32_t infer_c
     const size_t ocs = carve(I * 8), ocm = carve(I * 8), ocl = carve(I * 8), oca = carve(I * 8), ocg = carve(I * 8);
     const size_t ocu = carve(I * 2), ocst = carve(I * 2), octy = carve(I);
     s->bytes = off;
-    if (hipMalloc(&s->mem, s->bytes) != hipSuccess) return bail(HWT_ENOMEM, "hipMalloc surrogate workspace failed");
+    hipError_t em = hipMalloc(&s->mem, s->bytes);
+    if (em != hipSuccess) {  // again, with the idle one-shot workspaces given back
+        (void)hipGetLastError();
+        hwt_trim();
+        em = hipMalloc(&s->mem, s->bytes);
+    }
+    if (em != hipSuccess) return bail(HWT_ENOMEM, "hipMalloc surrogate workspace failed");
     char *b = (char *)s->mem;
     s->net.P = (float *)(b + oP);
     s->net.Wb = (uint16_t *)(b + oWb);
@@ -1157,11 +1245,7 @@ int hwt_surr_create(hwt_surrogate **out, int32_t train_capacity, int32_t infer_c
     a.B = (int)B;
     a.xb = (float *)(b + oxb);
     a.tb = (float *)(b + otb);
-    a.z = (float *)(b + oz);
-    a.a = (uint16_t *)(b + oa);
     a.aT = (uint16_t *)(b + oaT);
-    a.a4 = (float *)(b + oa4);
-    a.dz = (uint16_t *)(b + odz);
     a.dzT = (uint16_t *)(b + odzT);
     a.dz1T = (float *)(b + odz1);
     a.y = (float *)(b + oy);
@@ -1241,7 +1325,7 @@ int hwt_surr_train(hwt_surrogate *s, int32_t epochs, int32_t total_epochs, hwt_s
                 s->X, s->target, s->perm, s->ntrain, (int64_t)it * s->B, s->B, s->B, s->acts.xb, s->acts.tb, 0);
             const int rc = forward_backward(s, 0, s->members, s->B);
             if (rc) return rc;
-            const int arc = adam_launch(s, lr_at(s, s->step, total));
+            const int arc = adam_launch(s, lr_at(s, s->step, total), s->B / HEAD_ROWS);
             if (arc) return arc;
         }
         ++s->epochs_done;
@@ -1264,7 +1348,7 @@ int hwt_surr_train(hwt_surrogate *s, int32_t epochs, int32_t total_epochs, hwt_s
 int hwt_surr_eval_rows(hwt_surrogate *s, int32_t member, const int32_t *host_rows, int32_t n, float *host_out,
                        float *host_loss, float *host_grad)
 {
-    if (!s || member < 0 || member >= s->members || !host_rows || n < GEMM_ROWS || n % GEMM_ROWS != 0 || n > s->B)
+    if (!s || member < 0 || member >= s->members || !host_rows || n < BATCH_STEP || n % BATCH_STEP != 0 || n > s->B)
         return fail(HWT_EINVAL, "hwt_surr_eval_rows: bad arguments");
     for (int i = 0; i < n; ++i)
         if (host_rows[i] < 0 || host_rows[i] >= s->ntrain) return fail(HWT_EINVAL, "hwt_surr_eval_rows: row out of range");
@@ -1277,6 +1361,10 @@ int hwt_surr_eval_rows(hwt_surrogate *s, int32_t member, const int32_t *host_row
     k_zero_f64<<<1, 64, 0, s->stream>>>(s->acts.loss, s->members);
     const int rc = forward_backward(s, member, 1, n);
     if (rc) return rc;
+    if (host_grad) {
+        k_grad_reduce<<<dim3(PAR_BLOCKS, 1), 256, 0, s->stream>>>(s->acts, member, n / HEAD_ROWS);
+        SURR_HIP(hipGetLastError());
+    }
     SURR_HIP(hipMemcpyAsync(s->h_loss, s->acts.loss, s->members * sizeof(double), hipMemcpyDeviceToHost, s->stream));
     if (host_out)
         SURR_HIP(hipMemcpyAsync(host_out, s->acts.y + (size_t)member * s->B, (size_t)n * 4, hipMemcpyDeviceToHost,
@@ -1312,7 +1400,7 @@ int hwt_surr_adam_step(hwt_surrogate *s, const float *host_grad, float lr)
     for (int m = 0; m < s->members; ++m)
         SURR_HIP(hipMemcpyAsync(s->acts.g + (size_t)m * PSTRIDE, host_grad + (size_t)m * NPAR, (size_t)NPAR * 4,
                                 hipMemcpyHostToDevice, s->stream));
-    const int rc = adam_launch(s, lr);
+    const int rc = adam_launch(s, lr, 0);
     if (rc) return rc;
     SURR_HIP(hipStreamSynchronize(s->stream));
     return HWT_OK;
