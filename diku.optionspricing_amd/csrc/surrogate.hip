@@ -46,6 +46,8 @@ constexpr int NPAR = HWT_SURR_NPARAMS;
 constexpr int PSTRIDE = 200192;          // per-member stride of parameter-shaped vectors
 constexpr int LAYER_W = HID * HID;        // elements of one 256x256 weight matrix
 constexpr int BATCH_STEP = 128;           // the batch is a multiple (DW_SPLIT parts of whole 16-row blocks)
+constexpr int SMALL_PARTS = 4;            // partial sums of the small gradients (W1 and the biases)
+constexpr int SMALL_N = HID * (NIN + 4);  // ... their parameters
 constexpr int DW_SPLIT = 8;               // split of the batch in the weight-gradient GEMMs
 constexpr int HEAD_ROWS = 32;             // rows per partial sum of the output layer's gradients
 constexpr int INF_ROWS = 128;             // options per inference workgroup
@@ -225,10 +227,10 @@ struct Acts {
     float *xb, *tb;        // [m][B][8], [m][B]
     uint16_t *aT;          // [m][3][256][B]  a1..a3 (bf16), in fragment order (frag_unit)
     uint16_t *dzT;         // [m][3][256][B]  dz2..dz4 (bf16), likewise
-    float *dz1T;           // [m][256][B]
+    float *dz1;            // [m][B][256]
     float *y;              // [m][B] network outputs
     float *gw;             // [m][3][DW_SPLIT][256*256] weight-gradient partials (layers 2..4)
-    float *gs;             // [m][PSTRIDE] small gradients (W1, b1..b4), dense
+    float *gs;             // [m][SMALL_PARTS][SMALL_N] partial sums of W1, b1, b2, b3, b4
     float *hp;             // [m][B/HEAD_ROWS][257] head partials (dw5, db5)
     double *loss;          // [m] running sum of squared errors
     float *g;              // [m][PSTRIDE] dense gradient
@@ -273,8 +275,10 @@ __device__ inline uint32_t pack_bf16x2(float a, float b)
 // moves per step of 4 x 8192 rows (z, a, dz and a4 out and back, two layouts) only
 // what the weight gradients need leaves the chip: a1..a3 and dz2..dz4 (BF16) and dz1,
 // 134 MB.  Registers allow one workgroup per CU; a layer's first weights are
-// requested before the barrier that its input waits for.  4 x 8192 rows: 115 us,
-// where eight kernels took 344.
+// requested before the barrier that its input waits for.  4 x 8192 rows: 62 us,
+// where eight kernels took 344.  (115 us while the compiler kept sigmoids and
+// addresses from the forward pass and spilled them, z1 was kept too, and each phase
+// loaded its own biases.)
 constexpr int TILE_ROWS = 64;
 constexpr int TILE_LD = HID + 8;   // LDS row pitch (bf16): rows start 16 bytes on in the banks
 constexpr int TILE_LDF = HID + 4;  // ... of the FP32 tile
@@ -301,10 +305,12 @@ __device__ inline void tile_gemm(TileWeights &w, const uint16_t *in, int lane, T
 #pragma unroll
     for (int k = 0; k < HID / 16; ++k) {
         const bf16x8 a = w.w[k % TILE_AHEAD];
-        if (k + TILE_AHEAD < HID / 16) w.w[k % TILE_AHEAD] = load_frag(w.p + (k + TILE_AHEAD) * 64 * 8);
         const bf16x8 b0 = load_frag(b + 16 * k), b1 = load_frag(b + 32 * TILE_LD + 16 * k);
         acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b0, acc[0], 0, 0, 0);
         acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b1, acc[1], 0, 0, 0);
+        if (k + TILE_AHEAD < HID / 16) w.w[k % TILE_AHEAD] = load_frag(w.p + (k + TILE_AHEAD) * 64 * 8);
+        // reads no further ahead than that: the scheduler would fetch the whole tile
+        if (k % 2 == 1) __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -352,6 +358,11 @@ __device__ inline void tile_bias(Tile &z, const float *bias, int n0, int lane)
     }
 }
 
+// What the compiler would keep beside z from the forward pass for the backward one
+// (32 sigmoids a layer, the layer-1 addresses) spills; behind this it computes them
+// again.
+__device__ inline void forget(f32x16 &v) { asm volatile("" : "+v"(v)); }
+
 // Layers:  z1 = W1 x + b1 (FP32), z_l = a_{l-1} W_l^T + b_l, a_l = silu(z_l);
 //   head (FP32): y = w5 . a4 + b5, loss = mean (y - t)^2, dy = 2 (y - t) / B,
 //   dz4 = dy w5 * silu'(z4), and per 32 rows the partial sums of dw5 = sum dy a4 and
@@ -363,6 +374,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __shared__ __attribute__((aligned(16))) uint16_t tile[2][TILE_ROWS * TILE_LD];
     __shared__ __attribute__((aligned(16))) float a4[TILE_ROWS * TILE_LDF];
     __shared__ float dys[TILE_ROWS], lossp[TILE_ROWS / HEAD_ROWS * 4];
+    // the member's vectors and the tile's inputs, requested together once
+    __shared__ __attribute__((aligned(16))) float w1[HID * NIN], bias[4][HID], w5[HID];
+    __shared__ __attribute__((aligned(16))) float xs[TILE_ROWS * NIN];
+    __shared__ float target[TILE_ROWS];
     const int m = m0 + blockIdx.y;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int r0 = blockIdx.x * TILE_ROWS, n0 = 32 * wave;
@@ -370,76 +385,93 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const uint16_t *Wb = net.Wb + (size_t)m * 3 * LAYER_W, *WbT = net.WbT + (size_t)m * 3 * LAYER_W;
     auto layer = [](const uint16_t *W, int l) { return W + (size_t)(l - 2) * LAYER_W; };
     TileWeights w;
-    Tile z1, z2, z3, z;
-    w.start(layer(Wb, 2), n0, lane);
+    Tile z2, z3, z;
+    static_assert(TILE_ROWS * NIN == 512 && HID * NIN == 4 * 512 && HID == 256, "one load each");
     {
+        const float4 v = reinterpret_cast<const float4 *>(P + HWT_SURR_W1)[t];
+        const float x = s.xb[((size_t)m * s.B + r0) * NIN + t];
+        const float y = t < TILE_ROWS ? s.tb[(size_t)m * s.B + r0 + t] : 0.0f;
+        const float ba = P[(t < HID ? HWT_SURR_B1 : boff(2) - HID) + t], bb = P[(t < HID ? boff(3) : boff(4) - HID) + t];
+        const float v5 = t < HID ? P[HWT_SURR_W5 + t] : 0.0f;
+        w.start(layer(Wb, 2), n0, lane);
+        reinterpret_cast<float4 *>(w1)[t] = v;
+        xs[t] = x;
+        bias[t >> 8][t & (HID - 1)] = ba;
+        bias[2 + (t >> 8)][t & (HID - 1)] = bb;
+        if (t < HID) w5[t] = v5;
+        if (t < TILE_ROWS) target[t] = y;
+    }
+    __syncthreads();
+    auto layer1 = [&](Tile &z, int lane) {
         float x[2][NIN];
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb) {
-            const float4 *xb =
-                reinterpret_cast<const float4 *>(s.xb + ((size_t)m * s.B + r0 + 32 * rb + (lane & 31)) * NIN);
+        for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
-            for (int k = 0; k < NIN / 4; ++k) {
-                const float4 v = xb[k];
-                x[rb][4 * k] = v.x;
-                x[rb][4 * k + 1] = v.y;
-                x[rb][4 * k + 2] = v.z;
-                x[rb][4 * k + 3] = v.w;
-            }
-        }
+            for (int k = 0; k < NIN; ++k) x[rb][k] = xs[(32 * rb + (lane & 31)) * NIN + k];
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const int n = n0 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4;
-            const float *w1 = P + HWT_SURR_W1 + n * NIN;
-            const float b = P[HWT_SURR_B1 + n];
-            z1[0][v] = z1[1][v] = b;
+            z[0][v] = z[1][v] = bias[0][n];
 #pragma unroll
             for (int k = 0; k < NIN; ++k) {
-                z1[0][v] = fmaf(w1[k], x[0][k], z1[0][v]);
-                z1[1][v] = fmaf(w1[k], x[1][k], z1[1][v]);
+                z[0][v] = fmaf(w1[n * NIN + k], x[0][k], z[0][v]);
+                z[1][v] = fmaf(w1[n * NIN + k], x[1][k], z[1][v]);
             }
             // no more than four neurons' weights at a time in registers
             if (v % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
-    }
-    tile_store(tile[0], n0, lane, [&](int rb, int v) { return silu(z1[rb][v]); });
+    };
+    layer1(z, lane);
+    tile_store(tile[0], n0, lane, [&](int rb, int v) { return silu(z[rb][v]); });
     __syncthreads();
     tile_gemm(w, tile[0], lane, z2);
     w.start(layer(Wb, 3), n0, lane);
     tile_transposed(tile[0], s.aT + aoff(s, m, 1), r0);
-    tile_bias(z2, P + boff(2), n0, lane);
+    tile_bias(z2, bias[1], n0, lane);
     tile_store(tile[1], n0, lane, [&](int rb, int v) { return silu(z2[rb][v]); });
+    forget(z2[0]);
+    forget(z2[1]);
     __syncthreads();
     tile_gemm(w, tile[1], lane, z3);
     w.start(layer(Wb, 4), n0, lane);
     tile_transposed(tile[1], s.aT + aoff(s, m, 2), r0);
-    tile_bias(z3, P + boff(3), n0, lane);
+    tile_bias(z3, bias[2], n0, lane);
     tile_store(tile[0], n0, lane, [&](int rb, int v) { return silu(z3[rb][v]); });
+    forget(z3[0]);
+    forget(z3[1]);
     __syncthreads();
     tile_gemm(w, tile[0], lane, z);
     w.start(layer(WbT, 4), n0, lane);
     tile_transposed(tile[0], s.aT + aoff(s, m, 3), r0);
-    tile_bias(z, P + boff(4), n0, lane);
+    tile_bias(z, bias[3], n0, lane);
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
             *reinterpret_cast<float4 *>(a4 + (32 * rb + (lane & 31)) * TILE_LDF + n0 + 8 * q + 4 * (lane >> 5)) =
                 make_float4(silu(z[rb][4 * q]), silu(z[rb][4 * q + 1]), silu(z[rb][4 * q + 2]), silu(z[rb][4 * q + 3]));
+    forget(z[0]);
+    forget(z[1]);
     __syncthreads();
     {
-        // four waves per 32 rows
-        const int half = wave >> 2;
-        float w5[4], lsum = 0.0f;
+        // four waves per 32 rows, eight rows each
+        constexpr int ROWS = HEAD_ROWS / 4;
+        const int first = HEAD_ROWS * (wave >> 2) + (wave & 3);
+        const float b5 = P[HWT_SURR_B5];
+        float p[ROWS], lsum = 0.0f;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) w5[q] = P[HWT_SURR_W5 + lane + 64 * q];
-        for (int r = wave & 3; r < HEAD_ROWS; r += 4) {
-            const int row = HEAD_ROWS * half + r;
-            float p = 0.0f;
+        for (int i = 0; i < ROWS; ++i) {
+            p[i] = 0.0f;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) p = fmaf(w5[q], a4[row * TILE_LDF + lane + 64 * q], p);
-            const float yv = wave_sum_f(p) + P[HWT_SURR_B5];
-            const float err = yv - s.tb[(size_t)m * s.B + r0 + row];
+            for (int q = 0; q < 4; ++q) p[i] = fmaf(w5[lane + 64 * q], a4[(first + 4 * i) * TILE_LDF + lane + 64 * q], p[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) p[i] = wave_sum_f(p[i]);
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+            const int row = first + 4 * i;
+            const float yv = p[i] + b5;
+            const float err = yv - target[row];
             if (lane == 0) {
                 s.y[(size_t)m * s.B + r0 + row] = yv;
                 dys[row] = 2.0f * err / (float)Bn;
@@ -469,7 +501,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     {
         const float dy[2] = {dys[lane & 31], dys[32 + (lane & 31)]};
         tile_store(tile[1], n0, lane, [&](int rb, int v) {
-            return dy[rb] * P[HWT_SURR_W5 + n0 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4] * dsilu(z[rb][v]);
+            return dy[rb] * w5[n0 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4] * dsilu(z[rb][v]);
         });
     }
     __syncthreads();
@@ -485,21 +517,34 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __syncthreads();
     tile_gemm(w, tile[1], lane, z);
     tile_transposed(tile[1], s.dzT + dzoff(s, m, 2), r0);
-    float *dz1 = s.dz1T + (size_t)m * HID * s.B + r0 + (lane & 31);
+    int again = lane;
+    asm volatile("" : "+v"(again));
+    layer1(z2, again);  // rather than kept: 32 registers
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const size_t n = n0 + 8 * (v / 4) + 4 * (lane >> 5) + v % 4;
-        dz1[n * s.B] = z[0][v] * dsilu(z1[0][v]);
-        dz1[n * s.B + 32] = z[1][v] * dsilu(z1[1][v]);
-    }
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = z[rb][4 * q + k] * dsilu(z2[rb][4 * q + k]);
+            *reinterpret_cast<float4 *>(a4 + (32 * rb + (lane & 31)) * TILE_LDF + n0 + 8 * q + 4 * (lane >> 5)) =
+                make_float4(v[0], v[1], v[2], v[3]);
+        }
+    __syncthreads();
+    float4 *dz1 = reinterpret_cast<float4 *>(s.dz1 + ((size_t)m * s.B + r0) * HID);
+#pragma unroll
+    for (int i = 0; i < TILE_ROWS / 8; ++i)
+        dz1[(wave + 8 * i) * (HID / 4) + lane] =
+            *reinterpret_cast<const float4 *>(a4 + (wave + 8 * i) * TILE_LDF + 4 * lane);
 }
 
 // --- weight gradients
 // dW_l[n][k] = sum_b dz_l[b][n] a_{l-1}[b][k], one of DW_SPLIT parts of the batch per
 // workgroup and 128 x 128 outputs: each wave 64 x 64, four fragments (a contiguous
 // kilobyte each) per four matrix instructions, all layers in one launch, with the
-// small gradients: 60 us for 4 x 8192 rows, where four launches took 127.
-constexpr int DW_TILE = 128;
+// small gradients: 39 us for 4 x 8192 rows (35 without them), where four launches took
+// 127.  Bound by memory: 200 MB, of which 100 are the two operands.
+constexpr int DW_TILE = 128, DW_AHEAD = 4;
 constexpr int DW_BLOCKS = 3 * (HID / DW_TILE) * (HID / DW_TILE) * DW_SPLIT;  // per member
 __device__ inline void weight_gradient(const Acts &s, int m, int block, int Bn)
 {
@@ -511,16 +556,35 @@ __device__ inline void weight_gradient(const Acts &s, int m, int block, int Bn)
     const uint16_t *A = s.dzT + dzoff(s, m, l) + k0 + ((size_t)(row0 >> 5) * 64 + lane) * 8;
     const uint16_t *B = s.aT + aoff(s, m, l - 1) + k0 + ((size_t)(col0 >> 5) * 64 + lane) * 8;
     f32x16 acc[2][2] = {};
-#pragma unroll 4
-    for (int k = 0; k < K / 16; ++k) {
-        const size_t at = (size_t)k * (HID / 32) * 64 * 8;
-        const bf16x8 a0 = load_frag(A + at), a1 = load_frag(A + at + 64 * 8);
-        const bf16x8 b0 = load_frag(B + at), b1 = load_frag(B + at + 64 * 8);
-        acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b0, acc[0][0], 0, 0, 0);
-        acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b1, acc[0][1], 0, 0, 0);
-        acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b0, acc[1][0], 0, 0, 0);
-        acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, acc[1][1], 0, 0, 0);
+    struct Step {
+        bf16x8 a0, a1, b0, b1;
+    };
+    const int steps = K / 16;
+    auto load = [&](int k) {
+        const size_t at = (size_t)min(k, steps - 1) * (HID / 32) * 64 * 8;
+        return Step{load_frag(A + at), load_frag(A + at + 64 * 8), load_frag(B + at), load_frag(B + at + 64 * 8)};
+    };
+    auto product = [&](const Step &f) {
+        acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a0, f.b0, acc[0][0], 0, 0, 0);
+        acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a0, f.b1, acc[0][1], 0, 0, 0);
+        acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a1, f.b0, acc[1][0], 0, 0, 0);
+        acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a1, f.b1, acc[1][1], 0, 0, 0);
+    };
+    // DW_AHEAD steps' fragments in flight
+    Step f[DW_AHEAD];
+#pragma unroll
+    for (int q = 0; q < DW_AHEAD; ++q) f[q] = load(q);
+    int k = 0;
+    for (; k + DW_AHEAD <= steps; k += DW_AHEAD) {
+#pragma unroll
+        for (int q = 0; q < DW_AHEAD; ++q) {
+            product(f[q]);
+            f[q] = load(k + q + DW_AHEAD);
+        }
     }
+#pragma unroll
+    for (int q = 0; q < DW_AHEAD - 1; ++q)
+        if (k + q < steps) product(f[q]);
     float *gw = s.gw + (((size_t)m * 3 + (l - 2)) * DW_SPLIT + split) * LAYER_W;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -532,60 +596,146 @@ __device__ inline void weight_gradient(const Acts &s, int m, int block, int Bn)
                     acc[i][j][v];
 }
 
-// Gradients of the input layer and of the biases, SMALL_N neurons per workgroup:
+// Gradients of the input layer and of the biases:
 //   dW1[n][i] = sum_b dz1[b][n] x[b][i], db1[n] = sum_b dz1[b][n],
 //   db_l[n] = sum_b dz_l[b][n] (l = 2..4).
-// A thread sums the rows of one residue of 256; the neurons share its x row and the
-// 128-byte lines in which the transposed arrays hold eight neurons' rows.
-constexpr int SMALL_N = 4, SMALL_BLOCKS = HID / SMALL_N;
-__device__ inline void small_gradients(const Acts &s, int m, int block, int Bn)
+// The rows of each residue of 256 are summed in order, then the residues by halving
+// (c and c ^ 32, 16, .. 1 of every 64), then the four 64s (gradient_of).  A workgroup
+// takes one of the 64s, a lane one neuron and the eight residues whose rows lie side by
+// side, so every load of a wave is one contiguous piece.  (With a lane per residue a
+// load was eight pieces of 16 bytes: 52 us for 4 x 8192 rows, these 23 by themselves,
+// and 4 of the launch's 39.)
+// The last steps of the halving, over a lane's eight residues.
+template <class F>
+__device__ inline float halve8(F &&v)
 {
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int n0 = block * SMALL_N;
-    float acc[SMALL_N][12] = {};
-    const float *dz1 = s.dz1T + (size_t)m * HID * s.B + (size_t)n0 * s.B;
-    const float4 *xb = reinterpret_cast<const float4 *>(s.xb + (size_t)m * s.B * NIN);
-#pragma unroll 2
-    for (int r = t; r < Bn; r += 256) {
-        const float4 x0 = xb[2 * (size_t)r], x1 = xb[2 * (size_t)r + 1];
-        const float x[NIN] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+    const float a = v(0) + v(4), b = v(1) + v(5), c = v(2) + v(6), d = v(3) + v(7);
+    return (a + c) + (b + d);
+}
+
+// Orders this wave's LDS accesses on either side.
+__device__ inline void wave_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// dW1 and db1: 64 neurons and four of the inputs; wave w takes the rows 8 (w + 4 q) on
+// of each 256, q = 0, 1.  x is the same for all lanes: from LDS.
+constexpr int IN_BLOCKS = (HID / 64) * SMALL_PARTS * 2, IN_AHEAD = 8;
+__device__ inline void input_gradient(const Acts &s, int m, int block, int Bn, float *lds)
+{
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kh = block & 1, part = block / 2 % SMALL_PARTS, n = block / 2 / SMALL_PARTS * 64 + lane;
+    const float *dz1 = s.dz1 + (size_t)m * s.B * HID + n;
+    const float *xb = s.xb + (size_t)m * s.B * NIN + 4 * kh;
+    float *xw = lds + wave * (4 * 8 * IN_AHEAD);  // the wave's x rows of one round
+    float acc[2][8][5] = {};
 #pragma unroll
-        for (int j = 0; j < SMALL_N; ++j) {
-            const float d = dz1[(size_t)j * s.B + r];
+    for (int q = 0; q < 2; ++q) {
+        // rounds of IN_AHEAD 256s: the loads of all, then their sums
+        for (int row = 64 * part + 8 * (wave + 4 * q); row < Bn; row += 256 * IN_AHEAD) {
+            const int last = (Bn - 1 - row) / 256;  // of this round's, the last 256 that has the rows
+            float d[IN_AHEAD][8];
+            const float4 x = *reinterpret_cast<const float4 *>(
+                xb + (size_t)(row + 256 * min(lane / 8 % IN_AHEAD, last) + lane % 8) * NIN);
 #pragma unroll
-            for (int k = 0; k < NIN; ++k) acc[j][k] = fmaf(d, x[k], acc[j][k]);
-            acc[j][8] += d;
+            for (int i = 0; i < IN_AHEAD; ++i)
 #pragma unroll
-            for (int l = 2; l <= 4; ++l)
-                acc[j][7 + l] += from_bf16(s.dzT[dzoff(s, m, l) + frag_unit(n0 + j, r >> 3) * 8 + (r & 7)]);
+                for (int e = 0; e < 8; ++e) d[i][e] = dz1[(size_t)(row + 256 * min(i, last) + e) * HID];
+            if (lane < 8 * IN_AHEAD) *reinterpret_cast<float4 *>(xw + 4 * lane) = x;
+            wave_order();
+#pragma unroll
+            for (int i = 0; i < IN_AHEAD; ++i)
+                if (i <= last)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float4 xr = *reinterpret_cast<const float4 *>(xw + 4 * (8 * i + e));
+                        acc[q][e][0] = fmaf(d[i][e], xr.x, acc[q][e][0]);
+                        acc[q][e][1] = fmaf(d[i][e], xr.y, acc[q][e][1]);
+                        acc[q][e][2] = fmaf(d[i][e], xr.z, acc[q][e][2]);
+                        acc[q][e][3] = fmaf(d[i][e], xr.w, acc[q][e][3]);
+                        acc[q][e][4] += d[i][e];
+                    }
+            wave_order();
         }
     }
-    __shared__ float red[4][SMALL_N * 12];
+    float v[40];
 #pragma unroll
-    for (int j = 0; j < SMALL_N; ++j)
+    for (int k = 0; k < 40; ++k) v[k] = acc[0][k / 5][k % 5] + acc[1][k / 5][k % 5];
 #pragma unroll
-        for (int k = 0; k < 12; ++k) {
-            const float v = wave_sum_f(acc[j][k]);
-            if (lane == 0) red[wave][12 * j + k] = v;
-        }
-    __syncthreads();
-    if (t < SMALL_N * 12) {
-        const float v = red[0][t] + red[1][t] + red[2][t] + red[3][t];
-        const int n = n0 + t / 12, k = t % 12;
-        float *gs = s.gs + (size_t)m * PSTRIDE;
-        if (k < NIN) gs[HWT_SURR_W1 + n * NIN + k] = v;
-        else if (k == 8) gs[HWT_SURR_B1 + n] = v;
-        else gs[boff(k - 7) + n] = v;
+    for (int h = 2; h >= 1; h >>= 1) {  // residues ^ 16, then ^ 8: the other waves
+        __syncthreads();
+        if (wave >= h && wave < 2 * h)
+#pragma unroll
+            for (int k = 0; k < 40; ++k) lds[((wave - h) * 40 + k) * 64 + lane] = v[k];
+        __syncthreads();
+        if (wave < h)
+#pragma unroll
+            for (int k = 0; k < 40; ++k) v[k] += lds[(wave * 40 + k) * 64 + lane];
+    }
+    if (wave == 0) {
+        float *gs = s.gs + ((size_t)m * SMALL_PARTS + part) * SMALL_N;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) gs[HWT_SURR_W1 + n * NIN + 4 * kh + k] = halve8([&](int e) { return v[5 * e + k]; });
+        if (kh == 0) gs[HWT_SURR_B1 + n] = halve8([&](int e) { return v[5 * e + 4]; });
     }
 }
 
-// Both in one launch: the small gradients' loads fill the time in which the matrix
-// instructions' blocks finish.
-__global__ __launch_bounds__(256) void k_gradients(Acts s, int m0, int Bn)
+// db_l: 32 neurons of one layer; wave w takes the 16 rows 16 (4 part + w) on of each 256.
+constexpr int BIAS_BLOCKS = 3 * (HID / 32) * SMALL_PARTS, BIAS_AHEAD = 8;
+__device__ inline void bias_gradient(const Acts &s, int m, int block, int Bn, float *lds)
 {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int part = block % SMALL_PARTS, nb = block / SMALL_PARTS % (HID / 32), l = 2 + block / SMALL_PARTS / (HID / 32);
+    const uint16_t *T = s.dzT + dzoff(s, m, l) + ((size_t)nb * 64 + lane) * 8;
+    float acc[8] = {};
+    auto load = [&](int r16) { return *reinterpret_cast<const uint4 *>(T + (size_t)r16 * HID * 16); };
+    auto add = [&](const uint4 &u) {
+        const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] += __uint_as_float(e & 1 ? w[e / 2] & 0xffff0000u : w[e / 2] << 16);
+    };
+    int r16 = 4 * part + wave;
+    const int end = Bn / 16;
+    for (; r16 + 16 * (BIAS_AHEAD - 1) < end; r16 += 16 * BIAS_AHEAD) {
+        uint4 u[BIAS_AHEAD];
+#pragma unroll
+        for (int i = 0; i < BIAS_AHEAD; ++i) u[i] = load(r16 + 16 * i);
+#pragma unroll
+        for (int i = 0; i < BIAS_AHEAD; ++i) add(u[i]);
+    }
+    for (; r16 < end; r16 += 16) add(load(r16));
+#pragma unroll
+    for (int h = 2; h >= 1; h >>= 1) {  // residues ^ 32, then ^ 16: the other waves
+        __syncthreads();
+        if (wave >= h && wave < 2 * h)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) lds[((wave - h) * 8 + e) * 64 + lane] = acc[e];
+        __syncthreads();
+        if (wave < h)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[e] += lds[(wave * 8 + e) * 64 + lane];
+    }
+    if (wave == 0) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] += __shfl_xor(acc[e], 32, 64);
+        if (lane < 32)
+            s.gs[((size_t)m * SMALL_PARTS + part) * SMALL_N + HWT_SURR_B1 + (l - 1) * HID + 32 * nb + lane] =
+                halve8([&](int e) { return acc[e]; });
+    }
+}
+
+// All in one launch: the small gradients' loads fill the time in which the matrix
+// instructions' blocks finish.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_gradients(Acts s, int m0, int Bn)
+{
+    __shared__ __attribute__((aligned(16))) float lds[2 * 40 * 64];
     const int m = m0 + blockIdx.y;
-    if (blockIdx.x < SMALL_BLOCKS) small_gradients(s, m, blockIdx.x, Bn);
-    else weight_gradient(s, m, blockIdx.x - SMALL_BLOCKS, Bn);
+    const int block = blockIdx.x;
+    if (block < IN_BLOCKS) input_gradient(s, m, block, Bn, lds);
+    else if (block < IN_BLOCKS + DW_BLOCKS) weight_gradient(s, m, block - IN_BLOCKS, Bn);
+    else bias_gradient(s, m, block - IN_BLOCKS - DW_BLOCKS, Bn, lds);
 }
 
 // Dense gradient of parameter p from the partial sums, each in order.
@@ -600,7 +750,13 @@ __device__ inline float gradient_of(const Acts &s, int m, int p, int nhead)
         for (int q = 0; q < DW_SPLIT; ++q) g += src[(size_t)q * LAYER_W];
         return g;
     }
-    if (p < HWT_SURR_W5) return s.gs[(size_t)m * PSTRIDE + p];
+    if (p < HWT_SURR_W5) {
+        static_assert(HWT_SURR_W1 == 0 && HWT_SURR_B1 == HID * NIN && HWT_SURR_W2 == HWT_SURR_B1 + HID, "W1, b1 first");
+        const int b = p < HWT_SURR_W2 ? p : p < HWT_SURR_W3 ? p - HWT_SURR_B2 + HWT_SURR_W2
+                      : p < HWT_SURR_W4 ? p - HWT_SURR_B3 + HWT_SURR_W2 + HID : p - HWT_SURR_B4 + HWT_SURR_W2 + 2 * HID;
+        const float *src = s.gs + (size_t)m * SMALL_PARTS * SMALL_N + b;
+        return ((src[0] + src[SMALL_N]) + src[2 * SMALL_N]) + src[3 * SMALL_N];
+    }
     // w5 and b5: a chain of adds over the tiles, its loads 32 at a time (one at a time
     // they were 100 us of a step)
     const float *src = s.hp + (size_t)m * (s.B / HEAD_ROWS) * (HID + 1) + (p - HWT_SURR_W5);
@@ -1071,7 +1227,7 @@ namespace {
 int forward_backward(hwt_surrogate *s, int m0, int mc, int Bn)
 {
     k_train_tile<<<dim3(Bn / TILE_ROWS, mc), 512, 0, s->stream>>>(s->net, s->acts, m0, Bn);
-    k_gradients<<<dim3(SMALL_BLOCKS + DW_BLOCKS, mc), 256, 0, s->stream>>>(s->acts, m0, Bn);
+    k_gradients<<<dim3(IN_BLOCKS + DW_BLOCKS + BIAS_BLOCKS, mc), 256, 0, s->stream>>>(s->acts, m0, Bn);
     SURR_HIP(hipGetLastError());
     return HWT_OK;
 }
@@ -1220,7 +1376,7 @@ int hwt_surr_create(hwt_surrogate **out, int32_t train_capacity, int32_t infer_c
     const size_t om1 = carve(M * PSTRIDE * 4), om2 = carve(M * PSTRIDE * 4);
     const size_t oxb = carve(M * B * NIN * 4), otb = carve(M * B * 4);
     const size_t oaT = carve(M * 3 * B * HID * 2), odzT = carve(M * 3 * B * HID * 2), odz1 = carve(M * HID * B * 4);
-    const size_t oy = carve(M * B * 4), ogw = carve(M * 3 * DW_SPLIT * LAYER_W * 4), ogs = carve(M * PSTRIDE * 4);
+    const size_t oy = carve(M * B * 4), ogw = carve(M * 3 * DW_SPLIT * LAYER_W * 4), ogs = carve(M * SMALL_PARTS * SMALL_N * 4);
     const size_t ohp = carve(M * (B / HEAD_ROWS) * (HID + 1) * 4), oloss = carve(M * 8), og = carve(M * PSTRIDE * 4);
     const size_t oX = carve(T * NIN * 4), otg = carve(T * 4), operm = carve(M * T * 4), orows = carve(B * 4);
     const size_t obad = carve(4), ofbi = carve(I * 4), ofbc = carve(16 * 4), ofbt = carve(I * 8);
@@ -1247,7 +1403,7 @@ int hwt_surr_create(hwt_surrogate **out, int32_t train_capacity, int32_t infer_c
     a.tb = (float *)(b + otb);
     a.aT = (uint16_t *)(b + oaT);
     a.dzT = (uint16_t *)(b + odzT);
-    a.dz1T = (float *)(b + odz1);
+    a.dz1 = (float *)(b + odz1);
     a.y = (float *)(b + oy);
     a.gw = (float *)(b + ogw);
     a.gs = (float *)(b + ogs);
