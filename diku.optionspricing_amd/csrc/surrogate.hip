@@ -855,6 +855,10 @@ __global__ void k_refresh_bf16(Net net, int members)
 // accumulator starts at its bias.  The output layer reduces per row across
 // lanes and waves in a fixed order.  The yield curve is staged in LDS for the
 // inputs.
+// Bound by issue: 5.5 vector instructions a SiLU, two of them transcendental, keep
+// the vector unit busy for 60% of the time and the matrix unit is for 47%, and the two
+// hardly overlap.  (Neither wave priorities nor two tiles in one workgroup, one a step
+// behind the other, changed that: 991 and 1075 us.)
 constexpr int INF_YMAX = 256;  // keeps two 128-row tiles per CU in LDS
 
 struct InferArgs {
@@ -914,6 +918,26 @@ __device__ inline void silu_to_act(const f32x16 (&acc)[2][4], uint16_t *act, int
         }
 }
 
+// A wave's weights of one layer (two blocks of 32 neurons), INF_AHEAD of the 16
+// k-steps in flight, the first of the next layer during a layer's epilogue (475,000
+// rows: 1085 us without, 987; 3 or 4 steps ahead spill, 1000 and 1028).
+constexpr int INF_AHEAD = 2;
+struct InferWeights {
+    bf16x8 w[INF_AHEAD][2];
+    const uint16_t *p;
+    __device__ void start(const uint16_t *W, int n0, int lane)
+    {
+        p = W + ((size_t)(n0 >> 5) * (HID / 16) * 64 + lane) * 8;
+#pragma unroll
+        for (int k = 0; k < INF_AHEAD; ++k) load(k);
+    }
+    __device__ void load(int k)
+    {
+        w[k % INF_AHEAD][0] = load_frag(p + k * 64 * 8);
+        w[k % INF_AHEAD][1] = load_frag(p + (HID / 16 + k) * 64 * 8);
+    }
+};
+
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_infer(InferArgs g)
 {
     static_assert(INF_ROWS == 128, "the layer-1 and head mappings assume 128 rows per tile");
@@ -925,8 +949,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     __shared__ int32_t okf[INF_ROWS];
     __shared__ int32_t fb_local[INF_ROWS];
     __shared__ int32_t fb_n, fb_out, fb_base;
-    __shared__ double yr[INF_YMAX];
-    __shared__ int32_t yd[INF_YMAX];
+    // the curve, while the inputs are made; then each member's b2..b4 and w5
+    __shared__ __attribute__((aligned(16))) char front[4 * HID * 4];
+    static_assert(INF_YMAX * 12 <= (int)sizeof(front), "the curve fits");
+    double *yr = reinterpret_cast<double *>(front);
+    int32_t *yd = reinterpret_cast<int32_t *>(front + INF_YMAX * 8);
+    float *vec = reinterpret_cast<float *>(front);
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int r0 = blockIdx.x * INF_ROWS;
     const int nrows = g.rows ? *g.row_count : g.o.n;
@@ -967,8 +995,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 
     const int mrow = lane & 31, khalf = 8 * (lane >> 5);
     const int n0 = wave * 64;  // this wave's output neurons in the hidden layers
+    InferWeights w;
+    w.start(g.net.Wb, n0, lane);
     for (int m = 0; m < g.members; ++m) {
         const float *P = g.net.P + (size_t)m * PSTRIDE;
+        // the member's vectors into LDS, requested beside layer 1's (each layer
+        // fetching its own from L2 waited for it)
+        float own[4];
+#pragma unroll
+        for (int l = 2; l <= 4; ++l) own[l - 2] = P[boff(l) + t];
+        own[3] = P[HWT_SURR_W5 + t];
         // layer 1 (FP32 MFMA 32x32x2, K = 8 in four steps): D[neuron][row] =
         // b1 + W1 x^T, with the lane's A value W1[n][k] and B value x[row][k]
         {
@@ -986,27 +1022,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
                     acc[1][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, bx, acc[1][nb], 0, 0, 0);
                 }
             }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) vec[k * HID + t] = own[k];
             silu_to_act(acc, act, n0, lane);
         }
         __syncthreads();
         for (int l = 2; l <= 4; ++l) {
-            const uint16_t *W = g.net.Wb + ((size_t)m * 3 + (l - 2)) * LAYER_W;
-            const uint16_t *wa0 = W + ((size_t)(n0 >> 5) * (HID / 16) * 64 + lane) * 8;
-            const uint16_t *wa1 = wa0 + (HID / 16) * 64 * 8;
             const uint16_t *ab = act + mrow * ACT_LD + khalf;
             f32x16 acc[2][4];
-            bias_init(acc, P + boff(l), n0, lane);
-#pragma unroll 2
-            for (int k = 0; k < HID; k += 16) {
-                const bf16x8 a0 = load_frag(wa0 + 32 * k), a1 = load_frag(wa1 + 32 * k);
+            bias_init(acc, vec + (l - 2) * HID, n0, lane);
+#pragma unroll
+            for (int k = 0; k < HID / 16; ++k) {
+                const bf16x8 a0 = w.w[k % INF_AHEAD][0], a1 = w.w[k % INF_AHEAD][1];
 #pragma unroll
                 for (int nb = 0; nb < 4; ++nb) {
-                    const bf16x8 b =
-                        __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(ab + nb * 32 * ACT_LD + k));
+                    const bf16x8 b = load_frag(ab + nb * 32 * ACT_LD + 16 * k);
                     acc[0][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b, acc[0][nb], 0, 0, 0);
                     acc[1][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b, acc[1][nb], 0, 0, 0);
                 }
+                if (k + INF_AHEAD < HID / 16) w.load(k + INF_AHEAD);
+                __builtin_amdgcn_sched_barrier(0);  // reads no further ahead: registers are full
             }
+            // the next layer's first weights, during this one's epilogue (the last
+            // member's last: its own again)
+            w.start(g.net.Wb + ((size_t)min(l < 4 ? m : m + 1, g.members - 1) * 3 + (l < 4 ? l - 1 : 0)) * LAYER_W, n0, lane);
             __syncthreads();  // every wave has read this layer's input tile
             if (l < 4) {
                 silu_to_act(acc, act, n0, lane);
@@ -1021,7 +1060,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
                         const int col = n0 + 32 * mb + 8 * q + 4 * (lane >> 5);
-                        const float4 w5 = *reinterpret_cast<const float4 *>(P + HWT_SURR_W5 + col);
+                        const float4 w5 = *reinterpret_cast<const float4 *>(vec + 3 * HID + col);
 #pragma unroll
                         for (int nb = 0; nb < 4; ++nb) {
                             const f32x16 &a = acc[mb][nb];
