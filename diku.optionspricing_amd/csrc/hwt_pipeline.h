@@ -95,6 +95,8 @@ constexpr HWT_HD int tri_part(int w, bool spread)  // w up to TRI_GROUP_WIDTH, o
            : w <= 88 ? 3 + (w + 7) / 8
                      : (w + 15) / 16 - 3;
 }
+constexpr int SMALL_MAX = 2048;  // options of a batch that k_price_small takes, a wave each
+constexpr int SMALL_YMAX = 512;  // ... and points of its curve
 // Wave b takes tasks b % TRI_QUEUES + i * TRI_QUEUES, claimed from its own queue
 // head.  With one head for all, 4,096 waves' claims of 1,000 to 10,000 tasks
 // serialise at 9 ns each (60k skewed batch 486 us).
@@ -107,7 +109,7 @@ constexpr int NBUCKET_MAX = NBUCKET > NBUCKET_TRI ? NBUCKET : NBUCKET_TRI;
 constexpr int CLASS_ROWS = 1, CLASS_FLAT = 2;
 enum Tally {
     T_QUEUE = 0,    // next task of the wide-tree kernel (tasks [0, T_NLARGE))
-    T_QUEUE_S = 1,  // (unused: the narrow-tree kernel strides statically)
+    T_QUEUE_S = 1,  // next mid-class task (fused kernel; the narrow-tree kernel strides statically)
     T_NTASK = 2,
     T_NLARGE = 3,
     T_INVALID = 4,
@@ -153,6 +155,7 @@ enum Tally {
     T_TBIG = T_HOST,
     T_TWIN = T_HOST + 1,
     T_TNGROUP = T_HOST + 2,
+    T_SMALL = T_HOST + 3,   // options of the last execution if k_price_small ran it, else 0
     T_TSTART = T_HOST + 8,  // TRI_PARTS entries
     T_TGROUP = T_HOST + 56, // TRI_PARTS entries
     A_NWIDE = T_HOST + 104,  // accumulated by k_setup: wide trees
@@ -204,6 +207,8 @@ __global__ void k_price_fused(const OptConst *__restrict__ cst, const double *__
 __global__ void k_price_tri(const OptConst *__restrict__ cst, const double *__restrict__ edge,
                             const int32_t *__restrict__ order, int32_t *__restrict__ tally, double *__restrict__ out,
                             double *__restrict__ scratch);
+__global__ void k_price_small(DevOpts o, DevYield y, int32_t maxWidth, double unit_dmin, OptConst *__restrict__ cst,
+                              int32_t *__restrict__ tally, double *__restrict__ out, double *__restrict__ scratch);
 __global__ void k_price_redo(const OptConst *__restrict__ cst, const double *__restrict__ edge,
                              const int32_t *__restrict__ redo, int32_t *__restrict__ tally,
                              double *__restrict__ out, double *__restrict__ scratch);

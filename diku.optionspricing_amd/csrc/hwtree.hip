@@ -29,6 +29,7 @@
 // per-step reductions, against 2n steps plus n reductions in seq/Seq.hpp.
 #include "hwt_lane.h"
 #include "hwt_pipeline.h"
+#include "hwt_setup.h"
 #include "hwt_tri.h"
 #include "../../include/hwtree.h"
 #include "hwt_internal.h"
@@ -286,6 +287,7 @@ __device__ __forceinline__ void scan_offsets(const int32_t *__restrict__ hist, i
     if (writer && tid == 0) {
         tally[T_QUEUE] = 0;
         tally[T_QUEUE_S] = 0;
+        if (TRI) tally[T_SMALL] = 0;
         tally[T_QUEUE_R] = 0;
         tally[T_QUEUE_F] = 0;
         int64_t *t64 = reinterpret_cast<int64_t *>(tally);
@@ -392,19 +394,8 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, in
         reinterpret_cast<unsigned long long *>(tally)[T_T0 / 2] = __builtin_amdgcn_s_memrealtime();
     // the option's fields are requested before the curve is staged, so the
     // two loads overlap
-    double strike = 0.0, mat = 0.0, len = 0.0, a = 0.0, sigma = 0.0;
-    uint16_t tu = 0, ts = 0;
-    int8_t type = 0;
-    if (mine && !o.consts) {
-        strike = o.strike[i];
-        mat = o.maturity[i];
-        len = o.length[i];
-        tu = o.term_unit[i];
-        ts = o.term_steps[i];
-        a = o.a[i];
-        sigma = o.sigma[i];
-        type = o.type[i];
-    }
+    OptFields f{};
+    if (mine && !o.consts) f = option_fields(o, i);
     for (int k = tid; k < Y::NB; k += SETUP_BLOCK) lh[k] = 0;
     if (tid < 3) lsum[tid] = 0ull;
     if (tid < 3) lbad[tid] = 0;
@@ -435,101 +426,69 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, in
     bool invalid = false, unsupported = false, is_wide = false;
     int b = -1, r = 0;  // bucket, rank among the block's options in it
     if (mine) {
-        int32_t st;
-        if (o.consts) {
-            const hwt_option_constants_f64 k = o.consts[i];
-            tu = k.term_unit;
-            st = constants_given(k.t, k.dt, k.dr, k.X, k.M, k.jmax, k.n, k.width, k.term_unit, k.type, maxWidth,
-                                 o.consts_f32 != 0, c);
-        } else {
-            st = option_constants(strike, mat, len, tu, ts, a, sigma, type, maxWidth, c);
-        }
-        c.status = st;
-        if (st == ST_INVALID) {
-            out[i] = NAN;
-            invalid = true;
-        } else if (st == ST_UNSUPPORTED) {
-            out[i] = NAN;
-            unsupported = true;
-        } else if (c.n == 0) {
-            out[i] = 100.0;  // no steps: the face value (seq/Seq.hpp:119,171)
-        } else {
-            const double tn = c.n * c.dt;
-            c.Pn = exp(-yield(tn, tu) * tn);
-            if (c.e < 0) {
-                out[i] = 100.0 * c.Pn;  // exercise outside the tree: the zero-coupon bond
-            } else {
-                const double te = c.e * c.dt;
-                c.Pe = exp(-yield(te, tu) * te);
-                TreeShape t{c.w, c.jmax, c.M, c.dr, c.dt, 0.0, 0.0};
-                TriEdge edges{};
-                if constexpr (TRI) {
-                    const EdgeDiscounts ed = edge_discounts(t);
-                    edge_factors(t, ed);
-                    edges = tri_edge(t, ed);
-                    __builtin_memcpy(tab, &edges, sizeof(edges));
-                } else if (t.w >= 7) {
-                    // trees of 7 or more nodes (all but the tiniest) take their
-                    // edge discounts from four exponentials and the table from
-                    // its closed form
-                    const EdgeDiscounts ed = edge_discounts(t);
-                    edge_factors(t, ed);
-                    edge_table_closed(t, ed, tab);
-                    c.unit = unit_form_ok(t, tab, unit_dmin, ed.E0, ed.Ea) ? 1 : 0;
-                } else {
-                    edge_factors(t);
-                    double gtab[EDGE_TAB];
-                    edge_table_general(t, gtab);
-#pragma unroll
-                    for (int k = 0; k < EDGE_TAB; ++k) tab[k] = gtab[k];
-                    c.unit = unit_form_ok(t, tab, unit_dmin) ? 1 : 0;
-                }
-                c.rho = t.rho;
-                c.rhop = t.rhop;
-                work = (unsigned long long)dual_node_updates(c.n, c.e, c.jmax);
-                seq_work = (unsigned long long)seq_node_updates(c.n, c.jmax);
-                const bool wide = (c.w + WAVE - 1) / WAVE > KSMALL;
-                is_wide = wide;
-                if (!TRI && wide && reprice) c.sigmas = window_sigmas(c);  // should FP64 price it again
-                int64_t key = (int64_t)work;
-                bool grouped = false, held = false;  // TRI: a part's tree; the tridiagonal form holds it
-                if constexpr (TRI) {
-                    grouped = c.w <= (spread ? TRI_SPREAD_WIDTH : TRI_GROUP_WIDTH);
-                    int lo = c.jmax, up = c.jmax;
-                    if (!grouped) {
-                        // priced over the nodes that carry weight, most at step n
-                        c.sigmas = window_sigmas(c);
-                        const Reach reach = make_reach(c.sigmas, c.M, c.dr, c.dt, c.n, c.jmax);
-                        key = (int64_t)reach_updates(reach, c.n, c.e);
-                        reach_at(reach, c.n, min(c.e, c.jmax) + (c.n - c.e), lo, up);
+        const int32_t st = option_record(o, i, f, maxWidth, c);
+        invalid = st == ST_INVALID;
+        unsupported = st == ST_UNSUPPORTED;
+        int64_t key = 0;
+        TriKind kind = TRI_DONE;
+        double value = NAN;
+        if constexpr (TRI) {
+            TriEdge edges{};
+            kind = tri_setup(c, f.term_unit, yield, spread != 0, unit_dmin, edges, key, value);
+            __builtin_memcpy(tab, &edges, sizeof(edges));
+        } else if (st == ST_OK) {
+            value = 100.0;  // no steps: the face value (seq/Seq.hpp:119,171)
+            if (c.n > 0) {
+                const double tn = c.n * c.dt;
+                c.Pn = exp(-yield(tn, f.term_unit) * tn);
+                value = 100.0 * c.Pn;  // exercise outside the tree: the zero-coupon bond
+                if (c.e >= 0) {
+                    const double te = c.e * c.dt;
+                    c.Pe = exp(-yield(te, f.term_unit) * te);
+                    kind = TRI_GENERAL;
+                    TreeShape t{c.w, c.jmax, c.M, c.dr, c.dt, 0.0, 0.0};
+                    if (t.w >= 7) {
+                        // trees of 7 or more nodes (all but the tiniest) take their
+                        // edge discounts from four exponentials and the table from
+                        // its closed form
+                        const EdgeDiscounts ed = edge_discounts(t);
+                        edge_factors(t, ed);
+                        edge_table_closed(t, ed, tab);
+                        c.unit = unit_form_ok(t, tab, unit_dmin, ed.E0, ed.Ea) ? 1 : 0;
+                    } else {
+                        edge_factors(t);
+                        edge_table(t, tab);
+                        c.unit = unit_form_ok(t, tab, unit_dmin) ? 1 : 0;
                     }
-                    held = tri_ok(t, edges, c.n, max(lo, up), grouped ? 100.0f : 200.0f) &&
-                           (grouped || lo + up + 17 <= TRI_MAX_NODES);
-                    if (!held) {
-                        // the general kernel's scales (unit_form_ok)
-                        double etab[EDGE_TAB];
-                        edge_table(t, etab);
-                        c.unit = unit_form_ok(t, etab, unit_dmin) ? 1 : 0;
-                        c.sigmas = window_sigmas(c);
-                    }
+                    c.rho = t.rho;
+                    c.rhop = t.rhop;
                 }
-                switch (sort) {
-                case 'W': case 'w': key = c.w; break;
-                case 'H': case 'h': key = c.n; break;
-                case '-': key = 0; break;
-                default: break;
-                }
-                if (TRI) {
-                    if (!held) b = B_TRI_BIG + log_bucket(key, 2, NBUCKET_TRI - B_TRI_BIG);
-                    else if (!grouped) b = B_TRI_WIN + log_bucket(key, 8, B_TRI_BIG - B_TRI_WIN);
-                    else b = tri_bucket(tri_part(c.w, spread != 0), c.n);
-                } else if (wide) b = B_WIDE + log_bucket(key, 8, NBUCKET - B_WIDE);
-                else if ((classes & CLASS_FLAT) && c.w <= FLAT_MAX_WIDTH) b = flat_bucket(c.w, c.n);
-                else if (c.w > ROW_MAX_WIDTH || !(classes & CLASS_ROWS)) b = B_MID + log_bucket(key, 4, B_WIDE - B_MID);
-                else b = row_bucket(c.w, c.n);
-                r = atomicAdd(&lh[b], 1);
-                if (wide) wide_work = work;
             }
+        }
+        if (kind == TRI_DONE) out[i] = value;
+        else {
+            work = (unsigned long long)dual_node_updates(c.n, c.e, c.jmax);
+            seq_work = (unsigned long long)seq_node_updates(c.n, c.jmax);
+            const bool wide = (c.w + WAVE - 1) / WAVE > KSMALL;
+            is_wide = wide;
+            if (!TRI && wide && reprice) c.sigmas = window_sigmas(c);  // should FP64 price it again
+            if (!TRI || kind != TRI_WINDOWED) key = (int64_t)work;
+            switch (sort) {
+            case 'W': case 'w': key = c.w; break;
+            case 'H': case 'h': key = c.n; break;
+            case '-': key = 0; break;
+            default: break;
+            }
+            if (TRI) {
+                if (kind == TRI_GENERAL) b = B_TRI_BIG + log_bucket(key, 2, NBUCKET_TRI - B_TRI_BIG);
+                else if (kind == TRI_WINDOWED) b = B_TRI_WIN + log_bucket(key, 8, B_TRI_BIG - B_TRI_WIN);
+                else b = tri_bucket(tri_part(c.w, spread != 0), c.n);
+            } else if (wide) b = B_WIDE + log_bucket(key, 8, NBUCKET - B_WIDE);
+            else if ((classes & CLASS_FLAT) && c.w <= FLAT_MAX_WIDTH) b = flat_bucket(c.w, c.n);
+            else if (c.w > ROW_MAX_WIDTH || !(classes & CLASS_ROWS)) b = B_MID + log_bucket(key, 4, B_WIDE - B_MID);
+            else b = row_bucket(c.w, c.n);
+            r = atomicAdd(&lh[b], 1);
+            if (wide) wide_work = work;
         }
     }
     // the block's tallies: one LDS atomic per wave and counter (every lane
@@ -626,6 +585,48 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_order(int32_t n, const int32_t 
     const int2 s = (i < n) ? slot[i] : make_int2(-1, 0);  // requested first, so it arrives during the scan
     scan_offsets<TRI>(hist, soffs, order, tally, asc, classes, blockIdx.x == 0);
     if (s.x >= 0) order[soffs[s.x] + s.y] = i;
+}
+
+// The counts of an execution by k_price_small (T_SMALL), from its constants: one
+// block, at sync time (k_setup and k_order count a larger batch as they go).
+__global__ __launch_bounds__(256) void k_small_tally(const OptConst *__restrict__ cst, int32_t *__restrict__ tally)
+{
+    const int n = tally[T_SMALL];
+    if (n == 0) return;  // the last execution was another batch's
+    __shared__ unsigned long long sums[3];  // work, seq work, wide work
+    __shared__ int32_t counts[4];           // invalid, unsupported, tasks, wide
+    const int t = threadIdx.x;
+    if (t < 3) sums[t] = 0;
+    if (t < 4) counts[t] = 0;
+    __syncthreads();
+    for (int i = t; i < n; i += 256) {
+        const int st = cst[i].status, h = cst[i].n, e = cst[i].e, jmax = cst[i].jmax;
+        if (st == ST_INVALID) atomicAdd(&counts[0], 1);
+        else if (st == ST_UNSUPPORTED) atomicAdd(&counts[1], 1);
+        else if (h > 0 && e >= 0) {
+            const unsigned long long work = (unsigned long long)dual_node_updates(h, e, jmax);
+            atomicAdd(&counts[2], 1);
+            atomicAdd(&sums[0], work);
+            atomicAdd(&sums[1], (unsigned long long)seq_node_updates(h, jmax));
+            if ((cst[i].w + WAVE - 1) / WAVE > KSMALL) {
+                atomicAdd(&counts[3], 1);
+                atomicAdd(&sums[2], work);
+            }
+        }
+    }
+    __syncthreads();
+    if (t == 0) {
+        unsigned long long *t64 = reinterpret_cast<unsigned long long *>(tally);
+        t64[T_WORK / 2] = sums[0];
+        t64[T_SEQWORK / 2] = sums[1];
+        t64[T_WORKW / 2] = sums[2];
+        tally[T_INVALID] = counts[0];
+        tally[T_UNSUP] = counts[1];
+        tally[T_NTASK] = counts[2];
+        tally[T_NLARGE] = counts[3];
+        tally[T_NPAD] = tally[T_NREDO] = 0;
+        for (int k = T_XFLOP; k < T_XPLAIN + 2; ++k) tally[k] = 0;
+    }
 }
 
 // The wide trees' stencil steps over their light-cone windows, padding slots
@@ -800,6 +801,7 @@ struct hwt_plan {
     hipStream_t side = nullptr;       // narrow-tree kernel runs here, concurrently
     hipEvent_t fork = nullptr, join = nullptr;
     double *scratch_wide = nullptr;
+    bool small = false;  // k_price_small has run: its counts are made at sync time
     int32_t *redo = nullptr;  // mixed mode: options re-priced in FP64
     int grid_redo = 0;
     double *cols = nullptr;  // form 1 tree columns
@@ -845,6 +847,16 @@ static int waves_per_cu(Kernel *k, int fallback)
     return n;
 }
 
+// Whether a batch is priced by k_price_small: FP64, at most as many options as that
+// kernel's waves fit the chip and the plan has scratch slots for, a curve that a wave
+// stages.  It was the faster one wherever it fits: strike ladders of 100, 1,000, 2,000
+// options 17, 17.5, 20 us (general pipeline 32.5, 34, 36), trees 7 to 511 nodes wide
+// 55, 60, 74 (70, 76, 82).  A count in device memory goes the general way.
+static bool small_batch(const hwt_plan *p, const DevOpts &o, const DevYield &y)
+{
+    return plan_tri(p->cfg) && o.n <= std::min(SMALL_MAX, p->grid_wide) && y.n <= SMALL_YMAX && !o.count;
+}
+
 static int launch_pipeline(hwt_plan *p, const DevOpts &o, const DevYield &y, double *out, hipStream_t s, bool time_kernel)
 {
     const int n = o.n;
@@ -869,6 +881,16 @@ static int launch_pipeline(hwt_plan *p, const DevOpts &o, const DevYield &y, dou
         // form 1 prices trees up to its column length; wider ones are unsupported
         const int max_width = p->cfg.form == HWT_FORM_LANE ? p->lane_width : WAVE_MAX_WIDTH;
         const bool tri = plan_tri(p->cfg);
+        if (small_batch(p, o, y)) {
+            p->small = true;
+            if (time_kernel)
+                for (hipEvent_t e : {p->evk0, p->evw0}) HWT_HIP(hipEventRecord(e, s));
+            k_price_small<<<n, WAVE, 0, s>>>(o, y, max_width, unit_dmin, p->cst, p->tally, out, p->scratch_wide);
+            if (time_kernel)
+                for (hipEvent_t e : {p->evw1, p->evn0, p->evn1, p->evk1}) HWT_HIP(hipEventRecord(e, s));
+            HWT_HIP(hipGetLastError());
+            return HWT_OK;
+        }
         if (tri) {
             k_setup<true><<<blocks, SETUP_BLOCK, 0, s>>>(o, y, sort, max_width, unit_dmin, CLASS_ROWS,
                                                          n <= TRI_SPREAD ? 1 : 0, 0, p->cst, p->edge, p->slot, p->hist,
@@ -1222,6 +1244,11 @@ int hwt_plan_sync(hwt_plan *p, hwt_stats *stats)
 {
     if (!p) return fail(HWT_EINVAL, "hwt_plan_sync: null plan");
     hipStream_t s = p->last_stream ? p->last_stream : p->stream;
+    if (p->small) {
+        (void)hipGetLastError();
+        k_small_tally<<<1, 256, 0, s>>>(p->cst, p->tally);
+        HWT_HIP(hipGetLastError());
+    }
     // with stats: what the windowed kernel's steps executed in the last
     // execution, counted once from its schedule (form 2 only)
     if (stats && !p->steps_counted && p->last_n > 0 && p->cfg.form != HWT_FORM_LANE) {
@@ -2017,9 +2044,13 @@ int hwt_price_device_noalloc(const hwt_options_f64 *dopts, const hwt_yield_f64 *
     // the array keeps the last call's contents: counters start from zero by a
     // fill kernel (no memset node, so a caller may capture the call in a graph)
     (void)hipGetLastError();
-    k_reset<<<1, 1024, 0, s>>>(v.tally);
-    HWT_HIP(hipGetLastError());
-    return launch_pipeline(&v, dev_opts(*dopts), DevYield{dyield->n, dyield->rate, dyield->day}, dout, s, false);
+    const DevOpts o = dev_opts(*dopts);
+    const DevYield y{dyield->n, dyield->rate, dyield->day};
+    if (!small_batch(&v, o, y)) {
+        k_reset<<<1, 1024, 0, s>>>(v.tally);
+        HWT_HIP(hipGetLastError());
+    }
+    return launch_pipeline(&v, o, y, dout, s, false);
 }
 
 int hwt_alphas_f64(const hwt_options_f64 *opts, const hwt_yield_f64 *yield, int64_t *offsets, double *alphas)
