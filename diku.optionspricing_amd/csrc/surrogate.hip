@@ -1122,9 +1122,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // and stages both lists in LDS, so the global counters see one atomic per
 // list per block (same-address atomics serialise in L2: one per 256 options
 // cost more than the whole test).  Order inside the lists is arbitrary.
-constexpr int BOX_CHUNK = 4096;
+// A wave takes its places in a staged list with one LDS atomic: 4,096 a block on two
+// addresses took most of its time (500,000 options: 27 us with 256 threads, now 13.5;
+// chunks of 2,048 15 us, of 1,024 25: the lists' heads).
+constexpr int BOX_CHUNK = 4096, BOX_THREADS = 1024;
 
-__global__ __launch_bounds__(256) void k_box(SOpts o, int32_t *__restrict__ fb_idx, int32_t *__restrict__ fb_count,
+__global__ __launch_bounds__(BOX_THREADS) void k_box(SOpts o, int32_t *__restrict__ fb_idx, int32_t *__restrict__ fb_count,
                                              int32_t *__restrict__ rows, int32_t *__restrict__ row_count)
 {
     __shared__ int32_t nin, nout, bin, bout;
@@ -1132,11 +1135,24 @@ __global__ __launch_bounds__(256) void k_box(SOpts o, int32_t *__restrict__ fb_i
     const int t = threadIdx.x, i0 = blockIdx.x * BOX_CHUNK;
     if (t == 0) nin = nout = 0;
     __syncthreads();
-    for (int i = i0 + t; i < min(i0 + BOX_CHUNK, o.n); i += 256) {
+    const int lane = t & 63;
+    const unsigned long long below = (1ull << lane) - 1;
+#pragma unroll
+    for (int k = 0; k < BOX_CHUNK / BOX_THREADS; ++k) {
         // the parameter test alone; a listed option that still fails the tree
         // test is sent to the fallback list by the inference kernel
-        if (surr_param_box(o, i)) lin[atomicAdd(&nin, 1)] = i;
-        else lout[atomicAdd(&nout, 1)] = i;
+        const int i = i0 + t + BOX_THREADS * k;
+        const bool in = i < o.n && surr_param_box(o, i), off = i < o.n && !in;
+        const unsigned long long mi = __ballot(in), mo = __ballot(off);
+        int pi = 0, po = 0;
+        if (lane == 0) {
+            if (mi) pi = atomicAdd(&nin, (int)__popcll(mi));
+            if (mo) po = atomicAdd(&nout, (int)__popcll(mo));
+        }
+        pi = __builtin_amdgcn_readfirstlane(pi);
+        po = __builtin_amdgcn_readfirstlane(po);
+        if (in) lin[pi + __popcll(mi & below)] = i;
+        if (off) lout[po + __popcll(mo & below)] = i;
     }
     __syncthreads();
     if (t == 0) {
@@ -1145,8 +1161,18 @@ __global__ __launch_bounds__(256) void k_box(SOpts o, int32_t *__restrict__ fb_i
         if (nout) atomicAdd(&fb_count[1], nout);
     }
     __syncthreads();
-    for (int k = t; k < nin; k += 256) rows[bin + k] = lin[k];
-    for (int k = t; k < nout; k += 256) fb_idx[bout + k] = lout[k];
+    for (int k = t; k < nin; k += BOX_THREADS) rows[bin + k] = lin[k];
+    for (int k = t; k < nout; k += BOX_THREADS) fb_idx[bout + k] = lout[k];
+}
+
+// The start of a pass: its counters to zero and the device's constant-rate wall clock
+// into stamp 0.  Stamps mark a pass's parts, which events cannot give inside a graph:
+// 1 as the gather starts, 2 as the last of the scatter's blocks ends (kernels of their
+// own took 4 us each).
+__global__ void k_begin_pass(int32_t *count, uint64_t *stamps)
+{
+    if (threadIdx.x < 8) count[threadIdx.x] = 0;
+    if (threadIdx.x == 0) stamps[0] = stamps[1] = stamps[2] = __builtin_amdgcn_s_memrealtime();
 }
 
 // Fallback list -> compact option arrays, and prices back to input order.
@@ -1156,9 +1182,11 @@ struct Compact {
     int8_t *type;
 };
 
-__global__ void k_fb_gather(SOpts o, const int32_t *__restrict__ idx, const int32_t *__restrict__ count, Compact c)
+__global__ void k_fb_gather(SOpts o, const int32_t *__restrict__ idx, const int32_t *__restrict__ count, Compact c,
+                            uint64_t *__restrict__ stamps)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j == 0) stamps[1] = __builtin_amdgcn_s_memrealtime();
     if (j >= count[0]) return;
     const int i = idx[j];
     c.strike[j] = o.strike[i];
@@ -1172,16 +1200,13 @@ __global__ void k_fb_gather(SOpts o, const int32_t *__restrict__ idx, const int3
 }
 
 __global__ void k_fb_scatter(const int32_t *__restrict__ idx, const int32_t *__restrict__ count,
-                             const double *__restrict__ tmp, double *__restrict__ out)
+                             const double *__restrict__ tmp, double *__restrict__ out, uint64_t *__restrict__ stamps)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= count[0]) return;
-    out[idx[j]] = tmp[j];
+    const int j = blockIdx.x * blockDim.x + threadIdx.x, n = count[0];
+    if (j < n) out[idx[j]] = tmp[j];
+    if (threadIdx.x == 0 && (j < n || j == 0))
+        atomicMax(reinterpret_cast<unsigned long long *>(stamps + 2), (unsigned long long)__builtin_amdgcn_s_memrealtime());
 }
-
-// The device's constant-rate wall clock into slot i (a pass's timing marks,
-// which events cannot give inside a graph).
-__global__ void k_stamp(uint64_t *t, int i) { t[i] = __builtin_amdgcn_s_memrealtime(); }
 
 __global__ void k_zero_i32(int32_t *p, int n)
 {
@@ -1655,11 +1680,8 @@ static int enqueue_pass(hwt_surrogate *s, hwt_plan *tree, const hwt_options_f64 
                         double *out, hipStream_t st)
 {
     uint64_t *stamps = reinterpret_cast<uint64_t *>(s->fb_count + 8);
-    k_stamp<<<1, 1, 0, st>>>(stamps, 0);
-    k_zero_i32<<<1, 32, 0, st>>>(s->fb_count, 8);
+    k_begin_pass<<<1, 64, 0, st>>>(s->fb_count, stamps);
     if (o->n == 0) {
-        k_stamp<<<1, 1, 0, st>>>(stamps, 1);
-        k_stamp<<<1, 1, 0, st>>>(stamps, 2);
         SURR_HIP(hipGetLastError());
         return HWT_OK;
     }
@@ -1667,7 +1689,7 @@ static int enqueue_pass(hwt_surrogate *s, hwt_plan *tree, const hwt_options_f64 
     // split: out-of-box options to the fallback list, in-box ones to the
     // inference rows (running the tree on the out-of-box part beside the
     // inference was measured slower: both compete for the same CUs)
-    k_box<<<(o->n + BOX_CHUNK - 1) / BOX_CHUNK, 256, 0, st>>>(sopts(*o), s->fb_idx, s->fb_count, s->inf_rows,
+    k_box<<<(o->n + BOX_CHUNK - 1) / BOX_CHUNK, BOX_THREADS, 0, st>>>(sopts(*o), s->fb_idx, s->fb_count, s->inf_rows,
                                                             s->fb_count + 4);
     // the ensemble on the in-box rows; options it is unsure of join the list
     InferArgs g{};
@@ -1682,16 +1704,14 @@ static int enqueue_pass(hwt_surrogate *s, hwt_plan *tree, const hwt_options_f64 
     g.rows = s->inf_rows;
     g.row_count = s->fb_count + 4;
     k_infer<<<(o->n + INF_ROWS - 1) / INF_ROWS, 256, 0, st>>>(g);
-    k_stamp<<<1, 1, 0, st>>>(stamps, 1);
     SURR_HIP(hipGetLastError());
     // the whole list on the FP64 tree in one pass
-    k_fb_gather<<<blocks, 256, 0, st>>>(sopts(*o), s->fb_idx, s->fb_count, s->comp);
+    k_fb_gather<<<blocks, 256, 0, st>>>(sopts(*o), s->fb_idx, s->fb_count, s->comp, stamps);
     const hwt_options_f64 co{o->n,          s->comp.strike, s->comp.maturity, s->comp.length, s->comp.tu,
                              s->comp.steps, s->comp.a,      s->comp.sigma,    s->comp.type};
     const int rc = hwt_internal_plan_enqueue_counted(tree, &co, s->fb_count, y, s->fb_tmp, st);
     if (rc) return rc;
-    k_fb_scatter<<<blocks, 256, 0, st>>>(s->fb_idx, s->fb_count, s->fb_tmp, out);
-    k_stamp<<<1, 1, 0, st>>>(stamps, 2);
+    k_fb_scatter<<<blocks, 256, 0, st>>>(s->fb_idx, s->fb_count, s->fb_tmp, out, stamps);
     SURR_HIP(hipGetLastError());
     return HWT_OK;
 }
