@@ -4,14 +4,14 @@ Workload: the 60,000-option skewed batch (90% small trees: bond 1-5y at
 12 steps/yr, a in [0.1,0.2]; 10% large trees: bond 10-30y at 36 steps/yr,
 a in [0.01,0.05], widths up to 1,327 nodes, heights up to 1,080 steps),
 synthetic 120-knot yield curve, seeded inputs already resident in HBM.
-A step prices the whole batch: device-side constants and ordering plus the two
+A step prices the whole batch: device-side constants and ordering plus the
 pricing kernels, replayed from the plan's HIP graph or launched directly
 (HWT_FLAG_DIRECT), whichever the autotuner measured faster.
 
-Prints one JSON line.  `roofline` is for the dominant kernel (the wide-tree
-pricing kernel, timed alone with HIP events on its stream): FP64 vector FLOPs
-of the stencil (5 per node update: one multiply and two fused multiply-adds)
-against MI355X's 78.6 TFLOP/s FP64 peak.  `cpu_baseline` times the reference's
+Prints one JSON line.  `roofline` is for the dominant kernel (k_price_tri, timed
+with HIP events on its stream): the FP64 operations that the hardware counters
+saw it execute on this batch (2 per fused multiply-add; profiles/) against
+MI355X's 78.6 TFLOP/s FP64 peak.  `cpu_baseline` times the reference's
 own sequential pricer (built from its sources into oracle/_ref) on a bounded
 stratified sample on this host's cores.
 """
@@ -34,7 +34,6 @@ sys.path.insert(0, str(ROOT))
 METRIC = "options/sec on 1 MI355X: FP64 tree vs surrogate+fallback at max err 1e-3"
 FP64_PEAK_TFLOPS = 78.6
 HBM_PEAK_GBS = 8000.0
-FLOP_PER_NODE_UPDATE = 5
 
 
 def _cpu_model() -> str:
@@ -348,9 +347,8 @@ def main():
     # HIP events around the wide-tree kernel on the stream it runs on
     cfg_k = capi.config()
     C.memmove(C.byref(cfg_k), C.byref(tuned), C.sizeof(cfg_k))
-    # the wide-tree kernel on its own: serial arrangement whatever the tuner
-    # chose (fused, it would include the narrow trees; side by side, it would
-    # share the CUs with them)
+    # (in FP64 wide_ms spans every pricing kernel: k_price_wide<double>, which
+    # finds no task in this batch, and k_price_tri)
     cfg_k.flags = (cfg_k.flags & ~(capi.FLAG_FUSED | capi.FLAG_CONCURRENT)) | capi.FLAG_NO_GRAPH
     plan_k = capi.Plan(opts.N, y.N, cfg_k)
     wide, narrow, kern = [], [], []
@@ -363,29 +361,26 @@ def main():
             kern.append(s["kernel_ms"])
     plan_k.close()
     wide_ms = float(np.mean(wide))
-    wide_flop = FLOP_PER_NODE_UPDATE * s["wide_node_updates"]
-    dominant = "k_price_wide"
+    counted = {}
+    cfile = ROOT / "profiles" / "counters_pricing_skewed_60k.json"
+    if cfile.exists():
+        counted = json.loads(cfile.read_text())
+    wide_flop, dominant, traffic = counted.get("fp64_flop_per_launch"), "k_price_tri", counted.get("hbm_bytes_per_launch")
+    flop_model = ("FP64 operations of k_price_tri on this batch by the hardware counters "
+                  "(2 FMA + MUL + ADD instructions, 64 lanes each; profiles/counters_pricing_skewed_60k.json): "
+                  "two FMAs per node of the windows and groups, padding, set-up and sums included")
     if tuned.form == capi.FORM_LANE:  # the inspector chose form 1: one pricing kernel
-        wide_ms, wide_flop, dominant = float(np.mean(kern)), FLOP_PER_NODE_UPDATE * s["node_updates"], "k_price_lane"
-    achieved = wide_flop / (wide_ms * 1e-3) / 1e12
-    # what the kernel's stencil steps executed, counted by the kernel itself
-    # (padding slots included; 4K+1 operations per lane and step in the
-    # unit-diagonal form, 5K in the plain one)
-    exec_ops = s["wide_step_ops"] if dominant == "k_price_wide" else None
-    slots = s["wide_unit_slots"] + s["wide_plain_slots"]
+        wide_ms, wide_flop, dominant, traffic = float(np.mean(kern)), 4 * s["node_updates"], "k_price_lane", None
+        flop_model = "4 FP64 FLOP per node update (two FMAs) over the active tree region"
+    achieved = None if wide_flop is None else wide_flop / (wide_ms * 1e-3) / 1e12
 
-    # the drop-in one-shot call on host arrays (plan creation, H2D, pricing,
-    # D2H, plan destruction): the PCIe-inclusive rate, reported beside `value`
+    # the drop-in one-shot call on host arrays (H2D, pricing, D2H, from an idle
+    # workspace after the first): the PCIe-inclusive rate, reported beside `value`
     capi.price(opts, y)
     t0 = time.perf_counter()
     for _ in range(3):
         capi.price(opts, y)
     one_shot_s = (time.perf_counter() - t0) / 3
-
-    traffic = None
-    tfile = ROOT / "profiles" / "traffic_wide_kernel_skewed_60k.json"
-    if tfile.exists():
-        traffic = json.loads(tfile.read_text()).get("hbm_bytes_per_launch")
 
     line = {
         "metric": METRIC,
@@ -406,7 +401,7 @@ def main():
                         "and 6,000 large (width 267-1,327, height 360-1,080)",
             "options": opts.N,
             "precision": "fp64",
-            "pipeline": "device constants + LPT ordering + wide/narrow persistent pricing kernels, "
+            "pipeline": "device constants + LPT ordering + persistent pricing kernel, "
                         + ("launched directly" if tuned.flags & capi.FLAG_DIRECT else "one HIP graph"),
             "tuned": tuned.as_dict(),
         },
@@ -416,22 +411,11 @@ def main():
             "achieved": achieved,
             "peak": FP64_PEAK_TFLOPS,
             "unit": "TFLOP/s",
-            "frac": achieved / FP64_PEAK_TFLOPS,
+            "frac": None if achieved is None else achieved / FP64_PEAK_TFLOPS,
             "traffic": traffic,
             "kernel_ms": wide_ms,
             "flop_per_launch": wide_flop,
-            "flop_model": "5 FP64 FLOP per stencil node update (mul + 2 fma), node updates counted over "
-                          "the active tree region",
-            "executed": None if exec_ops is None else {
-                "flop_per_launch": exec_ops,
-                "achieved": exec_ops / (wide_ms * 1e-3) / 1e12,
-                "frac": exec_ops / (wide_ms * 1e-3) / 1e12 / FP64_PEAK_TFLOPS,
-                "unit_form_slots": s["wide_unit_slots"],
-                "plain_form_slots": s["wide_plain_slots"],
-                "slots_per_counted_update": slots / s["wide_node_updates"],
-                "note": "FP64 operations the kernel's stencil steps executed, counted by the kernel (window "
-                        "padding included): 4K+1 per lane and step in the unit-diagonal form, 5K in the plain form",
-            },
+            "flop_model": flop_model,
         },
         "detail": {
             "node_updates": st["node_updates"],
@@ -440,8 +424,8 @@ def main():
             "narrow_kernel_ms": float(np.mean(narrow)),
             "pricing_kernels_ms": float(np.mean(kern)),
             "one_shot_host_buffers": {"options_per_s": opts.N / one_shot_s, "ms": one_shot_s * 1e3,
-                                      "note": "hwt_price_f64 on host arrays: plan creation, H2D copies, "
-                                              "pricing, D2H copy and plan destruction (wall clock)"},
+                                      "note": "hwt_price_f64 on host arrays: H2D copy, pricing and D2H copy "
+                                              "from an idle workspace (wall clock)"},
             "total_ms_per_step": ms_per_step,
             "autotune": {"fp64": tune_rep, "mixed": tune_rep_mixed, "mixed_config": tuned_mixed.as_dict()},
             "mixed_precision": {

@@ -34,7 +34,7 @@ struct DevYield {
     const int32_t *day;
 };
 
-// Task classes, in task-list order:
+// Task classes of mixed mode and form 1, in task-list order:
 //   wide  (w > 64*KSMALL)           k_price_wide, one option per wave, LPT queue
 //   mid   (ROW_MAX_WIDTH < w <= 64*KSMALL)  k_price_narrow, one option per wave
 //   row   (w <= ROW_MAX_WIDTH)      k_price_narrow, four options per wave

@@ -187,8 +187,10 @@ __device__ __forceinline__ void price_tasks(const OptConst *__restrict__ cst, co
     int t = uni((int)blockIdx.x) + first;
     while (t < last) {
         const int o = uni(order[t]);
-        const OptConst c = cst[o];
+        OptConst c = cst[o];
         const double *eo = edge ? edge + (size_t)o * EDGE_TAB : nullptr;
+        // mixed mode's set-up leaves this to the few trees that FP64 prices again
+        if (sizeof(T) == sizeof(double) && edge) c.sigmas = window_sigmas(c);
         double p;
         if (NARROW) {
             const int K = (uni(c.w) + WAVE - 1) / WAVE;

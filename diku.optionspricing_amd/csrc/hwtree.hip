@@ -1,6 +1,7 @@
 // hwtree.hip -- kernels and C ABI of the MI355X-native HW1F trinomial pricer.
 //
-// Pipeline of one execution (captured once into a HIP graph per plan):
+// Pipeline of one execution (captured once into a HIP graph per plan).  FP64
+// batches of up to 2,048 options are one kernel (k_price_small); others:
 //   k_setup    one thread per option: tree constants (the reference's
 //              OptionConstants), P(e dt) and P(n dt) from the yield curve, edge
 //              factors, work estimate, bucket and rank inside the bucket;
@@ -12,11 +13,14 @@
 //              pricing kernel clears the histogram, so no clearing
 //              kernel or memset node runs per execution (k_reset only runs for
 //              an empty batch, which has no k_setup)
-//   k_price_wide / k_price_narrow  persistent kernels, launched side by side:
-//              each wavefront pulls options off its part of the task list and
-//              prices them with the on-chip tree column (hwt_wave.h); trees up to
-//              128 nodes wide go to the narrow kernel, which needs far fewer
-//              registers and so runs at higher occupancy
+//   k_price_tri  FP64, persistent: wavefronts pull trees wide enough for one of
+//              their own, then groups of narrower ones, off the task list
+//              (hwt_tri.h); k_price_wide before it takes the trees that form
+//              cannot hold, usually none
+//   k_price_wide / k_price_narrow  mixed mode, persistent: trees up to 128 nodes
+//              wide go to the narrow kernel, which needs far fewer registers and
+//              so runs at higher occupancy (hwt_wave.h); k_price_redo after them
+//   k_price_lane  form 1 (hwt_lane.h)
 //
 // Pricing identity.  With Q_e the Arrow-Debreu prices at the exercise step e
 // and B_e the bond values there, the reference's backward induction gives
@@ -310,8 +314,10 @@ __device__ __forceinline__ void scan_offsets(const int32_t *__restrict__ hist, i
 // Per-wave LDS staging of k_setup's outputs.  A lane's record (its 288-byte
 // edge table, its 96-byte constants) is written to LDS and the wave copies the
 // records out as contiguous 1 KB rows instead of one 16-byte piece per lane
-// and store (25.7 -> 22.7 us on the 60k skewed batch).  The kernel is bound
-// by writing its 24.6 MB, not by its arithmetic.
+// and store (25.7 -> 22.7 us on the 60k skewed batch).  The kernel waits for
+// latencies (FP64 divides and exponentials, L2 atomics, one wave per SIMD at 60,000
+// options), more than for the 10.6 MB it writes (mixed 24.6): half the LDS and
+// registers, and so 3 to 4 blocks per CU, gained 1 us of 24.
 // FP64 plans write the ten-entry edge record instead of the table, 176 bytes
 // per option in place of 384.
 template <bool TRI>
@@ -372,7 +378,6 @@ __device__ __forceinline__ void copy_out(u32x4 *__restrict__ dst, const u32x4 *s
 template <bool TRI>
 __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, int32_t sort, int32_t maxWidth,
                                                        double unit_dmin, int32_t classes, int32_t spread,
-                                                       int32_t reprice,
                                                        OptConst *__restrict__ cst, double *__restrict__ edge,
                                                        int2 *__restrict__ slot, int32_t *__restrict__ hist,
                                                        int32_t *__restrict__ tally, double *__restrict__ out)
@@ -394,8 +399,19 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, in
         reinterpret_cast<unsigned long long *>(tally)[T_T0 / 2] = __builtin_amdgcn_s_memrealtime();
     // the option's fields are requested before the curve is staged, so the
     // two loads overlap
-    OptFields f{};
-    if (mine && !o.consts) f = option_fields(o, i);
+    double strike = 0.0, mat = 0.0, len = 0.0, a = 0.0, sigma = 0.0;
+    uint16_t tu = 0, ts = 0;
+    int8_t type = 0;
+    if (mine && !o.consts) {
+        strike = o.strike[i];
+        mat = o.maturity[i];
+        len = o.length[i];
+        tu = o.term_unit[i];
+        ts = o.term_steps[i];
+        a = o.a[i];
+        sigma = o.sigma[i];
+        type = o.type[i];
+    }
     for (int k = tid; k < Y::NB; k += SETUP_BLOCK) lh[k] = 0;
     if (tid < 3) lsum[tid] = 0ull;
     if (tid < 3) lbad[tid] = 0;
@@ -425,70 +441,92 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, in
     unsigned long long work = 0, seq_work = 0, wide_work = 0;
     bool invalid = false, unsupported = false, is_wide = false;
     int b = -1, r = 0;  // bucket, rank among the block's options in it
+    auto sort_key = [&](int64_t key) {
+        switch (sort) {
+        case 'W': case 'w': return (int64_t)c.w;
+        case 'H': case 'h': return (int64_t)c.n;
+        case '-': return (int64_t)0;
+        default: return key;
+        }
+    };
     if (mine) {
-        const int32_t st = option_record(o, i, f, maxWidth, c);
-        invalid = st == ST_INVALID;
-        unsupported = st == ST_UNSUPPORTED;
-        int64_t key = 0;
-        TriKind kind = TRI_DONE;
-        double value = NAN;
+        int32_t st;
+        if (o.consts) {
+            const hwt_option_constants_f64 k = o.consts[i];
+            tu = k.term_unit;
+            st = constants_given(k.t, k.dt, k.dr, k.X, k.M, k.jmax, k.n, k.width, k.term_unit, k.type, maxWidth,
+                                 o.consts_f32 != 0, c);
+        } else {
+            st = option_constants(strike, mat, len, tu, ts, a, sigma, type, maxWidth, c);
+        }
+        c.status = st;
         if constexpr (TRI) {
             TriEdge edges{};
-            kind = tri_setup(c, f.term_unit, yield, spread != 0, unit_dmin, edges, key, value);
+            int64_t key = 0;
+            double value = NAN;
+            const TriKind kind = tri_setup(c, tu, yield, spread != 0, unit_dmin, edges, key, value);
             __builtin_memcpy(tab, &edges, sizeof(edges));
-        } else if (st == ST_OK) {
-            value = 100.0;  // no steps: the face value (seq/Seq.hpp:119,171)
-            if (c.n > 0) {
-                const double tn = c.n * c.dt;
-                c.Pn = exp(-yield(tn, f.term_unit) * tn);
-                value = 100.0 * c.Pn;  // exercise outside the tree: the zero-coupon bond
-                if (c.e >= 0) {
-                    const double te = c.e * c.dt;
-                    c.Pe = exp(-yield(te, f.term_unit) * te);
-                    kind = TRI_GENERAL;
-                    TreeShape t{c.w, c.jmax, c.M, c.dr, c.dt, 0.0, 0.0};
-                    if (t.w >= 7) {
-                        // trees of 7 or more nodes (all but the tiniest) take their
-                        // edge discounts from four exponentials and the table from
-                        // its closed form
-                        const EdgeDiscounts ed = edge_discounts(t);
-                        edge_factors(t, ed);
-                        edge_table_closed(t, ed, tab);
-                        c.unit = unit_form_ok(t, tab, unit_dmin, ed.E0, ed.Ea) ? 1 : 0;
-                    } else {
-                        edge_factors(t);
-                        edge_table(t, tab);
-                        c.unit = unit_form_ok(t, tab, unit_dmin) ? 1 : 0;
-                    }
-                    c.rho = t.rho;
-                    c.rhop = t.rhop;
+            invalid = st == ST_INVALID;
+            unsupported = st == ST_UNSUPPORTED;
+            if (kind == TRI_DONE) out[i] = value;
+            else {
+                work = (unsigned long long)dual_node_updates(c.n, c.e, c.jmax);
+                seq_work = (unsigned long long)seq_node_updates(c.n, c.jmax);
+                is_wide = (c.w + WAVE - 1) / WAVE > KSMALL;
+                if (is_wide) wide_work = work;
+                key = sort_key(kind == TRI_WINDOWED ? key : (int64_t)work);
+                b = kind == TRI_GENERAL    ? B_TRI_BIG + log_bucket(key, 2, NBUCKET_TRI - B_TRI_BIG)
+                    : kind == TRI_WINDOWED ? B_TRI_WIN + log_bucket(key, 8, B_TRI_BIG - B_TRI_WIN)
+                                           : tri_bucket(tri_part(c.w, spread != 0), c.n);
+                r = atomicAdd(&lh[b], 1);
+            }
+        } else if (st == ST_INVALID) {
+            out[i] = NAN;
+            invalid = true;
+        } else if (st == ST_UNSUPPORTED) {
+            out[i] = NAN;
+            unsupported = true;
+        } else if (c.n == 0) {
+            out[i] = 100.0;  // no steps: the face value (seq/Seq.hpp:119,171)
+        } else {
+            const double tn = c.n * c.dt;
+            c.Pn = exp(-yield(tn, tu) * tn);
+            if (c.e < 0) {
+                out[i] = 100.0 * c.Pn;  // exercise outside the tree: the zero-coupon bond
+            } else {
+                const double te = c.e * c.dt;
+                c.Pe = exp(-yield(te, tu) * te);
+                TreeShape t{c.w, c.jmax, c.M, c.dr, c.dt, 0.0, 0.0};
+                if (t.w >= 7) {
+                    // trees of 7 or more nodes (all but the tiniest) take their
+                    // edge discounts from four exponentials and the table from
+                    // its closed form
+                    const EdgeDiscounts ed = edge_discounts(t);
+                    edge_factors(t, ed);
+                    edge_table_closed(t, ed, tab);
+                    c.unit = unit_form_ok(t, tab, unit_dmin, ed.E0, ed.Ea) ? 1 : 0;
+                } else {
+                    edge_factors(t);
+                    double gtab[EDGE_TAB];
+                    edge_table_general(t, gtab);
+#pragma unroll
+                    for (int k = 0; k < EDGE_TAB; ++k) tab[k] = gtab[k];
+                    c.unit = unit_form_ok(t, tab, unit_dmin) ? 1 : 0;
                 }
+                c.rho = t.rho;
+                c.rhop = t.rhop;
+                work = (unsigned long long)dual_node_updates(c.n, c.e, c.jmax);
+                seq_work = (unsigned long long)seq_node_updates(c.n, c.jmax);
+                const bool wide = (c.w + WAVE - 1) / WAVE > KSMALL;
+                is_wide = wide;
+                const int64_t key = sort_key((int64_t)work);
+                if (wide) b = B_WIDE + log_bucket(key, 8, NBUCKET - B_WIDE);
+                else if ((classes & CLASS_FLAT) && c.w <= FLAT_MAX_WIDTH) b = flat_bucket(c.w, c.n);
+                else if (c.w > ROW_MAX_WIDTH || !(classes & CLASS_ROWS)) b = B_MID + log_bucket(key, 4, B_WIDE - B_MID);
+                else b = row_bucket(c.w, c.n);
+                r = atomicAdd(&lh[b], 1);
+                if (wide) wide_work = work;
             }
-        }
-        if (kind == TRI_DONE) out[i] = value;
-        else {
-            work = (unsigned long long)dual_node_updates(c.n, c.e, c.jmax);
-            seq_work = (unsigned long long)seq_node_updates(c.n, c.jmax);
-            const bool wide = (c.w + WAVE - 1) / WAVE > KSMALL;
-            is_wide = wide;
-            if (!TRI && wide && reprice) c.sigmas = window_sigmas(c);  // should FP64 price it again
-            if (!TRI || kind != TRI_WINDOWED) key = (int64_t)work;
-            switch (sort) {
-            case 'W': case 'w': key = c.w; break;
-            case 'H': case 'h': key = c.n; break;
-            case '-': key = 0; break;
-            default: break;
-            }
-            if (TRI) {
-                if (kind == TRI_GENERAL) b = B_TRI_BIG + log_bucket(key, 2, NBUCKET_TRI - B_TRI_BIG);
-                else if (kind == TRI_WINDOWED) b = B_TRI_WIN + log_bucket(key, 8, B_TRI_BIG - B_TRI_WIN);
-                else b = tri_bucket(tri_part(c.w, spread != 0), c.n);
-            } else if (wide) b = B_WIDE + log_bucket(key, 8, NBUCKET - B_WIDE);
-            else if ((classes & CLASS_FLAT) && c.w <= FLAT_MAX_WIDTH) b = flat_bucket(c.w, c.n);
-            else if (c.w > ROW_MAX_WIDTH || !(classes & CLASS_ROWS)) b = B_MID + log_bucket(key, 4, B_WIDE - B_MID);
-            else b = row_bucket(c.w, c.n);
-            r = atomicAdd(&lh[b], 1);
-            if (wide) wide_work = work;
         }
     }
     // the block's tallies: one LDS atomic per wave and counter (every lane
@@ -893,7 +931,7 @@ static int launch_pipeline(hwt_plan *p, const DevOpts &o, const DevYield &y, dou
         }
         if (tri) {
             k_setup<true><<<blocks, SETUP_BLOCK, 0, s>>>(o, y, sort, max_width, unit_dmin, CLASS_ROWS,
-                                                         n <= TRI_SPREAD ? 1 : 0, 0, p->cst, p->edge, p->slot, p->hist,
+                                                         n <= TRI_SPREAD ? 1 : 0, p->cst, p->edge, p->slot, p->hist,
                                                          p->tally, out);
             k_order<true><<<blocks, SETUP_BLOCK, 0, s>>>(n, o.count, p->slot, p->hist, p->order, p->tally, asc,
                                                          CLASS_ROWS);
@@ -917,8 +955,7 @@ static int launch_pipeline(hwt_plan *p, const DevOpts &o, const DevYield &y, dou
             return HWT_OK;
         }
         k_setup<false><<<blocks, SETUP_BLOCK, 0, s>>>(o, y, sort, max_width, unit_dmin, classes, 0,
-                                                      p->cfg.precision == HWT_PREC_MIXED ? 1 : 0, p->cst, p->edge,
-                                                      p->slot, p->hist, p->tally, out);
+                                                      p->cst, p->edge, p->slot, p->hist, p->tally, out);
         k_order<false><<<blocks, SETUP_BLOCK, 0, s>>>(n, o.count, p->slot, p->hist, p->order, p->tally, asc, classes);
         if (time_kernel) HWT_HIP(hipEventRecord(p->evk0, s));
         if (p->cfg.form == HWT_FORM_LANE) {

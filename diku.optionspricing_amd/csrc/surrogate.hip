@@ -10,16 +10,14 @@
 // Matrix-core layout (v_mfma_f32_32x32x16_bf16, one wavefront of 64 lanes):
 // lane l holds A[l%32][8(l/32) .. 8(l/32)+7] and B[8(l/32) .. +7][l%32]; the
 // 16 accumulators of lane l are D[8(v/4) + 4(l/32) + v%4][l%32], v = 0..15.
-// Every GEMM here is C = A B^T with both operands stored K-contiguous, so each
-// lane's operand is one 16-byte load.
+// Every GEMM here is C = A B^T; operands in memory are kept in the order in which
+// the lanes read them (weight_at, frag_unit), so a wave's operand is one contiguous
+// kilobyte.
 //
-// Buffers per member (batch rows b, neurons n, inputs k):
-//   z_l     FP32 [b][n]   pre-activations (for SiLU')
-//   a_l     BF16 [b][n] and a_l^T [n][b]   (operands of the next forward
-//                          GEMM and of this layer's weight-gradient GEMM)
-//   dz_l    BF16 [b][n] and dz_l^T [n][b]  (operands of the input-gradient
-//                          and weight-gradient GEMMs)
-//   W_l     BF16 [n][k] and W_l^T [k][n], refreshed by Adam from FP32 masters
+// Training buffers per member (batch rows b, neurons n, inputs k):
+//   a_l^T, dz_l^T  BF16 [n][b]  (operands of the weight-gradient GEMMs)
+//   dz_1           FP32 [b][n]
+//   W_l            BF16 [n][k] and W_l^T [k][n], refreshed by Adam from FP32 masters
 #include "hwt_math.h"
 #include "hwt_internal.h"
 #include "../../include/hwtsurr.h"
