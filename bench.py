@@ -124,8 +124,8 @@ def reference_sets_leg(pkg, capi, args):
         out[name] = {"ms": ms, "options_per_s": opts.N / (ms * 1e-3), "node_updates": st["node_updates"],
                      "seq_node_updates": st["seq_node_updates"], "tuned_form": cfg.form, "tuned_flags": cfg.flags}
         # form 1 (one lane per option, tree columns in HBM) on the same batch,
-        # pricing kernel alone: 16 B of column traffic per node update (the
-        # next value read, the new value written)
+        # pricing kernel alone: 16 B of column traffic per node and sweep (the
+        # old value read, the new one written), eight steps to a sweep
         plan = capi.Plan(opts.N, yref.N, capi.config(form=capi.FORM_LANE, flags=capi.FLAG_NO_GRAPH))
         plan.execute(dev)
         s1 = plan.sync()
@@ -136,7 +136,7 @@ def reference_sets_leg(pkg, capi, args):
         plan.close()
         if kms:
             km = float(np.median(kms))
-            gbs = 16.0 * s1["node_updates"] / (km * 1e-3) / 1e9
+            gbs = 16.0 / 8 * s1["node_updates"] / (km * 1e-3) / 1e9
             out[name]["form1"] = {"kernel_ms": km, "options_per_s": opts.N / (km * 1e-3),
                                   "column_gb_per_s": gbs, "hbm_frac": gbs / HBM_PEAK_GBS}
         else:
@@ -273,7 +273,7 @@ def main():
         km = float(np.mean(ks))
         print(json.dumps({"profile_lane": args.profile_lane, "options": opts.N, "kernel_ms_mean": km,
                           "node_updates": st["node_updates"],
-                          "column_gb_per_s": 16.0 * st["node_updates"] / (km * 1e-3) / 1e9}), flush=True)
+                          "column_gb_per_s": 16.0 / 8 * st["node_updates"] / (km * 1e-3) / 1e9}), flush=True)
         return
     if args.profile_surrogate:
         S = pkg.surrogate
