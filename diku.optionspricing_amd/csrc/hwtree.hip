@@ -1565,11 +1565,15 @@ struct OneShot {
 };
 
 std::mutex g_idle_mu;
-// most recently used last; never destroyed, since the HIP runtime may be gone first
-std::vector<OneShot *> &idle_workspaces()
+OneShot *g_idle[OneShot::IDLE];  // most recently used last; not freed at exit, when the HIP runtime may be gone
+size_t g_nidle = 0;
+
+// Takes entry i out (with g_idle_mu held).
+OneShot *take_idle(size_t i)
 {
-    static auto *v = new std::vector<OneShot *>();
-    return *v;
+    OneShot *s = g_idle[i];
+    for (--g_nidle; i < g_nidle; ++i) g_idle[i] = g_idle[i + 1];
+    return s;
 }
 
 int32_t round_up_pow2(int32_t v, int32_t least)
@@ -1588,16 +1592,13 @@ int one_shot_acquire(const hwt_config &c, int32_t n, int32_t ny, OneShot *&out)
     HWT_HIP(hipGetDevice(&dev));
     {
         std::lock_guard<std::mutex> lk(g_idle_mu);
-        auto &v = idle_workspaces();
-        size_t best = v.size();
-        for (size_t i = 0; i < v.size(); ++i)
-            if (v[i]->device == dev && v[i]->cap >= n && v[i]->ycap >= ny && std::memcmp(&v[i]->cfg, &c, sizeof(c)) == 0 &&
-                (best == v.size() || v[i]->cap < v[best]->cap))
+        size_t best = g_nidle;
+        for (size_t i = 0; i < g_nidle; ++i)
+            if (g_idle[i]->device == dev && g_idle[i]->cap >= n && g_idle[i]->ycap >= ny &&
+                std::memcmp(&g_idle[i]->cfg, &c, sizeof(c)) == 0 &&
+                (best == g_nidle || g_idle[i]->cap < g_idle[best]->cap))
                 best = i;
-        if (best < v.size()) {
-            out = v[best];
-            v.erase(v.begin() + (std::ptrdiff_t)best);
-        }
+        if (best < g_nidle) out = take_idle(best);
     }
     // a device reset since the last call has taken the workspace with it
     if (out && hipStreamQuery(out->plan->stream) != hipSuccess) {
@@ -1632,27 +1633,20 @@ int one_shot_acquire(const hwt_config &c, int32_t n, int32_t ny, OneShot *&out)
 
 void one_shot_release(OneShot *s)
 {
-    std::vector<OneShot *> out;
-    try {
+    OneShot *out[OneShot::IDLE + 1];
+    size_t nout = 0;
+    {
         std::lock_guard<std::mutex> lk(g_idle_mu);
-        auto &v = idle_workspaces();
-        v.reserve(OneShot::IDLE + 1);
-        out.reserve(v.size() + 1);
         size_t held = s->held();
-        for (OneShot *w : v) held += w->held();
-        while (!v.empty() && (v.size() >= OneShot::IDLE || held > OneShot::IDLE_BYTES)) {
-            out.push_back(v.front());
-            held -= v.front()->held();
-            v.erase(v.begin());
+        for (size_t i = 0; i < g_nidle; ++i) held += g_idle[i]->held();
+        while (g_nidle > 0 && (g_nidle >= OneShot::IDLE || held > OneShot::IDLE_BYTES)) {
+            held -= g_idle[0]->held();
+            out[nout++] = take_idle(0);
         }
-        if (held > OneShot::IDLE_BYTES) out.push_back(s);
-        else v.push_back(s);
-    } catch (const std::bad_alloc &) {
-        out.clear();
-        delete s;
-        return;
+        if (held > OneShot::IDLE_BYTES) out[nout++] = s;
+        else g_idle[g_nidle++] = s;
     }
-    for (OneShot *w : out) delete w;
+    for (size_t i = 0; i < nout; ++i) delete out[i];
 }
 
 bool one_shot_fits(const hwt_config &c, int32_t n, int32_t ny)
@@ -1732,12 +1726,13 @@ extern "C" {
 
 void hwt_trim(void)
 {
-    std::vector<OneShot *> out;
+    OneShot *out[OneShot::IDLE];
+    size_t nout = 0;
     {
         std::lock_guard<std::mutex> lk(g_idle_mu);
-        out.swap(idle_workspaces());
+        while (g_nidle > 0) out[nout++] = take_idle(g_nidle - 1);
     }
-    for (OneShot *w : out) delete w;
+    for (size_t i = 0; i < nout; ++i) delete out[i];
 }
 
 int hwt_batch_create(hwt_batch **out, const hwt_options_f64 *opts, const hwt_yield_f64 *yield)
