@@ -395,6 +395,8 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_setup(DevOpts o, DevYield y, in
     const int i = tid + blockIdx.x * SETUP_BLOCK;
     const int nopt = o.count ? min(*o.count, o.n) : o.n;
     const bool mine = i < nopt;
+    // a launch for a count that the device knows is sized for the most there can be
+    if (blockIdx.x > 0 && (int)blockIdx.x * SETUP_BLOCK >= nopt) return;
     if (i == 0)
         reinterpret_cast<unsigned long long *>(tally)[T_T0 / 2] = __builtin_amdgcn_s_memrealtime();
     // the option's fields are requested before the curve is staged, so the
@@ -620,6 +622,7 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_order(int32_t n, const int32_t 
     const int tid = threadIdx.x;
     const int i = tid + blockIdx.x * SETUP_BLOCK;
     if (count) n = min(*count, n);
+    if (blockIdx.x > 0 && (int)blockIdx.x * SETUP_BLOCK >= n) return;
     const int2 s = (i < n) ? slot[i] : make_int2(-1, 0);  // requested first, so it arrives during the scan
     scan_offsets<TRI>(hist, soffs, order, tally, asc, classes, blockIdx.x == 0);
     if (s.x >= 0) order[soffs[s.x] + s.y] = i;
