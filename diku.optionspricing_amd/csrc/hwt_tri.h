@@ -29,6 +29,7 @@
 
 #include "hwt_flat.h"
 #include "hwt_pipeline.h"
+#include "hwt_scale.h"
 
 namespace hwt {
 
@@ -251,32 +252,29 @@ __device__ __forceinline__ void tri_step(const double (&src)[K], double (&dst)[K
     }
 }
 
-// nsteps steps in place.  A state grows about sixfold per step; every 64 steps
-// (counted in `run` over the calls) it is scaled by 2^-165 = 6^-63.8.
+// nsteps steps in place, scaled on the way (hwt_scale.h).
 template <int L, int K>
 __device__ __forceinline__ void tri_steps(double (&z)[K], const double (&m)[K], const double (&r)[K], double in_lane0,
-                                          int nsteps, int &run)
+                                          int nsteps, SixfoldScale &scale)
 {
     double t[K];
-    while (nsteps > 0) {
-        const int c = min(nsteps, 64);
-        for (int it = 0; it + 1 < c; it += 2) {
-            tri_step<L, K>(z, t, m, r, in_lane0);
-            tri_step<L, K>(t, z, m, r, in_lane0);
-        }
-        if (c & 1) {
-            tri_step<L, K>(z, t, m, r, in_lane0);
+    scaled_steps(
+        scale, nsteps,
+        [&](int c) {
+            for (int it = 0; it + 1 < c; it += 2) {
+                tri_step<L, K>(z, t, m, r, in_lane0);
+                tri_step<L, K>(t, z, m, r, in_lane0);
+            }
+            if (c & 1) {
+                tri_step<L, K>(z, t, m, r, in_lane0);
 #pragma unroll
-            for (int s = 0; s < K; ++s) z[s] = t[s];
-        }
-        nsteps -= c;
-        run += c;
-        if (run >= 64) {
-            run = 0;
+                for (int s = 0; s < K; ++s) z[s] = t[s];
+            }
+        },
+        [&](double f) {
 #pragma unroll
-            for (int s = 0; s < K; ++s) z[s] *= 0x1p-165;
-        }
-    }
+            for (int s = 0; s < K; ++s) z[s] *= f;
+        });
 }
 
 // Price from the two states at the exercise step, u (forward) and v
@@ -383,7 +381,8 @@ __device__ __forceinline__ double price_tri_group(const OptConst *__restrict__ c
     const double in_lane0 = l == 0 ? 0.0 : 1.0;
     const int N = -wave_min_i32(-n);
     const int start = N - n, swap = start + e;
-    int i = 0, run = 0;
+    int i = 0;
+    SixfoldScale scale;
     for (;;) {
         if (i == start) {
 #pragma unroll
@@ -399,7 +398,7 @@ __device__ __forceinline__ double price_tri_group(const OptConst *__restrict__ c
         }
         if (i >= N) break;
         const int next = wave_min_i32(start > i ? start : (swap > i ? swap : N));
-        tri_steps<L, K>(z, m, r, in_lane0, next - i, run);
+        tri_steps<L, K>(z, m, r, in_lane0, next - i, scale);
         i = next;
     }
     double u[K];
@@ -428,7 +427,8 @@ struct TriPhase {
 // held in registers through the steps.
 template <int K>
 __device__ __forceinline__ double tri_phase(const OptConst *__restrict__ cst, const TriEdge *__restrict__ edge, int o,
-                                            const TriPhase &p, int lane, lds_f64 *lds, double *park, int &run)
+                                            const TriPhase &p, int lane, lds_f64 *lds, double *park,
+                                            SixfoldScale &scale)
 {
     asm volatile("" : "+s"(o), "+v"(lane));
     const OptConst c = cst[o];
@@ -449,7 +449,7 @@ __device__ __forceinline__ double tri_phase(const OptConst *__restrict__ cst, co
         double none[K];
         tri_coefs<WAVE, K, false>(t, ed, edges, p.base, lane, lane, m, r, none, lds);
     }
-    tri_steps<WAVE, K>(z, m, r, 1.0, p.steps, run);
+    tri_steps<WAVE, K>(z, m, r, 1.0, p.steps, scale);
     if (!p.last) {
 #pragma unroll
         for (int s = 0; s < K; ++s) lds[lane * K + s] = (k0 + s < t.w) ? z[s] : 0.0;
@@ -483,7 +483,7 @@ __device__ __forceinline__ double price_tri_window(const OptConst *__restrict__ 
     const Reach reach = make_reach(c.sigmas, t.M, t.dr, t.dt, n, t.jmax);
     TriPhase p{};
     double price = 0.0;
-    int run = 0;
+    SixfoldScale scale;
     for (int back = 0; back < 2; ++back) {
         int at = back ? n : 0, l0 = 0, u0 = 0;
         if (back) {
@@ -501,9 +501,9 @@ __device__ __forceinline__ double price_tri_window(const OptConst *__restrict__ 
             p.steps = abs(f.end - at);
             p.last = f.end == e;
             switch (p.K) {
-#define HWT_W(KK) case KK: price = tri_phase<KK>(cst, edge, o, p, lane, lds, park, run); break;
+#define HWT_W(KK) case KK: price = tri_phase<KK>(cst, edge, o, p, lane, lds, park, scale); break;
                 HWT_W(2) HWT_W(3) HWT_W(4) HWT_W(5) HWT_W(6) HWT_W(7) HWT_W(8) HWT_W(9) HWT_W(10)
-            default: price = tri_phase<TRI_MAXK>(cst, edge, o, p, lane, lds, park, run); break;
+            default: price = tri_phase<TRI_MAXK>(cst, edge, o, p, lane, lds, park, scale); break;
 #undef HWT_W
             }
             p.in_base = p.base;
