@@ -19,6 +19,7 @@
 // and the inner chunks free of branches, 150 at eight steps.
 #pragma once
 
+#include "hwt_scale.h"
 #include "hwt_tri.h"
 
 namespace hwt {
@@ -135,17 +136,16 @@ __device__ __forceinline__ double lane_price(const OptConst &c, const double *et
 // ------------------------------------------------- the tridiagonal form
 // S steps of u'_k = u_{k-1} + m_k u_k + r_k u_{k+1} in one sweep over nodes
 // [lo, hi], in place; the old state is nonzero on [olo, ohi] inside it and the
-// result scaled by 6^-S, nearly (2^-2.5 S: the state grows about sixfold a step).
+// result scaled by `down` (hwt_scale.h).
 // Level l of the sweep trails the one before by a node: with u_0[k] just read,
 // level l makes node k - l.  Nodes are read a chunk at a time, a chunk ahead of use.
 constexpr int LANE_CHUNK = 8;
 
 template <int S>
 __device__ __forceinline__ void lane_tri_sweep(const TreeShape &t, const TriEdge &e, LaneColumn col, int lo, int hi,
-                                               int olo, int ohi)
+                                               int olo, int ohi, double down)
 {
     static_assert(S == 1 || S == 2 || S == 4 || S == 8, "levels");
-    constexpr double down = S == 1 ? 0x1p-2 : S == 2 ? 0x1p-5 : S == 4 ? 0x1p-10 : 0x1p-20;
     double a[S], b[S], m[S], r[S];  // level l's last two nodes; the coefficients level l + 1 uses
 #pragma unroll
     for (int l = 0; l < S; ++l) a[l] = b[l] = m[l] = r[l] = 0.0;
@@ -241,14 +241,16 @@ __device__ __forceinline__ void lane_tri_steps(const TreeShape &t, const TriEdge
                                                bool grows, Range &&range)
 {
     const int J = t.jmax;
+    SixfoldScale scale;
     for (int i = 0; i < steps;) {
         const int left = steps - i, c = left >= LEVELS ? LEVELS : left >= 4 ? 4 : left >= 2 ? 2 : 1;
         const int from = range(i), to = range(i + c), h = grows ? to : from;
+        const double down = pow2_down(scale.bits(c));
         switch (c) {
-        case 8: lane_tri_sweep<LEVELS>(t, e, col, J - h, J + h, J - from, J + from); break;
-        case 4: lane_tri_sweep<4>(t, e, col, J - h, J + h, J - from, J + from); break;
-        case 2: lane_tri_sweep<2>(t, e, col, J - h, J + h, J - from, J + from); break;
-        default: lane_tri_sweep<1>(t, e, col, J - h, J + h, J - from, J + from); break;
+        case 8: lane_tri_sweep<LEVELS>(t, e, col, J - h, J + h, J - from, J + from, down); break;
+        case 4: lane_tri_sweep<4>(t, e, col, J - h, J + h, J - from, J + from, down); break;
+        case 2: lane_tri_sweep<2>(t, e, col, J - h, J + h, J - from, J + from, down); break;
+        default: lane_tri_sweep<1>(t, e, col, J - h, J + h, J - from, J + from, down); break;
         }
         i += c;
     }

@@ -83,3 +83,14 @@ def test_hundreds_of_thousands_of_steps(pkg, oracle, kernel):
     else:
         got = pkg.capi.price(pkg.Options.concat([_filler(pkg, 1100), opts, _filler(pkg, 1100)]), y)
         _check(oracle, opts, y, got[1100:1124])
+
+
+@pytest.mark.parametrize("block", [0, 512])
+@pytest.mark.parametrize("widths, steps, years", [(np.arange(7, 272, 2), 365, (25, 60)), ([25], 7300, (22, 30))])
+def test_tall_columns(pkg, oracle, block, widths, steps, years):
+    """Form 1, several steps to a sweep: above and below the 12,050 steps at which scaling
+    by 2^-20 for eight of them would lose the range."""
+    y = pkg.datasets.synthetic_yield()
+    opts = _options(pkg, 47, 64, widths, steps, years)
+    cfg = pkg.capi.config(form=pkg.capi.FORM_LANE, block_size=block)
+    _check(oracle, opts, y, pkg.capi.price(opts, y, cfg))
