@@ -235,19 +235,19 @@ __device__ __forceinline__ void lane_tri_sweep(const TreeShape &t, const TriEdge
 }
 
 // `steps` steps over a region that `range(i)` gives after i of them, up to
-// LEVELS (4 or 8) to a sweep.
-template <int LEVELS, class Range>
+// eight to a sweep.
+template <class Range>
 __device__ __forceinline__ void lane_tri_steps(const TreeShape &t, const TriEdge &e, LaneColumn col, int steps,
                                                bool grows, Range &&range)
 {
     const int J = t.jmax;
     SixfoldScale scale;
     for (int i = 0; i < steps;) {
-        const int left = steps - i, c = left >= LEVELS ? LEVELS : left >= 4 ? 4 : left >= 2 ? 2 : 1;
+        const int left = steps - i, c = left >= 8 ? 8 : left >= 4 ? 4 : left >= 2 ? 2 : 1;
         const int from = range(i), to = range(i + c), h = grows ? to : from;
         const double down = pow2_down(scale.bits(c));
         switch (c) {
-        case 8: lane_tri_sweep<LEVELS>(t, e, col, J - h, J + h, J - from, J + from, down); break;
+        case 8: lane_tri_sweep<8>(t, e, col, J - h, J + h, J - from, J + from, down); break;
         case 4: lane_tri_sweep<4>(t, e, col, J - h, J + h, J - from, J + from, down); break;
         case 2: lane_tri_sweep<2>(t, e, col, J - h, J + h, J - from, J + from, down); break;
         default: lane_tri_sweep<1>(t, e, col, J - h, J + h, J - from, J + from, down); break;
@@ -281,13 +281,12 @@ __device__ __forceinline__ void lane_tri_scales(const TreeShape &t, const TriEdg
     }
 }
 
-template <int LEVELS>
 __device__ __forceinline__ double lane_price_tri(const OptConst &c, const TreeShape &t, const TriEdge &ed, LaneColumn Y,
                                                  LaneColumn B)
 {
     const int J = c.jmax, n = c.n, e = c.e, top = c.w - 1;
     Y[J] = 1.0;
-    lane_tri_steps<LEVELS>(t, ed, Y, e, true, [&](int i) { return min(i, J); });
+    lane_tri_steps(t, ed, Y, e, true, [&](int i) { return min(i, J); });
     const int ep = min(e, J);
     auto need = [&](int s) { return min(J, ep + (s - e)); };
     lane_tri_scales(t, ed, need(n), [&](int k, double, double d2) {
@@ -296,7 +295,7 @@ __device__ __forceinline__ double lane_price_tri(const OptConst &c, const TreeSh
         if (k == top) v = (v - t.rhop) / ed.d2_t;
         B[k] = v / d2;
     });
-    lane_tri_steps<LEVELS>(t, ed, B, n - e, false, [&](int i) { return need(n - i); });
+    lane_tri_steps(t, ed, B, n - e, false, [&](int i) { return need(n - i); });
     // both states scaled back, node 0's d1 and node w-1's d2 by their factors
     lane_tri_scales(t, ed, ep, [&](int k, double d1, double d2) {
         if (k == 0) d1 *= ed.d1_0;

@@ -713,12 +713,16 @@ __global__ __launch_bounds__(256) void k_count_steps(const OptConst *__restrict_
 }
 
 // Form 1: one lane per option over every scheduled task (tasks ordered by
-// decreasing work, so the lanes of a wave carry similar trees).  BLOCK: the most
-// lanes per workgroup (1,024 leaves 128 VGPRs, too few for eight steps a sweep).
-template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_price_lane(const OptConst *__restrict__ cst, const double *__restrict__ edge,
-                             const int32_t *__restrict__ order, int32_t *__restrict__ tally,
-                             double *__restrict__ out, double *__restrict__ cols, int32_t colw)
+// decreasing work, so the lanes of a wave carry similar trees).  At most LANE_THREADS
+// lanes per workgroup: 1,024 leave 128 VGPRs, too few for a sweep of even one step
+// (290 spilled at four; 2,000 uniform options 2,270 us a call, 210 in workgroups of
+// 256).  What a lane does does not depend on its workgroup.
+constexpr int LANE_THREADS = 256;
+__global__ __launch_bounds__(LANE_THREADS) void k_price_lane(const OptConst *__restrict__ cst,
+                                                             const double *__restrict__ edge,
+                                                             const int32_t *__restrict__ order,
+                                                             int32_t *__restrict__ tally, double *__restrict__ out,
+                                                             double *__restrict__ cols, int32_t colw)
 {
     clear_bucket_counts(tally);
     const int gid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -729,7 +733,7 @@ __global__ __launch_bounds__(BLOCK) void k_price_lane(const OptConst *__restrict
         const LaneColumn Y{base}, B{base + (size_t)colw * WAVE};
         const TreeShape t{c.w, c.jmax, c.M, c.dr, c.dt, c.rho, c.rhop};
         const TriEdge ed = tri_edge(t, edge_discounts(t));
-        out[o] = tri_ok(t, ed, c.n, c.jmax, 200.0f) ? lane_price_tri<BLOCK <= 256 ? 8 : 4>(c, t, ed, Y, B)
+        out[o] = tri_ok(t, ed, c.n, c.jmax, 200.0f) ? lane_price_tri(c, t, ed, Y, B)
                                                     : lane_price(c, edge + (size_t)o * EDGE_TAB, Y, B);
     }
     stamp_wave_end(tally);
@@ -962,13 +966,9 @@ static int launch_pipeline(hwt_plan *p, const DevOpts &o, const DevYield &y, dou
         k_order<false><<<blocks, SETUP_BLOCK, 0, s>>>(n, o.count, p->slot, p->hist, p->order, p->tally, asc, classes);
         if (time_kernel) HWT_HIP(hipEventRecord(p->evk0, s));
         if (p->cfg.form == HWT_FORM_LANE) {
-            const int lb = p->lane_block;
-            if (lb <= 256)
-                k_price_lane<256><<<(n + lb - 1) / lb, lb, 0, s>>>(p->cst, p->edge, p->order, p->tally, out, p->cols,
-                                                                   p->lane_width);
-            else
-                k_price_lane<1024><<<(n + lb - 1) / lb, lb, 0, s>>>(p->cst, p->edge, p->order, p->tally, out, p->cols,
-                                                                    p->lane_width);
+            const int lb = std::min(p->lane_block, LANE_THREADS);
+            k_price_lane<<<(n + lb - 1) / lb, lb, 0, s>>>(p->cst, p->edge, p->order, p->tally, out, p->cols,
+                                                          p->lane_width);
             if (time_kernel) HWT_HIP(hipEventRecord(p->evk1, s));
             HWT_HIP(hipGetLastError());
             return HWT_OK;

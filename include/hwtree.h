@@ -84,8 +84,9 @@ typedef struct {
 typedef struct {
     int32_t form;        /* HWT_FORM_*                                  (0 = auto) */
     int32_t precision;   /* HWT_PREC_*                                  (0 = FP64) */
-    int32_t block_size;  /* form 1: lanes per workgroup (64..1024); <= 0 picks the
-                            default.  Form 2 runs one wavefront per workgroup. */
+    int32_t block_size;  /* form 1: lanes per workgroup (64..1024, above 256 runs as
+                            256); <= 0 picks the default.  Form 2 runs one wavefront
+                            per workgroup. */
     int32_t sort;        /* HWT_SORT_*: processing order of the wide and mid-width
                             trees (0 = work-descending) */
     int32_t device;      /* HIP device ordinal for hwt_price_f64; < 0 = current */
