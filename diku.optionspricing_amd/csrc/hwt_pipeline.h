@@ -155,7 +155,7 @@ enum Tally {
     T_TBIG = T_HOST,
     T_TWIN = T_HOST + 1,
     T_TNGROUP = T_HOST + 2,
-    T_SMALL = T_HOST + 3,   // options of the last execution if k_price_small ran it, else 0
+    T_SMALL = T_HOST + 3,   // options of the last execution if k_price_small ran it and no sync has counted it, else 0
     T_TSTART = T_HOST + 8,  // TRI_PARTS entries
     T_TGROUP = T_HOST + 56, // TRI_PARTS entries
     A_NWIDE = T_HOST + 104,  // accumulated by k_setup: wide trees

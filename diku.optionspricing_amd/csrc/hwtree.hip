@@ -629,11 +629,12 @@ __global__ __launch_bounds__(SETUP_BLOCK) void k_order(int32_t n, const int32_t 
 }
 
 // The counts of an execution by k_price_small (T_SMALL), from its constants: one
-// block, at sync time (k_setup and k_order count a larger batch as they go).
+// block, at the first sync after it (k_setup and k_order count a larger batch as
+// they go).
 __global__ __launch_bounds__(256) void k_small_tally(const OptConst *__restrict__ cst, int32_t *__restrict__ tally)
 {
     const int n = tally[T_SMALL];
-    if (n == 0) return;  // the last execution was another batch's
+    if (n == 0) return;  // counted already, or the last execution was a larger batch's
     __shared__ unsigned long long sums[3];  // work, seq work, wide work
     __shared__ int32_t counts[4];           // invalid, unsupported, tasks, wide
     const int t = threadIdx.x;
@@ -667,6 +668,7 @@ __global__ __launch_bounds__(256) void k_small_tally(const OptConst *__restrict_
         tally[T_NLARGE] = counts[3];
         tally[T_NPAD] = tally[T_NREDO] = 0;
         for (int k = T_XFLOP; k < T_XPLAIN + 2; ++k) tally[k] = 0;
+        tally[T_SMALL] = 0;  // a further sync finds the counts as they are
     }
 }
 
