@@ -2141,8 +2141,14 @@ namespace {
 std::mutex g_tune_mu;
 std::map<std::string, hwt_config> g_tune_cache;
 bool g_tune_loaded = false;
-// the flags the tuner chooses (the caller's others are kept as given)
-constexpr int TUNED_FLAGS = HWT_FLAG_NO_ROWS | HWT_FLAG_CONCURRENT | HWT_FLAG_FUSED | HWT_FLAG_NO_FLAT | HWT_FLAG_DIRECT;
+// the flags the tuner chooses (the caller's others are kept as given): the launch
+// mode, and between mixed mode's kernel arrangements, which mean nothing in FP64
+int tuned_flags(int precision)
+{
+    return precision == HWT_PREC_MIXED
+               ? HWT_FLAG_NO_ROWS | HWT_FLAG_NO_FLAT | HWT_FLAG_CONCURRENT | HWT_FLAG_FUSED | HWT_FLAG_DIRECT
+               : HWT_FLAG_DIRECT;
+}
 
 int ilog2(int64_t v)
 {
@@ -2180,7 +2186,7 @@ void tune_store_file(const std::string &key, const hwt_config &c)
     const char *path = getenv("HWT_TUNE_CACHE");
     if (!path || !*path) return;
     std::ofstream f(path, std::ios::app);
-    const int kept = c.flags & TUNED_FLAGS;
+    const int kept = c.flags & tuned_flags(c.precision);
     f << key << ' ' << c.form << ' ' << c.sort << ' ' << kept << ' '
       << c.wide_per_cu << ' ' << c.narrow_per_cu << '\n';
 }
@@ -2280,7 +2286,8 @@ extern "C" int hwt_autotune(const hwt_options_f64 *dev_opts, const hwt_yield_f64
             hwt_config c = base;
             c.form = it->second.form;
             c.sort = it->second.sort;
-            c.flags = (base.flags & ~TUNED_FLAGS) | (it->second.flags & TUNED_FLAGS);
+            const int tuned = tuned_flags(base.precision);
+            c.flags = (base.flags & ~tuned) | (it->second.flags & tuned);
             c.wide_per_cu = it->second.wide_per_cu;
             c.narrow_per_cu = it->second.narrow_per_cu;
             *cfg = c;
@@ -2317,6 +2324,7 @@ extern "C" int hwt_autotune(const hwt_options_f64 *dev_opts, const hwt_yield_f64
         if ((rc = consider(c))) return rc;
     }
     for (int bit : {HWT_FLAG_NO_ROWS, HWT_FLAG_NO_FLAT, HWT_FLAG_CONCURRENT, HWT_FLAG_FUSED, HWT_FLAG_DIRECT}) {
+        if (!(bit & tuned_flags(base.precision))) continue;
         hwt_config c = best;
         c.flags ^= bit;
         if ((rc = consider(c))) return rc;
