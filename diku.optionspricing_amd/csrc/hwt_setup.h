@@ -62,15 +62,18 @@ __device__ __forceinline__ TriKind tri_setup(OptConst &c, int tu, Yield &&yield,
     c.rho = t.rho;
     c.rhop = t.rhop;
     const bool grouped = c.w <= (spread ? TRI_SPREAD_WIDTH : TRI_GROUP_WIDTH);
-    int lo = c.jmax, up = c.jmax;
+    int lo = c.jmax, up = c.jmax, half = c.jmax;
     if (!grouped) {
         // priced over the nodes that carry weight, most at step n
         c.sigmas = window_sigmas(c);
         const Reach reach = make_reach(c.sigmas, c.M, c.dr, c.dt, c.n, c.jmax);
         key = (int64_t)reach_updates(reach, c.n, c.e);
         reach_at(reach, c.n, min(c.e, c.jmax) + (c.n - c.e), lo, up);
+        // a window's other nodes have scales too: whole lanes' spare nodes lie up to
+        // WAVE - 1 beyond those kept, and the smallest window is MIN_WINDOW nodes a lane
+        half = min(max(max(lo, up) + WAVE - 1, MIN_WINDOW * WAVE - 1), c.jmax);
     }
-    if (tri_ok(t, edges, c.n, max(lo, up), grouped ? 100.0f : 200.0f) && (grouped || lo + up + 17 <= TRI_MAX_NODES))
+    if (tri_ok(t, edges, c.n, half, grouped ? 100.0f : 200.0f) && (grouped || lo + up + 17 <= TRI_MAX_NODES))
         return grouped ? TRI_GROUPED : TRI_WINDOWED;
     // the general kernel's scales (unit_form_ok)
     double etab[EDGE_TAB];

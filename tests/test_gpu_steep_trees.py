@@ -1,0 +1,36 @@
+"""Wide trees of a few steps whose rates lie far apart: the nodes a price depends on are
+close to the root, the discounts of the windows' other nodes leave FP64's range."""
+import numpy as np
+import pytest
+
+from conftest import parity_tol
+
+pytestmark = pytest.mark.gpu
+
+
+def _options(pkg, seed, n, h, heights):
+    """Yearly steps; h is the rate spacing times the step, drawn between the given bounds."""
+    r = np.random.default_rng(seed)
+    jmax = r.integers(33, 346, n)
+    a = -np.log1p(-0.184 / (jmax - 0.5))
+    height = r.integers(heights[0], heights[1] + 1, n)
+    e = (r.uniform(size=n) * height).astype(int)
+    sigma = np.exp(r.uniform(*np.log(h), n)) / np.sqrt(3 * -np.expm1(-2 * a) / (2 * a))
+    return pkg.Options(strike=np.exp(r.uniform(0, np.log(400), n)), maturity=height + 0.5, length=e + 0.5,
+                       term_unit=np.full(n, 365, np.uint16), term_steps=np.ones(n, np.uint16), a=a, sigma=sigma,
+                       type=r.integers(0, 2, n).astype(np.int8))
+
+
+def _check(pkg, oracle, opts):
+    y = pkg.datasets.synthetic_yield()
+    ref = oracle.price(opts, y)
+    fin = np.isfinite(ref)
+    assert fin.mean() > 0.9
+    for n in (opts.N, 600):  # through the general pipeline, and the kernel for small batches
+        got = pkg.capi.price(opts.take(np.arange(n)), y)
+        bad = np.nonzero(fin[:n] & ~(np.abs(got - ref[:n]) <= parity_tol(ref[:n])))[0]
+        assert bad.size == 0, (bad.size, bad[:4], got[bad[:4]], ref[bad[:4]])
+
+
+def test_windows_within_the_scales_range(pkg, oracle):
+    _check(pkg, oracle, _options(pkg, 67, 2500, (0.02, 0.5), (1, 3)))
