@@ -276,6 +276,11 @@ __device__ __forceinline__ void stencil_steps(T (&z)[K], const T (&cl)[K], const
     }
 }
 
+// A node's discount by itself, for the rare trees whose discounts of neighbouring nodes
+// lie so far apart (e^32) that one advanced by multiplication along a lane's nodes
+// could overflow or vanish on the way to one of an ordinary size.
+__device__ __noinline__ static double far_disc(const TreeShape t, int k) { return node_disc(k, t.jmax, t.dr, t.dt); }
+
 // Coefficients of this lane's K nodes for the forward operator G (FWD) or the
 // backward operator G^T, computed in FP64 and stored as T.  Interior nodes use
 // the closed forms with the node discounts E_k = e^{-(k-jmax) dr dt} advanced
@@ -307,6 +312,7 @@ __device__ __forceinline__ void window_coefs(const TreeShape &t, int base, int l
             if (k0 + s >= t.w) cl[s] = cm[s] = cr[s] = (T)0;
     } else {
         double E = node_disc(k0, t.jmax, t.dr, t.dt);
+        const bool steep = sizeof(T) == sizeof(double) && t.dr * t.dt > 32.0;
 #pragma unroll
         for (int s = 0; s < K; ++s) {
             const int j = k0 + s - t.jmax;
@@ -315,6 +321,7 @@ __device__ __forceinline__ void window_coefs(const TreeShape &t, int base, int l
             cm[s] = (T)(pm_std(j, t.M) * Ek);
             cr[s] = (T)(pu_std(j, t.M) * Ek);
             E *= q;
+            if (steep) E = far_disc(t, k0 + s + 1);
         }
     }
     const lds_f64 *tab = etab + (FWD ? 0 : 18);

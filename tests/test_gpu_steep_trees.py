@@ -34,3 +34,9 @@ def _check(pkg, oracle, opts):
 
 def test_windows_within_the_scales_range(pkg, oracle):
     _check(pkg, oracle, _options(pkg, 67, 2500, (0.02, 0.5), (1, 3)))
+
+
+def test_discounts_out_of_range_beside_the_root(pkg, oracle):
+    """One step, rate spacing times step up to 5,000: the root's own discount is 1, its
+    neighbours' may overflow and underflow."""
+    _check(pkg, oracle, _options(pkg, 71, 2500, (20.0, 5000.0), (1, 1)))
