@@ -46,7 +46,6 @@ __device__ __forceinline__ double price_option(const OptConst &cv, const double 
         }
     }
     if (!made) load_edge_table(edge, lane, etab);
-    int flo, fhi, blo, bhi;
     const bool unit = uni((int)cv.unit) != 0;
     // wide trees change window four nodes per lane at a time (a 60k batch of
     // wide and narrow trees: 283 us with single steps, 252 us with 2, 243 us
@@ -54,50 +53,58 @@ __device__ __forceinline__ double price_option(const OptConst &cv, const double 
     constexpr int G = KMAX > KSMALL ? WIDE_WINDOW_STEP : 1;
     constexpr int RG = REACH_WINDOW_STEP;
     const Reach reach = make_reach(cv.sigmas, t.M, t.dr, t.dt, n, t.jmax);
-    forward_pass<T, KMAX, G, RG>(t, reach, e, lane, lds, etab, fscratch, flo, fhi, unit);
-    backward_pass<T, KMAX, G, RG>(t, reach, n, e, lane, lds, etab, blo, bhi, unit);
+    // FP64 states that overflow, or whose products do, are made again from starts 2^900
+    // smaller: the price does not depend on the starts' size
+    for (double one = 1.0;; one = 0x1p-900) {
+        int flo, fhi, blo, bhi;
+        forward_pass<T, KMAX, G, RG>(t, reach, e, lane, lds, etab, fscratch, flo, fhi, unit, one);
+        backward_pass<T, KMAX, G, RG>(t, reach, n, e, lane, lds, etab, blo, bhi, unit, one);
 
-    const int ep = min(e, t.jmax);
-    int klo = t.jmax - ep, khi = t.jmax + ep;
-    if constexpr (sizeof(T) == sizeof(double)) {  // both windows hold the nodes kept at step e
-        klo = max(klo, max(flo, blo));
-        khi = min(khi, min(fhi, bhi) - 1);
-    }
-    auto fy = [&](int k) { return (k >= flo && k < fhi) ? (double)fscratch[k] : 0.0; };
-    auto fb = [&](int k) { return (k >= blo && k < bhi) ? (double)lds[k] : 0.0; };
-    auto yk = [&](int k) {
-        double v = fy(k);
-        if (k == 1) v -= t.rho * fy(0);
-        if (k == t.w - 2) v -= t.rhop * fy(t.w - 1);
-        return v;
-    };
-    auto bk = [&](int k) {
-        double v = fb(k);
-        if (k == 0) v += t.rho * fb(1);
-        if (k == t.w - 1) v += t.rhop * fb(t.w - 2);
-        return v;
-    };
-    typename SumOf<T>::type a1, a2, a3;
-    bool big = false;
-    for (int k = klo + lane; k <= khi; k += WAVE) {
-        const double yv = yk(k), bv = bk(k);
-        a1.add(yv);
-        a2.add(yv * bv);
-        big |= !(fabs(bv) <= F32_SAFE_STATE);
-    }
-    const double s1 = a1.wave_total(), s2 = a2.wave_total();
-    if constexpr (sizeof(T) == sizeof(float)) {
-        // FP32 state out of range: NaN asks for the FP64 re-pricing
-        if (__ballot(big) != 0 || !isfinite(s1) || !isfinite(s2)) {
-            __syncthreads();
-            return NAN;
+        const int ep = min(e, t.jmax);
+        int klo = t.jmax - ep, khi = t.jmax + ep;
+        if constexpr (sizeof(T) == sizeof(double)) {  // both windows hold the nodes kept at step e
+            klo = max(klo, max(flo, blo));
+            khi = min(khi, min(fhi, bhi) - 1);
         }
+        auto fy = [&](int k) { return (k >= flo && k < fhi) ? (double)fscratch[k] : 0.0; };
+        auto fb = [&](int k) { return (k >= blo && k < bhi) ? (double)lds[k] : 0.0; };
+        auto yk = [&](int k) {
+            double v = fy(k);
+            if (k == 1) v -= t.rho * fy(0);
+            if (k == t.w - 2) v -= t.rhop * fy(t.w - 1);
+            return v;
+        };
+        auto bk = [&](int k) {
+            double v = fb(k);
+            if (k == 0) v += t.rho * fb(1);
+            if (k == t.w - 1) v += t.rhop * fb(t.w - 2);
+            return v;
+        };
+        typename SumOf<T>::type a1, a2, a3;
+        bool big = false;
+        for (int k = klo + lane; k <= khi; k += WAVE) {
+            const double yv = yk(k), bv = bk(k);
+            a1.add(yv);
+            a2.add(yv * bv);
+            big |= !(fabs(bv) <= F32_SAFE_STATE);
+        }
+        const double s1 = a1.wave_total(), s2 = a2.wave_total();
+        if constexpr (sizeof(T) == sizeof(float)) {
+            // FP32 state out of range: NaN asks for the FP64 re-pricing
+            if (__ballot(big) != 0 || !isfinite(s1) || !isfinite(s2)) {
+                __syncthreads();
+                return NAN;
+            }
+        } else if (one == 1.0 && __ballot(!isfinite(s1) || !isfinite(s2)) != 0) {
+            __syncthreads();
+            continue;
+        }
+        const double scale = 100.0 * s1 * cv.Pn / (s2 * cv.Pe);
+        for (int k = klo + lane; k <= khi; k += WAVE) a3.add(yk(k) * payoff<T>(cv, scale * bk(k)));
+        const double s3 = a3.wave_total();
+        __syncthreads();
+        return cv.Pe / s1 * s3;
     }
-    const double scale = 100.0 * s1 * cv.Pn / (s2 * cv.Pe);
-    for (int k = klo + lane; k <= khi; k += WAVE) a3.add(yk(k) * payoff<T>(cv, scale * bk(k)));
-    const double s3 = a3.wave_total();
-    __syncthreads();
-    return cv.Pe / s1 * s3;
 }
 
 // Narrow trees (width <= 64*K): the whole tree in one full window, both passes

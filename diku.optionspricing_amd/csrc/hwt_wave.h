@@ -353,9 +353,10 @@ __device__ __forceinline__ void window_coefs(const TreeShape &t, int base, int l
     }
 }
 
-// Initial values: forward delta at the root node; backward T^{-T} * 100.
+// Initial values: forward delta at the root node; backward T^{-T} * 100; times `one`, a
+// power of two (price_option).
 template <class T, int K, bool FWD>
-__device__ __forceinline__ void init_window(T (&z)[K], const TreeShape &t, int base, int lane)
+__device__ __forceinline__ void init_window(T (&z)[K], const TreeShape &t, int base, int lane, double one = 1.0)
 {
 #pragma unroll
     for (int s = 0; s < K; ++s) {
@@ -368,7 +369,7 @@ __device__ __forceinline__ void init_window(T (&z)[K], const TreeShape &t, int b
             if (k == 0) v -= t.rho * 100.0;
             if (k == t.w - 1) v -= t.rhop * 100.0;
         }
-        z[s] = (T)v;
+        z[s] = (T)(v * one);
     }
 }
 
@@ -603,11 +604,12 @@ HWT_HD bool unit_form_ok(const TreeShape &t, const double *tab, double dmin)
 // and leave the window's tree nodes in LDS, or in `out` when given.
 template <class T, int K, bool FWD>
 __device__ __forceinline__ void phase_fn(const TreeShape &t, int base, int nsteps, int in_lo, int in_hi, int lane,
-                                         typename Lds<T>::type *lds, const lds_f64 *etab, T *out, bool unit)
+                                         typename Lds<T>::type *lds, const lds_f64 *etab, T *out, bool unit,
+                                         double one)
 {
     T z[K];
     if (in_lo >= in_hi) {
-        init_window<T, K, FWD>(z, t, base, lane);
+        init_window<T, K, FWD>(z, t, base, lane, one);
     } else {
 #pragma unroll
         for (int s = 0; s < K; ++s) {
@@ -655,13 +657,14 @@ __device__ __forceinline__ void phase_fn(const TreeShape &t, int base, int nstep
 template <class T, int KMAX, bool FWD>
 __device__ __forceinline__ void dispatch_phase(int K, const TreeShape &t, int base, int nsteps, int in_lo, int in_hi,
                                                int lane, typename Lds<T>::type *lds, const lds_f64 *etab, T *out,
-                                               bool unit)
+                                               bool unit, double one)
 {
     switch (K) {
 #define HWT_C(KK)                                                                                        \
     case KK:                                                                                             \
         if (KK <= KMAX)                                                                                  \
-            phase_fn<T, (KK <= KMAX ? KK : 1), FWD>(t, base, nsteps, in_lo, in_hi, lane, lds, etab, out, unit); \
+            phase_fn<T, (KK <= KMAX ? KK : 1), FWD>(t, base, nsteps, in_lo, in_hi, lane, lds, etab, out, unit, \
+                                                       one);                                             \
         break;
         HWT_KCASES(HWT_C)
 #undef HWT_C
@@ -963,11 +966,11 @@ __device__ __forceinline__ bool unit_phase(int K, bool unit)
 template <class T, int KMAX, int CG, int RG>
 __device__ __forceinline__ void forward_pass(const TreeShape &t, const Reach &r, int e, int lane,
                                              typename Lds<T>::type *lds, const lds_f64 *etab, T *out, int &lo, int &hi,
-                                             bool unit)
+                                             bool unit, double one)
 {
     auto phase = [&](const Window &win, int nsteps, int in_lo, int in_hi, bool last) {
         dispatch_phase<T, KMAX, true>(win.K, t, win.base, nsteps, in_lo, in_hi, lane, lds, etab,
-                                      last ? out : nullptr, unit);
+                                      last ? out : nullptr, unit, one);
     };
     if constexpr (sizeof(T) == sizeof(float)) cone_forward<CG>(t, e, lo, hi, phase);
     else reach_forward<RG>(t, r, e, lane, lo, hi, phase);
@@ -978,11 +981,11 @@ __device__ __forceinline__ void forward_pass(const TreeShape &t, const Reach &r,
 template <class T, int KMAX, int CG, int RG>
 __device__ __forceinline__ void backward_pass(const TreeShape &t, const Reach &r, int n, int e, int lane,
                                               typename Lds<T>::type *lds, const lds_f64 *etab, int &lo, int &hi,
-                                              bool unit)
+                                              bool unit, double one)
 {
     auto phase = [&](const Window &win, int nsteps, int in_lo, int in_hi, bool) {
         dispatch_phase<T, KMAX, false>(win.K, t, win.base, nsteps, in_lo, in_hi, lane, lds, etab, (T *)nullptr,
-                                       unit);
+                                       unit, one);
     };
     if constexpr (sizeof(T) == sizeof(float)) cone_backward<CG>(t, n, e, lo, hi, phase);
     else reach_backward<RG>(t, r, n, e, lane, lo, hi, phase);

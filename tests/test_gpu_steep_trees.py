@@ -40,3 +40,28 @@ def test_discounts_out_of_range_beside_the_root(pkg, oracle):
     """One step, rate spacing times step up to 5,000: the root's own discount is 1, its
     neighbours' may overflow and underflow."""
     _check(pkg, oracle, _options(pkg, 71, 2500, (20.0, 5000.0), (1, 1)))
+
+
+@pytest.mark.parametrize("n", [2500, 600])
+def test_states_beyond_the_range(pkg, oracle, n):
+    """Volatilities at which a tree's undiscounted states, or their products, exceed 1e308
+    (n h jmax up to 900): out of the tridiagonal form's range, priced by the general
+    kernel.  The bar as for tall trees: the steps' own rounding on top of the parity bar."""
+    r = np.random.default_rng(73)
+    jmax = r.integers(1, 86, n)
+    a = np.where(jmax == 1, 0.9, -np.log1p(-0.184 / (jmax - 0.5)))
+    height = r.integers(300, 3000, n)
+    h = r.uniform(310, 900, n) / (height * jmax)
+    opts = pkg.Options(strike=np.exp(r.uniform(0, np.log(400), n)), maturity=height + 0.5,
+                       length=(r.uniform(size=n) * height).astype(int) + 0.5, term_unit=np.full(n, 365, np.uint16),
+                       term_steps=np.ones(n, np.uint16), a=a, sigma=h / np.sqrt(3 * -np.expm1(-2 * a) / (2 * a)),
+                       type=r.integers(0, 2, n).astype(np.int8))
+    days = np.array([365, 365000], np.int32)
+    y = pkg.formats.Yield(np.array([0.001, 0.0012]), days)  # bonds of thousands of years worth something
+    ref = oracle.price(opts, y)
+    fin = np.isfinite(ref)
+    assert fin.mean() > 0.9
+    got = pkg.capi.price(opts, y)
+    tol = parity_tol(ref) + 100 * 8 * height * 2.0**-53
+    bad = np.nonzero(fin & ~(np.abs(got - ref) <= tol))[0]
+    assert bad.size == 0, (bad.size, bad[:4], got[bad[:4]], ref[bad[:4]])
