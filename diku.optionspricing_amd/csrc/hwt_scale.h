@@ -36,6 +36,14 @@ struct SixfoldScale {
     }
 };
 
+// Bits by which a state is larger (below 0: smaller) than it would be had it been
+// scaled at each of its own steps, to one bit or two: its steps were those from the
+// `from`th to the `to`th counted.
+constexpr int sixfold_left(int from, int to)
+{
+    return (int)(2.5849625f * (float)((to & (SixfoldScale::EVERY - 1)) - (from & (SixfoldScale::EVERY - 1))));
+}
+
 // 2^-bits, bits < 1023
 constexpr double pow2_down(int bits) { return __builtin_bit_cast(double, (uint64_t)(1023 - bits) << 52); }
 

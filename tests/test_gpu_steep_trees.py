@@ -65,3 +65,22 @@ def test_states_beyond_the_range(pkg, oracle, n):
     tol = parity_tol(ref) + 100 * 8 * height * 2.0**-53
     bad = np.nonzero(fin & ~(np.abs(got - ref) <= tol))[0]
     assert bad.size == 0, (bad.size, bad[:4], got[bad[:4]], ref[bad[:4]])
+
+
+@pytest.mark.parametrize("n", [300, 3000, 17000])
+def test_bonds_of_any_finite_price(pkg, oracle, n):
+    """Thousands of years at -4%: bonds worth up to 1e300, puts on them nothing."""
+    r = np.random.default_rng(79)
+    jmax = np.resize(np.r_[np.arange(2, 60), 88, 90, 150], n)
+    height = r.integers(13000, 17001, n)
+    opts = pkg.Options(strike=r.uniform(60, 100, n), maturity=height + 0.5, length=r.integers(0, 200, n) + 0.5,
+                       term_unit=np.full(n, 365, np.uint16), term_steps=np.ones(n, np.uint16),
+                       a=-np.log1p(-0.184 / (jmax - 0.5)), sigma=r.uniform(1e-5, 1e-4, n),
+                       type=r.integers(0, 2, n).astype(np.int8))
+    y = pkg.formats.Yield(np.array([-0.04, -0.04]), np.array([1, 2], np.int32))
+    some = np.arange(0, n, n // 30)
+    ref, got = oracle.price(opts.take(some), y), pkg.capi.price(opts, y)
+    assert np.isfinite(ref).all() and ref.max() > 1e270 and (ref[opts.type[some] == 1] == 0).all()
+    # relative: the oracle rounds each of its 2 x 17,000 steps
+    assert np.all(np.abs(got[some] - ref) <= 1e-10 * ref), (got[some][:5], ref[:5])
+    assert np.isfinite(got).all() and (got[opts.type == 1] == 0).all()

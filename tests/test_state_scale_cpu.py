@@ -78,3 +78,44 @@ def test_scaling_follows_the_growth(emulate, name):
     slack = 1e-5 + steps * 2.0**-33  # the sum's own rounding here, and log2 6 in units of 2^-32
     assert -slack <= lo and hi < 1 + slack
     assert -slack <= end < 64 * math.log2(6) + 1 + slack
+
+
+LEFT = r"""
+#include "hwt_scale.h"
+#include <cstdio>
+// argv: from, to.  Out: log2 of a state that grew from step `from` to step `to` of a count
+// scaled all along, less what sixfold_left gives.
+int main()
+{
+    int from, to;
+    while (std::scanf("%d %d", &from, &to) == 2) {
+        hwt::SixfoldScale s;
+        double bits = 0;
+        auto steps = [](int) {};
+        auto scale = [&](double f) {
+            int e = 0;
+            __builtin_frexp(f, &e);
+            bits += e - 1;
+        };
+        hwt::scaled_steps(s, from, steps, scale);
+        bits = 0;
+        hwt::scaled_steps(s, to - from, steps, scale);
+        std::printf("%.17g\n", (to - from) * 2.5849625007211561815 + bits - hwt::sixfold_left(from, to));
+    }
+}
+"""
+
+
+def test_what_the_scaling_left(tmp_path):
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if not cxx:
+        pytest.skip("no host compiler")
+    (tmp_path / "left.cpp").write_text(LEFT)
+    inc = ROOT / "diku.optionspricing_amd" / "csrc"
+    subprocess.run([cxx, "-O2", "-std=c++17", f"-I{inc}", "-o", tmp_path / "left", tmp_path / "left.cpp"], check=True)
+    r = np.random.default_rng(3)
+    pairs = [(0, 0), (0, 63), (0, 64), (63, 64), (63, 127), (1, 64), (64, 64), (0, 1_000_000)]
+    pairs += [tuple(sorted(r.integers(0, 300_000, 2))) for _ in range(500)]
+    text = " ".join(f"{a} {b}" for a, b in pairs)
+    out = subprocess.run([tmp_path / "left"], input=text, check=True, capture_output=True, text=True).stdout
+    assert all(-2 <= float(v) <= 2 for v in out.split())
