@@ -281,12 +281,12 @@ __device__ __forceinline__ void tri_steps(double (&z)[K], const double (&m)[K], 
 // (backward), in the same window:
 //   S1 = sum y, S2 = sum y b (equal in edge-transformed and plain states),
 //   scale = 100 S1 Pn / (S2 Pe), price = Pe / S1 sum y payoff(scale b).
-// u took the steps counted from `start` to `swap`, v those to `end`; what the scaling
-// left of their growth goes with d1 and d2, so that any bond price in FP64's range fits.
+// What the scaling left of the states' growth (sixfold_left) goes with d1 and d2, so that
+// any bond price in FP64's range fits.
 template <int L, int K>
 __device__ __forceinline__ double tri_price(const TreeShape &t, const TriEdge &e, bool edges, int base, int lane, int l,
-                                            double (&u)[K], double (&v)[K], int start, int swap, int end, double X,
-                                            double Pe, double Pn, int type, lds_f64 *lds)
+                                            double (&u)[K], double (&v)[K], int left_u, int left_v, double X, double Pe,
+                                            double Pn, int type, lds_f64 *lds)
 {
     // u and v times the scales' products along the lane, then times the lane's own
     double p1 = 1.0, p2 = 1.0;
@@ -305,8 +305,8 @@ __device__ __forceinline__ double tri_price(const TreeShape &t, const TriEdge &e
         d1 /= readlane_f64(d1, root);
         d2 /= readlane_f64(d2, root);
     }
-    d1 = ldexp(d1, -sixfold_left(start, swap));
-    d2 = ldexp(d2, -sixfold_left(swap, end));
+    d1 = ldexp(d1, -left_u);
+    d2 = ldexp(d2, -left_v);
 #pragma unroll
     for (int s = 0; s < K; ++s) {
         u[s] *= d1;
@@ -412,7 +412,8 @@ __device__ __forceinline__ double price_tri_group(const OptConst *__restrict__ c
     const OptConst c = cst[o];
     const TreeShape t{c.w, c.jmax, c.M, c.dr, c.dt, c.rho, c.rhop};
     __syncthreads();
-    return tri_price<L, K>(t, edge[o], true, 0, lane, l, u, z, start, swap, N, c.X, c.Pe, c.Pn, c.type, lds);
+    return tri_price<L, K>(t, edge[o], true, 0, lane, l, u, z, sixfold_left(start, swap), sixfold_left(swap, N), c.X, c.Pe,
+                           c.Pn, c.type, lds);
 }
 
 // ------------------------------------------------------------------ windows
@@ -425,6 +426,7 @@ struct TriPhase {
     bool first, last, back;
     int in_base, in_n;  // the previous window's nodes in LDS
     int f_base, f_n;    // the parked forward state's
+    int left_u, left_v; // what the scaling leaves of either state's growth
 };
 
 // The tree's records are read again in each phase (scalar loads) rather than
@@ -474,8 +476,8 @@ __device__ __forceinline__ double tri_phase(const OptConst *__restrict__ cst, co
     asm volatile("" : "+s"(o));
     const OptConst ce = cst[o];
     const TreeShape te = uni(TreeShape{ce.w, ce.jmax, ce.M, ce.dr, ce.dt, ce.rho, ce.rhop});
-    return tri_price<WAVE, K>(te, edge[o], edges, p.base, lane, lane, u, z, 0, uni(ce.e), uni(ce.n), ce.X, ce.Pe, ce.Pn,
-                              ce.type, lds);
+    return tri_price<WAVE, K>(te, edge[o], edges, p.base, lane, lane, u, z, p.left_u, p.left_v, ce.X, ce.Pe, ce.Pn, ce.type,
+                              lds);
 }
 
 // Prices one tree wider than a group, alone in its wave.
@@ -487,6 +489,8 @@ __device__ __forceinline__ double price_tri_window(const OptConst *__restrict__ 
     const int n = uni(c.n), e = uni(c.e);
     const Reach reach = make_reach(c.sigmas, t.M, t.dr, t.dt, n, t.jmax);
     TriPhase p{};
+    p.left_u = uni(sixfold_left(0, e));
+    p.left_v = uni(sixfold_left(e, n));
     double price = 0.0;
     SixfoldScale scale;
     for (int back = 0; back < 2; ++back) {
