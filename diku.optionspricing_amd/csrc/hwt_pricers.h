@@ -53,16 +53,21 @@ __device__ __forceinline__ double price_option(const OptConst &cv, const double 
     constexpr int G = KMAX > KSMALL ? WIDE_WINDOW_STEP : 1;
     constexpr int RG = REACH_WINDOW_STEP;
     const Reach reach = make_reach(cv.sigmas, t.M, t.dr, t.dt, n, t.jmax);
-    // FP64 states that overflow, or whose products do, are made again from starts 2^900
-    // smaller: the price does not depend on the starts' size
-    for (double one = 1.0;; one = 0x1p-900) {
+    // an FP64 state that overflows is made again from a start 2^900 smaller: the price
+    // does not depend on the starts' size.  States span up to e^{2 n h jmax}; above a span
+    // that has been checked (677 of 677 random trees right up to n h jmax = 1,200, 7 of 711
+    // off by 1e-8 and more above), what the smaller start loses at its lower end may count,
+    // and the price is NaN
+    constexpr bool fp64 = sizeof(T) == sizeof(double);
+    double yone = 1.0, bone = 1.0;
+    for (;;) {
         int flo, fhi, blo, bhi;
-        forward_pass<T, KMAX, G, RG>(t, reach, e, lane, lds, etab, fscratch, flo, fhi, unit, one);
-        backward_pass<T, KMAX, G, RG>(t, reach, n, e, lane, lds, etab, blo, bhi, unit, one);
+        forward_pass<T, KMAX, G, RG>(t, reach, e, lane, lds, etab, fscratch, flo, fhi, unit, yone);
+        backward_pass<T, KMAX, G, RG>(t, reach, n, e, lane, lds, etab, blo, bhi, unit, bone);
 
         const int ep = min(e, t.jmax);
         int klo = t.jmax - ep, khi = t.jmax + ep;
-        if constexpr (sizeof(T) == sizeof(double)) {  // both windows hold the nodes kept at step e
+        if constexpr (fp64) {  // both windows hold the nodes kept at step e
             klo = max(klo, max(flo, blo));
             khi = min(khi, min(fhi, bhi) - 1);
         }
@@ -86,24 +91,38 @@ __device__ __forceinline__ double price_option(const OptConst &cv, const double 
             const double yv = yk(k), bv = bk(k);
             a1.add(yv);
             a2.add(yv * bv);
-            big |= !(fabs(bv) <= F32_SAFE_STATE);
+            big |= !(fabs(bv) <= (fp64 ? DBL_MAX : F32_SAFE_STATE));
         }
-        const double s1 = a1.wave_total(), s2 = a2.wave_total();
-        if constexpr (sizeof(T) == sizeof(float)) {
+        const double s1 = a1.wave_total();
+        double s2 = a2.wave_total(), down = 1.0;
+        if constexpr (!fp64) {
             // FP32 state out of range: NaN asks for the FP64 re-pricing
             if (__ballot(big) != 0 || !isfinite(s1) || !isfinite(s2)) {
                 __syncthreads();
                 return NAN;
             }
-        } else if (one == 1.0 && __ballot(!isfinite(s1) || !isfinite(s2)) != 0) {
-            __syncthreads();
-            continue;
+        } else {
+            const bool again_y = __ballot(!isfinite(s1)) != 0, again_b = __ballot(big) != 0;
+            if (again_y || again_b) {
+                __syncthreads();
+                if (yone != 1.0 || bone != 1.0 || n * (t.dr * t.dt) * t.jmax > 1200.0) return NAN;
+                if (again_y) yone = 0x1p-900;
+                if (again_b) bone = 0x1p-900;
+                continue;
+            }
+            if (__ballot(!isfinite(s2)) != 0) {  // only the products overflow
+                down = 0x1p-512;
+                typename SumOf<T>::type again;
+                for (int k = klo + lane; k <= khi; k += WAVE) again.add((yk(k) * down) * (bk(k) * down));
+                s2 = again.wave_total();
+            }
         }
-        const double scale = 100.0 * s1 * cv.Pn / (s2 * cv.Pe);
-        for (int k = klo + lane; k <= khi; k += WAVE) a3.add(yk(k) * payoff<T>(cv, scale * bk(k)));
+        const double scale = 100.0 * (s1 * down) * cv.Pn / (s2 * cv.Pe) * down;
+        const double ydown = fp64 && s1 > 0x1p512 ? 0x1p-512 : 1.0;  // room for the payoffs
+        for (int k = klo + lane; k <= khi; k += WAVE) a3.add(yk(k) * ydown * payoff<T>(cv, scale * bk(k)));
         const double s3 = a3.wave_total();
         __syncthreads();
-        return cv.Pe / s1 * s3;
+        return cv.Pe / (s1 * ydown) * s3;
     }
 }
 

@@ -84,3 +84,25 @@ def test_bonds_of_any_finite_price(pkg, oracle, n):
     # relative: the oracle rounds each of its 2 x 17,000 steps
     assert np.all(np.abs(got[some] - ref) <= 1e-10 * ref), (got[some][:5], ref[:5])
     assert np.isfinite(got).all() and (got[opts.type == 1] == 0).all()
+
+
+def test_states_beyond_any_start_are_no_number(pkg, oracle):
+    """n h jmax from 1,300 to 4,000: where a state leaves the range the price is right or
+    NaN, never a wrong number."""
+    n = 2500
+    r = np.random.default_rng(83)
+    jmax = r.integers(1, 400, n)
+    a = np.where(jmax == 1, 0.9, -np.log1p(-0.184 / (np.maximum(jmax, 2) - 0.5)))
+    height = r.integers(600, 3000, n)
+    h = r.uniform(1300, 4000, n) / (height * jmax)
+    opts = pkg.Options(strike=np.exp(r.uniform(0, np.log(100), n)), maturity=height + 0.5,
+                       length=(r.uniform(size=n) * height).astype(int) + 0.5, term_unit=np.full(n, 365, np.uint16),
+                       term_steps=np.ones(n, np.uint16), a=a, sigma=h / np.sqrt(3 * -np.expm1(-2 * a) / (2 * a)),
+                       type=r.integers(0, 2, n).astype(np.int8))
+    y = pkg.formats.Yield(np.array([0.001, 0.0012]), np.array([365, 365000], np.int32))
+    ref, got = oracle.price(opts, y), pkg.capi.price(opts, y)
+    fin = np.isfinite(ref) & ~np.isnan(got)
+    tol = parity_tol(ref) + 100 * 8 * height * 2.0**-53
+    print(f"\n{np.isnan(got).sum()} NaN, {fin.sum()} to compare")
+    bad = np.nonzero(fin & ~(np.abs(got - ref) <= tol))[0]
+    assert bad.size == 0, (bad.size, bad[:4], got[bad[:4]], ref[bad[:4]])
