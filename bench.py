@@ -10,16 +10,19 @@ pricing kernels, replayed from the plan's HIP graph or launched directly
 
 Prints one JSON line.  `roofline` is for the dominant kernel (k_price_tri, timed
 with HIP events on its stream): the FP64 operations that the hardware counters
-saw it execute on this batch (2 per fused multiply-add; profiles/) against
-MI355X's 78.6 TFLOP/s FP64 peak.  `cpu_baseline` times the reference's
+saw it execute on this batch (2 per fused multiply-add; profiles/, used while the
+kernel's sources are the ones that were counted) against MI355X's 78.6 TFLOP/s FP64
+peak.  `cpu_baseline` times the reference's
 own sequential pricer (built from its sources into oracle/_ref) on a bounded
 stratified sample on this host's cores.
 """
 from __future__ import annotations
 
 import argparse
+import hashlib
 import json
 import os
+import re
 import subprocess
 import sys
 import tempfile
@@ -34,6 +37,22 @@ sys.path.insert(0, str(ROOT))
 METRIC = "options/sec on 1 MI355X: FP64 tree vs surrogate+fallback at max err 1e-3"
 FP64_PEAK_TFLOPS = 78.6
 HBM_PEAK_GBS = 8000.0
+
+
+COUNTERS = ROOT / "profiles" / "counters_pricing_skewed_60k.json"
+# what decides which operations k_price_tri executes on the 60k skewed batch
+COUNTED_SOURCES = ("csrc/hwt_k_tri.hip", "csrc/hwt_tri.h", "csrc/hwt_scale.h", "csrc/hwt_wave.h", "csrc/hwt_flat.h",
+                   "csrc/hwt_pipeline.h", "csrc/hwt_setup.h", "csrc/hwt_math.h", "datasets.py")
+
+
+def counted_sources_sha() -> str:
+    """The counted kernel's sources and its workload's, comments and blanks aside."""
+    h = hashlib.sha256()
+    for name in COUNTED_SOURCES:
+        text = (ROOT / "diku.optionspricing_amd" / name).read_text()
+        code = text if name.endswith(".py") else re.sub(r"//[^\n]*", "", text)
+        h.update("".join(code.split()).encode())
+    return h.hexdigest()[:16]
 
 
 def _cpu_model() -> str:
@@ -361,10 +380,9 @@ def main():
             kern.append(s["kernel_ms"])
     plan_k.close()
     wide_ms = float(np.mean(wide))
-    counted = {}
-    cfile = ROOT / "profiles" / "counters_pricing_skewed_60k.json"
-    if cfile.exists():
-        counted = json.loads(cfile.read_text())
+    counted = json.loads(COUNTERS.read_text()) if COUNTERS.exists() else {}
+    if counted.get("sources_sha") != counted_sources_sha():
+        counted = {}  # counted on another kernel
     wide_flop, dominant, traffic = counted.get("fp64_flop_per_launch"), "k_price_tri", counted.get("hbm_bytes_per_launch")
     flop_model = ("FP64 operations of k_price_tri on this batch by the hardware counters "
                   "(2 FMA + MUL + ADD instructions, 64 lanes each; profiles/counters_pricing_skewed_60k.json): "

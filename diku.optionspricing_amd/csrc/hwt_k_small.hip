@@ -16,7 +16,7 @@ __device__ __noinline__ static double price_general(const OptConst *c, int lane,
 // nodes, a wave above), so nothing is sorted, queued or counted, and prices are the
 // same to the bit.  A batch this small waits for latencies, not for issue: the launches
 // of the general pipeline (k_setup, k_order, the big trees' empty kernel, k_price_tri)
-// took 34 us for 1,000 options, this one 17.5 (13.3 in the kernel).
+// took 34 us for 1,000 options, this one 17.4 (13.4 in the kernel).
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(2))) void k_price_small(
     DevOpts o, DevYield y, int32_t maxWidth, double unit_dmin, OptConst *__restrict__ cst,
     int32_t *__restrict__ tally, double *__restrict__ out, double *__restrict__ scratch)

@@ -162,7 +162,10 @@ __device__ __forceinline__ int scan_bucket(int p, int asc)
 // row class (one K) is padded to a multiple of four tasks and each part of the
 // flat class (one width w) to a multiple of 64 / w, with idle slots (order
 // -1), so every group a wave takes shares one K or one width and an option's
-// arithmetic never depends on which options share its wave.  The flat parts'
+// arithmetic never depends on which options share its wave.  (FP64: nor on
+// anything but its tree and whether the batch has more than TRI_SPREAD options,
+// which decides how its nodes are split over lanes, and so its last bits; where
+// a shared wave scales its states, it does so by powers of two.)  The flat parts'
 // first tasks and first group numbers go to the tally for the flat kernel.
 template <bool TRI>
 __device__ __forceinline__ void scan_offsets(const int32_t *__restrict__ hist, int32_t *soffs,

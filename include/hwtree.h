@@ -88,12 +88,15 @@ typedef struct {
                             256); <= 0 picks the default.  Form 2 runs one wavefront
                             per workgroup. */
     int32_t sort;        /* HWT_SORT_*: processing order of the wide and mid-width
-                            trees (0 = work-descending) */
+                            trees, FP64: of those priced a wavefront each
+                            (0 = work-descending) */
     int32_t device;      /* HIP device ordinal for hwt_price_f64; < 0 = current */
     int32_t flags;       /* HWT_FLAG_* */
     int32_t wide_per_cu;   /* form 2: resident workgroups per CU of the persistent
-                              wide-tree kernel; 0 = as many as fit */
-    int32_t narrow_per_cu; /* form 2: the same for the narrow-tree kernel */
+                              wide-tree kernel (FP64: of the general kernel, and so the
+                              most options priced in one kernel); 0 = as many as fit */
+    int32_t narrow_per_cu; /* form 2: the same for the narrow-tree kernel (FP64: for the
+                              kernel that prices all others) */
     int32_t lane_max_width;/* form 1: the widest tree the plan prices (its tree columns in
                               HBM are sized for it; wider options are unsupported);
                               0 = hwt_max_width.  The one-shot calls set it from the batch. */
@@ -311,8 +314,8 @@ int hwt_alphas_f64(const hwt_options_f64 *opts, const hwt_yield_f64 *yield,
  * block size and sort order from the command line, cuda-option/Kernel.cuh:303
  * and cuda-multi/Kernel.cuh:374).  Prices the device batch repeatedly with
  * candidate settings of form 2 -- processing order of the wide trees (work,
- * height or width), narrow trees four or one per wavefront, the two pricing
- * kernels in sequence, side by side or fused, graph replays or direct
+ * height or width), in mixed mode narrow trees four or one per wavefront and the
+ * two pricing kernels in sequence, side by side or fused, graph replays or direct
  * launches (HWT_FLAG_DIRECT), and resident workgroups per CU of each -- and
  * then form 1 instead of form 2 for FP64 batches of at most 262,144 options
  * (an inspector choosing the kernel form per batch), by greedy coordinate
