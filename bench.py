@@ -168,9 +168,9 @@ def reference_sets_leg(pkg, capi, args):
 
 
 def tiny_trees_leg(pkg, capi, y, n: int = 1_000_000):
-    """The flattened form against the row form on a batch of tiny trees
-    (widths 3-21, uniform): the same options priced with trees packed 64 / w
-    to a wavefront one node per lane (default), four per wavefront in 16-lane
+    """A batch of tiny trees (widths 3-21, uniform) in FP64, and in mixed mode, whose
+    flattened form is set against its row form: trees packed 64 / w to a
+    wavefront one node per lane (default), four per wavefront in 16-lane
     rows (HWT_FLAG_NO_FLAT), and one per wavefront (also HWT_FLAG_NO_ROWS).
     Graph replays timed with HIP events."""
     import ctypes as C
@@ -180,9 +180,10 @@ def tiny_trees_leg(pkg, capi, y, n: int = 1_000_000):
     stream = C.c_void_p()
     dm._ck(dm.hip().hipStreamCreate(C.byref(stream)))
     out = {"options": n}
-    for name, flags in (("flat", 0), ("rows", capi.FLAG_NO_FLAT),
-                        ("one_per_wave", capi.FLAG_NO_FLAT | capi.FLAG_NO_ROWS)):
-        plan = capi.Plan(n, y.N, capi.config(flags=flags))
+    for name, precision, flags in (("fp64", capi.PREC_FP64, 0), ("mixed_flat", capi.PREC_MIXED, 0),
+                                   ("mixed_rows", capi.PREC_MIXED, capi.FLAG_NO_FLAT),
+                                   ("mixed_one_per_wave", capi.PREC_MIXED, capi.FLAG_NO_FLAT | capi.FLAG_NO_ROWS)):
+        plan = capi.Plan(n, y.N, capi.config(precision=precision, flags=flags))
         for _ in range(3):
             plan.execute(dev, stream=stream.value)
         st = plan.sync()
@@ -196,7 +197,7 @@ def tiny_trees_leg(pkg, capi, y, n: int = 1_000_000):
         plan.close()
         ms = e0.elapsed_ms(e1) / 10
         out[name] = {"ms": ms, "options_per_s": n / (ms * 1e-3), "tasks": st["tasks"]}
-    out["flat_speedup_over_rows"] = out["rows"]["ms"] / out["flat"]["ms"]
+    out["flat_speedup_over_rows"] = out["mixed_rows"]["ms"] / out["mixed_flat"]["ms"]
     dm._ck(dm.hip().hipStreamDestroy(stream))
     for k in list(dev):
         if hasattr(dev[k], "free"):
