@@ -293,8 +293,8 @@ __device__ __forceinline__ double tri_price(const TreeShape &t, const TriEdge &e
     const int in = t.w - (base + l * K);
     tri_walk<K>(t, e, base + l * K, [&](int s, double a, double c, double, double) {
         if (s > 0 || l > 0) {
-            p1 *= s < in ? a : 0.0;
-            p2 *= s < in ? c : 0.0;
+            p1 *= s < in ? a : 0.0;  // padding: no weight, and a bond value above 0, which an
+            p2 *= s < in ? c : 1.0;  // infinite scale does not turn into a NaN
         }
         u[s] *= p1;
         v[s] *= p2;

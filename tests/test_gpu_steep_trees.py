@@ -106,3 +106,18 @@ def test_states_beyond_any_start_are_no_number(pkg, oracle):
     print(f"\n{np.isnan(got).sum()} NaN, {fin.sum()} to compare")
     bad = np.nonzero(fin & ~(np.abs(got - ref) <= tol))[0]
     assert bad.size == 0, (bad.size, bad[:4], got[bad[:4]], ref[bad[:4]])
+
+
+@pytest.mark.parametrize("n", [300, 3000, 17000])
+def test_puts_on_bonds_beyond_the_range(pkg, n):
+    """18,000 to 30,000 years at -4%: the bond is worth more than 1e308, a put on it
+    nothing, in groups and windows with and without padding nodes.  (The oracle steps
+    through infinite bond values and has no number here.)"""
+    r = np.random.default_rng(97)
+    jmax = np.resize(np.r_[np.arange(1, 60), 88, 90, 150], n)
+    opts = pkg.Options(strike=r.uniform(60, 100, n), maturity=r.integers(18000, 30001, n) + 0.5,
+                       length=r.integers(0, 200, n) + 0.5, term_unit=np.full(n, 365, np.uint16),
+                       term_steps=np.ones(n, np.uint16), sigma=r.uniform(1e-5, 1e-4, n), type=np.ones(n, np.int8),
+                       a=np.where(jmax == 1, 0.9, -np.log1p(-0.184 / (np.maximum(jmax, 2) - 0.5))))
+    got = pkg.capi.price(opts, pkg.formats.Yield(np.array([-0.04, -0.04]), np.array([1, 2], np.int32)))
+    assert (got == 0).all(), (np.isnan(got).sum(), got[got != 0][:5])
